@@ -7,20 +7,22 @@ gather), inputs resident on the device (the entry takes scalars only), the
 result left in device memory.
 
 Reported:
-  value       options/s of the FP32 + FP64-residual-refinement form
-              (futhark_entry_main, the headline form);
+  value       options/s of futhark_entry_main in its default form (f32
+              prices, to the accuracy of FP32 sweeps with an FP64-residual
+              refinement or better: computed in FP64);
   fp64        options/s of the FP64 form (futhark_entry_main_f64) and the
               ratio; p50/p99 per-call latency of both;
-  roofline    the dominant kernel (the x sweep of the FP32+refine form):
-              algorithmic bytes per launch (read R + write Y, 2*N*4 bytes per
-              option, 128 options) / its mean launch duration, against 8 TB/s.
-              The duration: the event-free timed calls' time per call times
-              the kernel's share of the GPU time per call, the share from HIP
-              events recorded around every launch on the library's stream in
-              a second pass of the same calls (a call is its kernels back to
-              back, with no gaps between them, so the event-free call time is
-              their sum; the events themselves lengthen each launch);
-              `valu` beside it from the committed rocprofv3 counters;
+  roofline    the kernel with the largest share of a call's GPU time: the
+              bytes it has to move (kernel_bytes) over its mean launch
+              duration, against 8 TB/s, and `fp64` beside it, the call's FP64
+              operations per second against the vector peak.  Neither is
+              near: a call's work is one grid's modes, a few hundred
+              wavefronts, so it lasts as long as one wavefront's chain of
+              dependent operations.  The duration: the event-free timed
+              calls' time per call times the kernel's share of the GPU time
+              per call, the share from HIP events recorded around every
+              launch on the library's stream in a second pass of the same
+              calls;
   accuracy    per workload, max abs / relative price error against the FP64
               oracle (the C restatement, Thomas form);
   workloads   main(16, 32, 256, 256) (the CPU-sized plain method),
@@ -44,6 +46,7 @@ sys.path.insert(0, ROOT)
 OUTER, NX, NY, NT = 128, 256, 256, 64
 PARAMS = (0.03, 5.0, 0.2, 0.6, 0.5)
 HBM_PEAK_GBS = 8000.0
+FP64_VECTOR_TFLOPS = 78.6
 
 
 def log(msg):
@@ -66,31 +69,6 @@ def time_calls(ctx, raw, free, steps, warmup):
     ctx.sync()
     total = time.perf_counter() - t_start
     return total, lat
-
-
-def profiled_traffic(kernel):
-    """HBM bytes per launch of `kernel` measured by rocprofv3 (FETCH_SIZE +
-    WRITE_SIZE, scaled by a device copy of known size) for this workload,
-    from the committed profile summary; None when there is none."""
-    path = os.path.join(ROOT, "profiles",
-                        "lvc_sweeps_main_128x256x256x64_fp32refine.traffic.json")
-    try:
-        with open(path) as f:
-            return json.load(f)["hbm_bytes_per_launch"].get(kernel)
-    except (OSError, ValueError, KeyError):
-        return None
-
-
-def profiled_valu(kernel):
-    """VALU issue fraction of `kernel` from the committed rocprofv3 counters
-    (SQ_INSTS_VALU over the SIMDs' issue slots in its measured duration)."""
-    path = os.path.join(ROOT, "profiles",
-                        "lvc_sweeps_main_128x256x256x64_fp32refine.traffic.json")
-    try:
-        with open(path) as f:
-            return json.load(f)["valu"].get(kernel)
-    except (OSError, ValueError, KeyError):
-        return None
 
 
 def accuracy(got, ref):
@@ -158,6 +136,15 @@ def bench_main_workload(lvc, outer, nx, ny, nt, params=PARAMS, reps=10, check=Tr
         out["fp64"]["accuracy_vs_fp64_oracle"] = accuracy(
             res["fp64"], oracle_main(outer, nx, ny, nt, params, False))
     return out
+
+
+def kernel_bytes(kernel):
+    """Bytes one launch of `kernel` has to move in a headline call: the modes'
+    eigenvalues and values f (8 bytes each), one coefficient per mode and
+    option, the f32 prices."""
+    modes = NX - 2
+    return {"lvc_modes": 8 * modes * (1 + OUTER), "lvc_evolve": 8 * modes * 2,
+            "lvc_price": 8 * modes * (1 + OUTER) + 4 * OUTER}.get(kernel, 0)
 
 
 def pct(v, q):
@@ -575,10 +562,8 @@ def main():
 
     v32 = OUTER * args.steps / total32
     v64 = OUTER * args.steps / total64
-    xs = rep32.get("lvc_xsweep", {"count": 0, "total_us": 0.0})
-    ys = rep32.get("lvc_ysweep", {"count": 0, "total_us": 0.0})
-    dom, other = (xs, ys) if xs["total_us"] >= ys["total_us"] else (ys, xs)
-    dom_name = "lvc_xsweep" if dom is xs else "lvc_ysweep"
+    dom_name, dom = max(((k, v) for k, v in rep32.items() if isinstance(v, dict)),
+                        key=lambda kv: kv[1]["total_us"])
     avg_us_events = dom["total_us"] / max(dom["count"], 1)
     # the kernel's share of the event-timed GPU time, applied to the
     # event-free call time (the calls' kernels run back to back)
@@ -586,8 +571,10 @@ def main():
     share = dom["total_us"] / gpu_us if gpu_us > 0 else 0.0
     launches_per_call = dom["count"] / max(args.steps, 1)
     avg_us = (1e6 * total32 / args.steps) * share / max(launches_per_call, 1e-9)
-    bytes_launch = OUTER * 2 * NX * NY * 4
+    bytes_launch = kernel_bytes(dom_name)
     achieved = bytes_launch / (avg_us * 1e-6) / 1e9 if avg_us > 0 else 0.0
+    # 18 FP64 operations per mode, row and step (fused multiply-adds as two)
+    flops_call = 26.0 * (NX - 2) * NY * (NT - 1)
     rel = float(np.max(np.abs(p32 - p64) / np.abs(p64)))
 
     out = {
@@ -601,13 +588,12 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32",
+        "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": "LocVolCalib main(128, 256, 256, 64) plain method, "
                                "s0=0.03 t=5 alpha=0.2 nu=0.6 beta=0.5",
                    "outer": OUTER, "numX": NX, "numY": NY, "numT": NT,
-                   "precision": "FP32 state and sweeps + one FP64-residual refinement "
-                                "per implicit solve; FP64 setup and price gather"},
+                   "precision": "FP64 throughout (the modes of the x operator), f32 prices"},
         "p50_ms": round(pct(lat32, 50), 4),
         "p99_ms": round(pct(lat32, 99), 4),
         "fp64": {"value": round(v64, 2), "unit": "options/s",
@@ -620,13 +606,13 @@ def main():
         "ms_per_step_with_events": round(1e3 * total32p / args.steps, 4),
         "roofline": {"bound": "hbm", "kernel": dom_name,
                      "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": profiled_traffic(dom_name),
+                     "frac": round(achieved / HBM_PEAK_GBS, 10),
                      "bytes_per_launch": bytes_launch, "avg_launch_us": round(avg_us, 3),
                      "avg_launch_us_how": "event-free time per call x the kernel's share of "
                                           "the event-timed GPU time / its launches per call",
                      "avg_launch_us_with_events": round(avg_us_events, 3),
-                     "valu": profiled_valu(dom_name)},
+                     "fp64": {"tflops": round(flops_call / (total32 / args.steps) / 1e12, 3),
+                              "peak": FP64_VECTOR_TFLOPS}},
     }
     log(f"headline: {out['ms_per_step']} ms per call (FP32+refine), "
         f"{out['fp64']['ms_per_step']} ms (FP64)")

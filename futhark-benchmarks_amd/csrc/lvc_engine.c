@@ -145,7 +145,7 @@ static int batch_xshare(struct futhark_context *ctx, int precision, int nruns,
 /* Problems whose factorisations coincide: everything but the strike (and
  * the state) equal.  The reference's main is a batch of such problems
  * (LocVolCalib.fut:244-251). */
-static int same_factor(const lvc_problem *a, const lvc_problem *b) {
+int lvc_same_factor(const lvc_problem *a, const lvc_problem *b) {
   return a->nx == b->nx && a->ny == b->ny && a->nt == b->nt && a->s0 == b->s0 &&
          a->t == b->t && a->alpha == b->alpha && a->nu == b->nu && a->beta == b->beta &&
          a->grid32 == b->grid32;
@@ -210,7 +210,7 @@ int lvc_batch_build(struct futhark_context *ctx, lvc_batch *b, int n,
       const int p = order[oi];
       int cnt = 1;
       while (oi + cnt < n && order[oi + cnt] == p + cnt &&
-             same_factor(&b->h_probs[p], &b->h_probs[p + cnt]))
+             lvc_same_factor(&b->h_probs[p], &b->h_probs[p + cnt]))
         cnt++;
       const int rows = LVC_BLOCK / lvc_lanes_for(b->h_probs[p].nx, seg_x);
       gsize[nruns] = cnt;                                    /* run length */
@@ -224,7 +224,7 @@ int lvc_batch_build(struct futhark_context *ctx, lvc_batch *b, int n,
     const int p = order[oi];
     int cnt = 1;
     while (cnt < xshare && oi + cnt < n && order[oi + cnt] == p + cnt &&
-           same_factor(&b->h_probs[p], &b->h_probs[p + cnt]))
+           lvc_same_factor(&b->h_probs[p], &b->h_probs[p + cnt]))
       cnt++;
     gsize[oi] = cnt;
     if (cnt > 1)
@@ -480,14 +480,13 @@ int lvc_batch_gather(struct futhark_context *ctx, lvc_batch *b, void *out,
 static int download(struct futhark_context *ctx, void *dst, const void *src,
                     size_t bytes);
 
-/* Runs a batch end to end into a new device array of n prices.  Each
- * problem takes its own size class's segment pair; the problems of each
- * distinct pair form a sub-batch, the sub-batches advance together, and
- * each problem's price goes to its own place in the output. */
+/* Runs problems by the sweeps into out.  Each problem takes its own size
+ * class's segment pair; the problems of each distinct pair form a sub-batch,
+ * the sub-batches advance together, and each problem's price goes to its own
+ * place in the output. */
 #define LVC_MAX_GROUPS 16
-static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *probs,
-                     int precision, int out_f64, void **out_mem) {
-  const size_t ob = (size_t)n * (out_f64 ? sizeof(double) : sizeof(float));
+static int run_sweeps(struct futhark_context *ctx, int n, const lvc_problem *probs,
+                      int precision, int out_f64, void *out) {
   int gsx[LVC_MAX_GROUPS], gsy[LVC_MAX_GROUPS], gcnt[LVC_MAX_GROUPS] = {0}, ng = 0;
   int *grp = malloc((size_t)(n ? n : 1) * sizeof(int));
   lvc_problem *sub = malloc((size_t)(n ? n : 1) * sizeof(lvc_problem));
@@ -518,36 +517,75 @@ static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *prob
   }
   lvc_batch bs[LVC_MAX_GROUPS];
   memset(bs, 0, sizeof(bs));
-  int rc = lvc_dev_alloc(ctx, ob, out_mem);
+  int rc = 0;
   for (int g = 0; !rc && g < ng; g++) {
     int m = 0;
     for (int p = 0; p < n; p++)
-      if (grp[p] == g) {
-        sub[m] = probs[p];
-        sub[m].out_index = p;
-        m++;
-      }
+      if (grp[p] == g)
+        sub[m++] = probs[p];
     rc = lvc_batch_build(ctx, &bs[g], m, sub, precision, gsx[g], gsy[g]);
   }
   if (!rc)
     rc = run_batches(ctx, bs, ng);
   for (int g = 0; !rc && g < ng; g++)
-    rc = lvc_batch_gather(ctx, &bs[g], *out_mem, out_f64);
-  if (!rc && n > 0 && ctx->cfg && ctx->cfg->debugging) {
-    /* the index the gather read: problem 0's device descriptor (the first
-     * problem of the first sub-batch) */
-    lvc_problem q;
-    rc = download(ctx, &q, bs[0].d_probs, sizeof(q));
-    if (!rc) {
-      ctx->dbg_index[0] = q.yindex;
-      ctx->dbg_index[1] = q.xindex;
-      ctx->dbg_index_valid = 1;
-    }
-  }
+    rc = lvc_batch_gather(ctx, &bs[g], out, out_f64);
   for (int g = 0; g < ng; g++)
     lvc_batch_release(ctx, &bs[g]);
   free(grp);
   free(sub);
+  return rc;
+}
+
+/* debugging: the index the prices are taken at (problem 0's) */
+static void note_index(struct futhark_context *ctx, const lvc_problem *q) {
+  if (!ctx->cfg || !ctx->cfg->debugging)
+    return;
+  ctx->dbg_index[0] = q->yindex;
+  ctx->dbg_index[1] = q->xindex;
+  ctx->dbg_index_valid = 1;
+}
+
+/* Runs a batch end to end into a new device array of n prices: in FP64 the
+ * problems whose x direction separates (lvc_modes_fit) by their modes, the
+ * others, and the FP32 forms, whose FP64 prices show the arithmetic that was
+ * asked for, by the sweeps.  A problem's way depends on the precision and its
+ * own sizes and parameters only, so its price has the same bits alone and in
+ * any batch. */
+static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *probs,
+                     int precision, int out_f64, void **out_mem) {
+  const size_t ob = (size_t)n * (out_f64 ? sizeof(double) : sizeof(float));
+  lvc_problem *by = malloc((size_t)(n ? n : 1) * sizeof(*by));
+  if (!by) {
+    lvc_set_error(ctx, "host allocation failed");
+    return 1;
+  }
+  /* the separated problems from the front, the others from the back */
+  int nm = 0, ns = 0;
+  for (int p = 0; p < n; p++) {
+    lvc_problem q = probs[p];
+    lvc_grid_scalars(&q, q.grid32);
+    q.out_index = p;
+    if (p == 0)
+      note_index(ctx, &q);
+    if (precision == LVC_FP64 && lvc_modes_fit(&q)) {
+      by[nm++] = q;
+      /* "lvc.autotune" asks for every class's sweeps to be timed */
+      int sx, sy;
+      if (ctx->cfg && ctx->cfg->autotune)
+        lvc_choose_segs(ctx, precision, q.nx, q.ny, &sx, &sy);
+    } else {
+      by[n - ++ns] = q;
+    }
+  }
+  for (int i = n - ns, j = n - 1; i < j; i++, j--) {
+    const lvc_problem q = by[i];
+    by[i] = by[j];
+    by[j] = q;
+  }
+  const int rc = lvc_dev_alloc(ctx, ob, out_mem) ||
+                 lvc_modes_batch(ctx, nm, by, *out_mem, out_f64) ||
+                 (ns && run_sweeps(ctx, ns, by + nm, precision, out_f64, *out_mem));
+  free(by);
   if (rc) {
     lvc_dev_free(ctx, *out_mem, ob);
     *out_mem = NULL;
@@ -597,6 +635,48 @@ static int check_main_index(struct futhark_context *ctx, int outer, int nx, int 
   return 1;
 }
 
+/* main's options into a new device array: one grid with strikes 0.001 * i
+ * (:247; f32 = the reference's f32 entry, strikes and initGrid's scalars in
+ * f32), by its modes where it separates, else as a batch. */
+static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int nt,
+                    double s0, double t, double alpha, double nu, double beta,
+                    int f32, int precision, void **mem) {
+  lvc_problem q;
+  fill_main(&q, 1, nx, ny, nt, s0, t, alpha, nu, beta, f32);
+  lvc_grid_scalars(&q, f32);
+  int rc = 0;
+  *mem = NULL;
+  if (outer > 0 && lvc_modes_fit(&q)) {
+    const size_t ob = (size_t)outer * (f32 ? sizeof(float) : sizeof(double));
+    const size_t wb = (size_t)lvc_modes_main_work(outer, nx) * sizeof(double);
+    double *work = NULL;
+    pthread_mutex_lock(&ctx->lock);
+    note_index(ctx, &q);
+    rc = lvc_dev_alloc(ctx, ob, mem) || lvc_dev_alloc(ctx, wb, (void **)&work) ||
+         lvc_modes_main(ctx, &q, outer, f32, work, *mem, !f32);
+    lvc_dev_free(ctx, work, wb);
+    if (rc) {
+      lvc_dev_free(ctx, *mem, ob);
+      *mem = NULL;
+    }
+    pthread_mutex_unlock(&ctx->lock);
+    return rc;
+  }
+  lvc_problem *probs = malloc((size_t)(outer ? outer : 1) * sizeof(*probs));
+  if (!probs) {
+    lvc_set_error(ctx, "host allocation failed");
+    return 1;
+  }
+  fill_main(probs, outer, nx, ny, nt, s0, t, alpha, nu, beta, f32);
+  for (int i = 0; i < outer; i++)
+    probs[i].strike = f32 ? (double)(0.001f * (float)(int64_t)i) : 0.001 * (double)(int64_t)i;
+  pthread_mutex_lock(&ctx->lock);
+  rc = run_batch(ctx, outer, probs, precision, !f32, mem);
+  pthread_mutex_unlock(&ctx->lock);
+  free(probs);
+  return rc;
+}
+
 /* LocVolCalib.fut:238-252 */
 int futhark_entry_main(struct futhark_context *ctx, struct futhark_f32_1d **out0,
                        const int32_t outer, const int32_t numX,
@@ -613,22 +693,10 @@ int futhark_entry_main(struct futhark_context *ctx, struct futhark_f32_1d **out0
   if (lvc_validate_sizes(ctx, numX, numY, numT) || !lvc_ready(ctx) ||
       check_main_index(ctx, outer, numX, numY, s0, t, alpha, nu, 1))
     return 1;
-  lvc_problem *probs = malloc((size_t)(outer ? outer : 1) * sizeof(*probs));
-  if (!probs) {
-    lvc_set_error(ctx, "host allocation failed");
-    return 1;
-  }
-  /* the f32 entry: initGrid's scalars in f32, as the reference */
-  fill_main(probs, outer, numX, numY, numT, s0, t, alpha, nu, beta, 1);
-  for (int i = 0; i < outer; i++)
-    probs[i].strike = (double)(0.001f * (float)(int64_t)i); /* :247, in f32 */
-  pthread_mutex_lock(&ctx->lock);
   void *mem = NULL;
-  int rc = run_batch(ctx, outer, probs, ctx->cfg ? ctx->cfg->precision
-                                                 : LVC_FP32_REFINE, 0, &mem);
-  pthread_mutex_unlock(&ctx->lock);
-  free(probs);
-  if (rc)
+  /* the f32 entry: initGrid's scalars in f32, as the reference */
+  if (run_main(ctx, outer, numX, numY, numT, s0, t, alpha, nu, beta, 1,
+               ctx->cfg ? ctx->cfg->precision : LVC_FP32_REFINE, &mem))
     return 1;
   *out0 = lvc_array_adopt_f32(mem, outer);
   if (!*out0) {
@@ -654,20 +722,8 @@ int futhark_entry_main_f64(struct futhark_context *ctx,
   if (lvc_validate_sizes(ctx, numX, numY, numT) || !lvc_ready(ctx) ||
       check_main_index(ctx, outer, numX, numY, s0, t, alpha, nu, 0))
     return 1;
-  lvc_problem *probs = malloc((size_t)(outer ? outer : 1) * sizeof(*probs));
-  if (!probs) {
-    lvc_set_error(ctx, "host allocation failed");
-    return 1;
-  }
-  fill_main(probs, outer, numX, numY, numT, s0, t, alpha, nu, beta, 0);
-  for (int i = 0; i < outer; i++)
-    probs[i].strike = 0.001 * (double)(int64_t)i;
-  pthread_mutex_lock(&ctx->lock);
   void *mem = NULL;
-  int rc = run_batch(ctx, outer, probs, LVC_FP64, 1, &mem);
-  pthread_mutex_unlock(&ctx->lock);
-  free(probs);
-  if (rc)
+  if (run_main(ctx, outer, numX, numY, numT, s0, t, alpha, nu, beta, 0, LVC_FP64, &mem))
     return 1;
   *out0 = lvc_array_adopt_f64(mem, outer);
   if (!*out0) {
@@ -760,6 +816,14 @@ int futhark_entry_main_noalloc(struct futhark_context *ctx, float *out,
                        "the static scratch holds %lld",
                   outer, numX, numY, numT, (long long)need, (long long)LVC_SCRATCH_BYTES);
     return 1;
+  }
+  if (lvc_modes_fit(&tmpl)) {
+    /* the work memory (lambda, f and a row of coefficients per option) is
+     * less than the geometry above */
+    pthread_mutex_lock(&ctx->lock);
+    const int rc = lvc_modes_main(ctx, &tmpl, outer, 1, (double *)ctx->scratch, out, 0);
+    pthread_mutex_unlock(&ctx->lock);
+    return rc;
   }
   char *base = (char *)ctx->scratch;
   lvc_problem *probs = (lvc_problem *)base;

@@ -158,6 +158,59 @@ int lvc_launch_setup_list(void *stream, int precision, lvc_problem *probs,
                           const lvc_problem *src, const int32_t *list, int nprob,
                           double *geo, void *R);
 
+/* ---- prices by separation of x (lvc_modes_kernels.hip) ---------------------- */
+
+/* One grid: consecutive options that differ only in the strike. */
+typedef struct lvc_mgrid {
+  int32_t nx, ny, nt, xindex, yindex;
+  int32_t first, count; /* its options */
+  int32_t mode0;        /* its nx - 2 modes' place in lambda and f */
+  int32_t lanes, kind;  /* lanes per mode (a power of two), LVC_MODES_* */
+  int64_t coef_off;     /* its count * (nx - 2) coefficients */
+  double s0, t, nu, beta, dx, dy, log_alpha;
+} lvc_mgrid;
+
+/* One wavefront's share: modes first, first + 1, ... of a grid. */
+typedef struct lvc_mtile {
+  int32_t grid, first;
+} lvc_mtile;
+
+#define LVC_MODES_PER_WAVE 4
+/* dynamic LDS of the mode kernel, in blocks of 16 nodes: the weights (and two
+ * blocks read ahead), the modes' values and their scales */
+#define LVC_MODES_BLOCKS(nx) (((nx) - 2 + 15) / 16)
+#define LVC_MODES_LDS(nx)                                                              \
+  (((size_t)(1 + LVC_MODES_PER_WAVE) * LVC_MODES_BLOCKS(nx) + 2) * 16 * sizeof(double) + \
+   (size_t)LVC_MODES_PER_WAVE * LVC_MODES_BLOCKS(nx) * sizeof(int32_t))
+
+/* How a mode's rows lie in a wavefront: 4 or 8 per lane over up to 16 lanes,
+ * 4, 8 or 16 per lane over all 64. */
+enum {
+  LVC_MODES_ROW4 = 0,
+  LVC_MODES_ROW8,
+  LVC_MODES_WAVE4,
+  LVC_MODES_WAVE8,
+  LVC_MODES_WAVE16,
+  LVC_MODES_KINDS
+};
+
+/* Kernel arguments.  One grid (main): `one`, the pointers NULL, option i's
+ * strike 0.001 * i.  Several: grids[] and, per launch, tiles[]. */
+typedef struct lvc_modes_args {
+  lvc_mgrid one;
+  int32_t strike_f32, pad_;
+  const lvc_mgrid *grids;
+  const lvc_mtile *mode_tiles, *tiles[LVC_MODES_KINDS];
+  const double *strikes;     /* [options] */
+  const int32_t *grid_of;    /* [options] */
+  const int32_t *out_index;  /* [options] */
+  double *lambda, *f, *coef;
+} lvc_modes_args;
+
+int lvc_launch_modes(void *stream, const lvc_modes_args *a, int tiles, int max_nx);
+int lvc_launch_evolve(void *stream, const lvc_modes_args *a, int kind, int tiles);
+int lvc_launch_price(void *stream, const lvc_modes_args *a, int n, void *out, int out_f64);
+
 /* Batched f32 tridiagonal solves of [n][m] systems (the ocean-sim entries):
  * form 0 = the scan form (tridagPar), 1 = Thomas (tridagSeq).  scratch holds
  * n*m floats and is needed when m > lvc_tridag_lds_rows(); systems of up to

@@ -1,0 +1,224 @@
+/*
+ * Host side of the prices by separation of x (lvc_modes_kernels.hip): which
+ * problems take it, and the launches of main's one grid and of a batch.
+ */
+#include <math.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include "lvc_runtime.h"
+
+/* Time steps from which the three launches of this path are the faster way
+ * (the sweeps launch two kernels per step). */
+#define MODES_MIN_STEPS 6
+
+static int64_t align64(int64_t v) { return (v + 63) & ~(int64_t)63; }
+
+/* Whether a problem (its initGrid scalars set) separates, in FP64, to the
+ * accuracy of the sweeps.  The weights 4 dx^2 / x^(2 beta) of the interior
+ * nodes have to be positive, fall with x and stay within 1e8 of each other
+ * (the kernel rescales its recurrence every 16 nodes), and x^beta at the
+ * price node within 256 times the first node's (the factor by which the sum
+ * over modes can amplify rounding there); every exponential has to stay far
+ * from the range's ends.  x[0] enters the reference's log(x) too (:63): where
+ * that is not finite every price is NaN, and the sweeps give that. */
+int lvc_modes_fit(const lvc_problem *q) {
+  if (q->status != 0 || q->nt - 1 < MODES_MIN_STEPS)
+    return 0;
+  const double s0 = q->s0, t = q->t, alpha = q->alpha, nu = q->nu, beta = q->beta;
+  const int in_range = s0 > 1e-30 && s0 < 1e30 && t > 1e-30 && t < 1e30 && alpha > 1e-30 &&
+                       alpha < 1e30 && nu > 1e-6 && nu < 1e6 && beta >= 0.0 && beta < 1e3 &&
+                       q->dx > 1e-60 && q->dx < 1e60 && q->dy > 1e-30 && q->dy < 1e30;
+  if (!in_range || !(q->x0log > 0.0 || (q->x0log == 0.0 && beta > 0.0)))
+    return 0;
+  /* 2 y reaches 10 nu sqrt(t) + 2 log(alpha), the time factor nu^2 t */
+  if (!(10.0 * nu * sqrt(t) < 100.0 && nu * nu * t < 100.0))
+    return 0;
+  const double x1 = q->dx - (double)q->xindex * q->dx + s0;
+  const double xn = (double)(q->nx - 2) * q->dx - (double)q->xindex * q->dx + s0;
+  if (!(x1 > 0.0) || !(fabs(2.0 * beta * log(x1)) < 100.0) ||
+      !(fabs(2.0 * beta * log(xn)) < 100.0))
+    return 0;
+  return 2.0 * beta * log(xn / x1) < log(1e8) && beta * log(s0 / x1) < log(256.0);
+}
+
+/* The lanes per mode of a column of ny rows, and how its rows lie in them. */
+static int modes_kind(int ny, int32_t *lanes) {
+  *lanes = ny <= 64 ? lvc_lanes_for(ny, 4) : ny <= 128 ? 16 : 64;
+  return ny <= 64 ? LVC_MODES_ROW4 : ny <= 128 ? LVC_MODES_ROW8
+                  : ny <= 256 ? LVC_MODES_WAVE4 : ny <= 512 ? LVC_MODES_WAVE8
+                  : LVC_MODES_WAVE16;
+}
+
+static lvc_mgrid make_grid(const lvc_problem *q, int first, int count) {
+  lvc_mgrid g;
+  memset(&g, 0, sizeof(g));
+  g.nx = q->nx;
+  g.ny = q->ny;
+  g.nt = q->nt;
+  g.xindex = q->xindex;
+  g.yindex = q->yindex;
+  g.first = first;
+  g.count = count;
+  g.kind = modes_kind(q->ny, &g.lanes);
+  g.s0 = q->s0;
+  g.t = q->t;
+  g.nu = q->nu;
+  g.beta = q->beta;
+  g.dx = q->dx;
+  g.dy = q->dy;
+  g.log_alpha = log(q->alpha);
+  return g;
+}
+
+static int launch(struct futhark_context *ctx, const lvc_modes_args *a, int mode_tiles, int max_nx,
+                  const int64_t tiles[LVC_MODES_KINDS], int n, void *out, int out_f64) {
+  void *st = (void *)ctx->stream;
+  int tok = lvc_prof_begin(ctx, "lvc_modes");
+  int e = lvc_launch_modes(st, a, mode_tiles, max_nx);
+  lvc_prof_end(ctx, tok);
+  for (int kind = LVC_MODES_KINDS - 1; kind >= 0 && !e; kind--) {
+    if (tiles[kind] == 0)
+      continue;
+    tok = lvc_prof_begin(ctx, "lvc_evolve");
+    e = lvc_launch_evolve(st, a, kind, (int)tiles[kind]);
+    lvc_prof_end(ctx, tok);
+  }
+  if (!e) {
+    tok = lvc_prof_begin(ctx, "lvc_price");
+    e = lvc_launch_price(st, a, n, out, out_f64);
+    lvc_prof_end(ctx, tok);
+  }
+  return lvc_check_hip(ctx, e, "price kernels");
+}
+
+/* Doubles of work memory of main: lambda and f per mode, one coefficient per
+ * mode and option. */
+int64_t lvc_modes_main_work(int outer, int nx) {
+  return 2 * align64(nx - 2) + (int64_t)outer * (nx - 2);
+}
+
+/* main's options on q's grid, strikes 0.001 * i: prices into out. */
+int lvc_modes_main(struct futhark_context *ctx, const lvc_problem *q, int outer, int strike_f32,
+                   double *work, void *out, int out_f64) {
+  lvc_modes_args a;
+  memset(&a, 0, sizeof(a));
+  a.one = make_grid(q, 0, outer);
+  a.strike_f32 = strike_f32;
+  const int modes = q->nx - 2, per = 64 / a.one.lanes;
+  a.lambda = work;
+  a.f = work + align64(modes);
+  a.coef = work + 2 * align64(modes);
+  int64_t tiles[LVC_MODES_KINDS] = {0};
+  tiles[a.one.kind] = (modes + per - 1) / per;
+  return launch(ctx, &a, (modes + LVC_MODES_PER_WAVE - 1) / LVC_MODES_PER_WAVE, q->nx, tiles,
+                outer, out, out_f64);
+}
+
+static int by_steps(const void *x, const void *y) {
+  const int64_t a = *(const int64_t *)x, b = *(const int64_t *)y;
+  return (a < b) - (a > b);
+}
+
+/* n problems (initGrid scalars set, lvc_modes_fit), each one's price to
+ * out[out_index].  Runs of consecutive problems that differ only in the
+ * strike share their modes. */
+int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs, void *out,
+                    int out_f64) {
+  if (n == 0)
+    return 0;
+  /* the grids, then tiles counted per kind */
+  lvc_mgrid *grids = malloc((size_t)n * sizeof(*grids));
+  int64_t *order = malloc((size_t)n * sizeof(*order));
+  if (!grids || !order) {
+    free(grids);
+    free(order);
+    lvc_set_error(ctx, "host allocation failed");
+    return 1;
+  }
+  int ng = 0, max_nx = 0;
+  int64_t modes = 0, coefs = 0, nmode = 0, tiles[LVC_MODES_KINDS] = {0};
+  for (int p = 0; p < n;) {
+    int c = 1;
+    while (p + c < n && lvc_same_factor(&probs[p], &probs[p + c]))
+      c++;
+    lvc_mgrid g = make_grid(&probs[p], p, c);
+    const int m = g.nx - 2, per = 64 / g.lanes;
+    g.mode0 = (int32_t)modes;
+    g.coef_off = coefs;
+    modes += m;
+    coefs += (int64_t)c * m;
+    nmode += (m + LVC_MODES_PER_WAVE - 1) / LVC_MODES_PER_WAVE;
+    tiles[g.kind] += (m + per - 1) / per;
+    if (g.nx > max_nx)
+      max_nx = g.nx;
+    order[ng] = (int64_t)g.nt << 24 | ng; /* most steps first */
+    grids[ng++] = g;
+    p += c;
+  }
+  if (modes > INT32_MAX) {
+    free(grids);
+    free(order);
+    lvc_set_error(ctx, "batch too large");
+    return 1;
+  }
+  qsort(order, (size_t)ng, sizeof(*order), by_steps);
+  /* one upload: grids, strikes, tiles, each option's grid and output place */
+  const size_t o_strikes = (size_t)ng * sizeof(lvc_mgrid);
+  const size_t o_mode = o_strikes + (size_t)n * sizeof(double);
+  size_t o_tiles[LVC_MODES_KINDS + 1] = {o_mode + (size_t)nmode * sizeof(lvc_mtile)};
+  for (int i = 0; i < LVC_MODES_KINDS; i++)
+    o_tiles[i + 1] = o_tiles[i] + (size_t)tiles[i] * sizeof(lvc_mtile);
+  const size_t o_grid = o_tiles[LVC_MODES_KINDS];
+  const size_t o_out = o_grid + (size_t)n * sizeof(int32_t);
+  const size_t up = o_out + (size_t)n * sizeof(int32_t);
+  const size_t work = (size_t)(2 * align64(modes) + coefs) * sizeof(double);
+  char *h = malloc(up), *d = NULL;
+  double *w = NULL;
+  int rc = !h;
+  if (rc) {
+    lvc_set_error(ctx, "host allocation failed");
+  } else {
+    memcpy(h, grids, o_strikes);
+    lvc_mtile *mt = (lvc_mtile *)(h + o_mode), *et[LVC_MODES_KINDS];
+    for (int i = 0; i < LVC_MODES_KINDS; i++)
+      et[i] = (lvc_mtile *)(h + o_tiles[i]);
+    for (int i = 0; i < ng; i++) {
+      const int gi = (int)(order[i] & 0xffffff);
+      const lvc_mgrid *g = &grids[gi];
+      const int m = g->nx - 2, per = 64 / g->lanes;
+      for (int k = 0; k < m; k += LVC_MODES_PER_WAVE)
+        *mt++ = (lvc_mtile){gi, k};
+      for (int k = 0; k < m; k += per)
+        *et[g->kind]++ = (lvc_mtile){gi, k};
+      for (int p = g->first; p < g->first + g->count; p++) {
+        ((double *)(h + o_strikes))[p] = probs[p].strike;
+        ((int32_t *)(h + o_grid))[p] = gi;
+        ((int32_t *)(h + o_out))[p] = probs[p].out_index;
+      }
+    }
+    rc = lvc_dev_alloc(ctx, up, (void **)&d) || lvc_dev_alloc(ctx, work, (void **)&w) ||
+         lvc_upload(ctx, d, h, up);
+  }
+  if (!rc) {
+    lvc_modes_args a;
+    memset(&a, 0, sizeof(a));
+    a.grids = (const lvc_mgrid *)d;
+    a.strikes = (const double *)(d + o_strikes);
+    a.mode_tiles = (const lvc_mtile *)(d + o_mode);
+    for (int i = 0; i < LVC_MODES_KINDS; i++)
+      a.tiles[i] = (const lvc_mtile *)(d + o_tiles[i]);
+    a.grid_of = (const int32_t *)(d + o_grid);
+    a.out_index = (const int32_t *)(d + o_out);
+    a.lambda = w;
+    a.f = w + align64(modes);
+    a.coef = w + 2 * align64(modes);
+    rc = launch(ctx, &a, (int)nmode, max_nx, tiles, n, out, out_f64);
+  }
+  lvc_dev_free(ctx, d, up);
+  lvc_dev_free(ctx, w, work);
+  free(h);
+  free(grids);
+  free(order);
+  return rc;
+}

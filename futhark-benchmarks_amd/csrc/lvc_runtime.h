@@ -186,6 +186,16 @@ int lvc_validate_sizes(struct futhark_context *ctx, int64_t nx, int64_t ny,
 void lvc_choose_segs(struct futhark_context *ctx, int precision, int nx, int ny,
                      int *seg_x, int *seg_y);
 int lvc_xshare(struct futhark_context *ctx, int precision);
+/* everything but the strike (and the state) equal */
+int lvc_same_factor(const lvc_problem *a, const lvc_problem *b);
+
+/* prices by separation of x (lvc_modes.c) */
+int lvc_modes_fit(const lvc_problem *q);
+int64_t lvc_modes_main_work(int outer, int nx);
+int lvc_modes_main(struct futhark_context *ctx, const lvc_problem *q, int outer,
+                   int strike_f32, double *work, void *out, int out_f64);
+int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs,
+                    void *out, int out_f64);
 /* LocVolCalib's context-ready hook: the tuning cache and the scratch address */
 void lvc_context_ready(struct futhark_context *ctx);
 
