@@ -4,8 +4,8 @@
  * sizes impose, fixes the move schedule (which depends only on Sobol
  * numbers at data-independent offsets), lays out the swaption tables and
  * the wavefront work lists, and launches csrc/ic_kernels.hip on the
- * context's stream: per call one setup, one initial evaluation, then three
- * launches per MCMC iteration (evaluate, accept, propose), the winner and
+ * context's stream: per call one setup, one initial evaluation, then two
+ * launches per MCMC iteration (evaluate, accept and propose), the winner and
  * its summary, with one synchronisation at the end for the six scalar
  * results.
  */
@@ -62,12 +62,10 @@ static void move_schedule(int32_t pop, int32_t conv, const ic_dirvec *dv, ic_mov
   }
 }
 
-/* The lanes of one evaluation and the schedule periods each lane holds.
- * An iteration's evaluations fill only a few wavefronts per SIMD, so a
- * launch lasts about as long as its slowest wavefront: 2 periods a lane (1
- * for a one-period swaption) measured fastest on the reference's datasets
- * (against 1, 4 and 8), up to 128 periods; longer schedules take 4 or 8
- * periods a lane in the second launch. */
+/* The (virtual) lanes of one evaluation and the schedule periods each lane
+ * holds: 2 (1 for a one-period swaption) up to 128 periods, longer schedules
+ * 4 or 8 in the second launch.  This fixes the order of the sums; how many
+ * virtual lanes a physical one stands for does not (pack_of). */
 static void layout_of(int32_t n, int32_t *lanes, int32_t *per_lane) {
   const int32_t per = n <= 1 ? 1 : n <= 128 ? 2 : n <= 256 ? 4 : 8;
   int32_t l = 1;
@@ -75,6 +73,10 @@ static void layout_of(int32_t n, int32_t *lanes, int32_t *per_lane) {
   *lanes = l;
   *per_lane = per;
 }
+
+/* Wavefronts per CU that a packed launch keeps at least (128 genomes on 196
+ * swaptions: 66 us an iteration with 8, 79 with 4, 73 with 16). */
+#define IC_PACK_WAVES 8
 
 /* Everything one call keeps on the device. */
 typedef struct {
@@ -84,7 +86,7 @@ typedef struct {
   ic_work *work;          /* the work lists below, back to back */
   ic_worklists pop_lists; /* for `pop` genomes */
   ic_worklists one_lists; /* for one genome (the winner's summary) */
-  float *state;  /* genomes, props [pop][5]; logliks, fb [pop]; out [8], winner [8] */
+  float *state;  /* two populations (population_of), then out [8], winner [8] */
   float *terms;  /* [nswap][pop] */
   size_t sw_bytes, per_bytes, work_bytes, state_bytes, terms_bytes;
 } ic_call;
@@ -112,11 +114,29 @@ static void sort_by_periods(int64_t *order, int64_t n, const ic_swaption *sw) {
   }
 }
 
-static int64_t add_work(ic_work *w, int64_t k, int32_t s, int32_t lanes, int32_t npop) {
-  const int32_t per_wave = 64 / lanes;
+/* Packing of a swaption's lanes at most `want` to a physical lane, and to no
+ * fewer than 4 physical lanes: with fewer a wavefront holds so many genomes
+ * that its root searches wait for the slowest of them (packed to one lane, an
+ * iteration of 256 genomes on 196 swaptions took 101 us, to 4 lanes 92; 8
+ * lanes 104). */
+static int32_t pack_of(const ic_swaption *sw, int32_t want) {
+  const int32_t most = sw->lanes / 4 > 1 ? sw->lanes / 4 : 1;
+  return sw->per_lane != 2 ? 1 : want < most ? want : most;
+}
+
+/* Wavefronts of one swaption's evaluations of npop genomes. */
+static int64_t waves_of(const ic_swaption *sw, int32_t want, int32_t npop) {
+  const int64_t per_wave = 64 / (sw->lanes / pack_of(sw, want));
+  return (npop + per_wave - 1) / per_wave;
+}
+
+static int64_t add_work(ic_work *w, int64_t k, int32_t s, const ic_swaption *sw, int32_t want,
+                        int32_t npop) {
+  const int32_t pack = pack_of(sw, want), per_wave = 64 / (sw->lanes / pack);
   for (int32_t g = 0; g < npop; g += per_wave) {
     w[k].swaption = s;
     w[k].genome0 = g;
+    w[k].pack = pack;
     k++;
   }
   return k;
@@ -175,10 +195,21 @@ static int call_prepare(struct futhark_context *ctx, ic_call *c, const lvc_ndarr
       sw[s].lanes = lanes;
       sw[s].per_lane = per;
       nper += n;
-      nwp[per > 2] += (pop + 64 / lanes - 1) / (64 / lanes);
-      nwo[per > 2] += 1;
     }
   }
+  /* A group's physical lanes all do its root finder's own arithmetic, so they
+   * are packed 4 or 2 to a lane while that leaves the device enough
+   * wavefronts. */
+  int32_t want = 4;
+  for (; !rc && want >= 1; want /= 2) {
+    nwp[0] = nwp[1] = 0;
+    for (int64_t s = 0; s < nswap; s++)
+      nwp[sw[s].per_lane > 2] += waves_of(&sw[s], want, pop);
+    if (want == 1 || nwp[0] >= (int64_t)IC_PACK_WAVES * ctx->num_cus)
+      break;
+  }
+  for (int64_t s = 0; !rc && s < nswap; s++)
+    nwo[sw[s].per_lane > 2] += 1;
   ic_work *work = NULL;
   int64_t *order = NULL;
   int64_t total = 0;
@@ -209,7 +240,7 @@ static int call_prepare(struct futhark_context *ctx, ic_call *c, const lvc_ndarr
         for (int64_t r = 0; r < nswap; r++) {
           const int64_t s = order[r];
           if ((sw[s].per_lane > 2) == cl)
-            k = add_work(work, k, (int32_t)s, sw[s].lanes, one ? 1 : pop);
+            k = add_work(work, k, (int32_t)s, &sw[s], one ? 1 : want, one ? 1 : pop);
         }
       }
     for (int cl = 0; cl < IC_LAUNCHES; cl++) {
@@ -239,9 +270,19 @@ static int call_prepare(struct futhark_context *ctx, ic_call *c, const lvc_ndarr
   return rc;
 }
 
+/* The call's population `which` (0 or 1: a step reads one, writes the other). */
+static ic_state population_of(const ic_call *c, int which) {
+  const size_t pop = (size_t)c->pop;
+  float *p = c->state + (size_t)which * 12 * pop;
+  const ic_state s = {p, p + 5 * pop, p + 10 * pop, p + 11 * pop};
+  return s;
+}
+
+static float *results_of(const ic_call *c) { return c->state + 24 * (size_t)c->pop; }
+
 static int alloc_state(struct futhark_context *ctx, ic_call *c) {
   const size_t pop = (size_t)c->pop;
-  c->state_bytes = (pop * 12 + 16) * sizeof(float);
+  c->state_bytes = (2 * pop * 12 + 16) * sizeof(float);
   c->terms_bytes = ((size_t)c->nswap * pop > 0 ? (size_t)c->nswap * pop : 1) * sizeof(float);
   return lvc_dev_alloc(ctx, c->state_bytes, (void **)&c->state) ||
          lvc_dev_alloc(ctx, c->terms_bytes, (void **)&c->terms);
@@ -292,42 +333,43 @@ static int run_calibration(struct futhark_context *ctx, ic_call *c, int32_t conv
                            float *summary) {
   void *st = (void *)ctx->stream;
   const int32_t pop = c->pop;
-  float *genomes = c->state, *props = genomes + 5 * (size_t)pop;
-  float *logliks = props + 5 * (size_t)pop, *fb = logliks + pop;
-  float *out = fb + pop, *winner = out + 8;
+  const ic_state ps[2] = {population_of(c, 0), population_of(c, 1)};
+  float *out = results_of(c), *winner = out + 8;
   const ic_move none = {0, 0, 0, 0};
   /* with profiling on, each launch is timed under its name (events on the
    * context's stream): ic_eval (the population's evaluations), ic_step
    * (accept + propose), ic_other (init, winner, summary) */
   int tok = lvc_prof_begin(ctx, "ic_other");
-  int e = ic_launch_init(st, pop, dv, genomes, props);
+  int e = ic_launch_init(st, pop, dv, ps[0].genomes, ps[0].props);
   lvc_prof_end(ctx, tok);
   if (!e) {
     tok = lvc_prof_begin(ctx, "ic_eval");
-    e = ic_launch_eval(st, c->sw, c->per, &c->pop_lists, genomes, pop, hx, hw, c->nherm,
+    e = ic_launch_eval(st, c->sw, c->per, &c->pop_lists, ps[0].genomes, pop, hx, hw, c->nherm,
                        c->nswap, IC_OUT_TERMS, c->terms, NULL);
     lvc_prof_end(ctx, tok);
   }
   if (!e) {
     tok = lvc_prof_begin(ctx, "ic_step");
-    e = ic_launch_step(st, pop, c->nswap, c->terms, genomes, props, logliks, fb, 1, 0,
+    e = ic_launch_step(st, pop, c->nswap, c->terms, &ps[0], &ps[1], 1, 0,
                        conv > 0 ? &moves[0] : &none, dv, -1, conv, trace);
     lvc_prof_end(ctx, tok);
   }
+  int at = 1; /* the current population */
   for (int32_t it = 0; !e && it < conv; it++) {
     tok = lvc_prof_begin(ctx, "ic_eval");
-    e = ic_launch_eval(st, c->sw, c->per, &c->pop_lists, props, pop, hx, hw, c->nherm,
+    e = ic_launch_eval(st, c->sw, c->per, &c->pop_lists, ps[at].props, pop, hx, hw, c->nherm,
                        c->nswap, IC_OUT_TERMS, c->terms, NULL);
     lvc_prof_end(ctx, tok);
     if (!e) {
       tok = lvc_prof_begin(ctx, "ic_step");
-      e = ic_launch_step(st, pop, c->nswap, c->terms, genomes, props, logliks, fb, 0, acc[it],
+      e = ic_launch_step(st, pop, c->nswap, c->terms, &ps[at], &ps[at ^ 1], 0, acc[it],
                          it + 1 < conv ? &moves[it + 1] : &none, dv, it, conv, trace);
       lvc_prof_end(ctx, tok);
+      at ^= 1;
     }
   }
   tok = lvc_prof_begin(ctx, "ic_other");
-  if (!e) e = ic_launch_winner(st, pop, genomes, logliks, out, winner);
+  if (!e) e = ic_launch_winner(st, pop, ps[at].genomes, ps[at].logliks, out, winner);
   if (!e && c->nswap > 0)
     e = ic_launch_eval(st, c->sw, c->per, &c->one_lists, winner, 1, hx, hw, c->nherm, c->nswap,
                        IC_OUT_SUMMARY, summary, NULL);
@@ -440,7 +482,7 @@ int futhark_entry_main(struct futhark_context *ctx, float *out0, float *out1, fl
                          lvc_array_mem_f32(herm_coefs), lvc_array_mem_f32(herm_weights), NULL,
                          summary->a.mem);
   if (!rc)
-    rc = lvc_check_hip(ctx, hipMemcpyAsync(res, c.state + 12 * (size_t)c.pop, 8 * sizeof(float),
+    rc = lvc_check_hip(ctx, hipMemcpyAsync(res, results_of(&c), 8 * sizeof(float),
                                            hipMemcpyDeviceToHost, ctx->stream),
                        "hipMemcpyAsync") ||
          lvc_check_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
@@ -503,7 +545,7 @@ int interestcalib_trace(struct futhark_context *ctx, const int32_t pop, const in
       const float *src;
       size_t n;
     } cp[] = {{genomes, t.genomes, g_n}, {logliks, t.logliks, l_n}, {props, t.props, pr_n},
-              {fb, t.fb, f_n}, {newl, t.newl, f_n}, {out, c.state + 12 * p, 6},
+              {fb, t.fb, f_n}, {newl, t.newl, f_n}, {out, results_of(&c), 6},
               {summary, sm, (size_t)c.nswap * 3}};
     for (size_t i = 0; !rc && i < sizeof(cp) / sizeof(cp[0]); i++)
       if (cp[i].n)
@@ -560,7 +602,8 @@ int interestcalib_eval(struct futhark_context *ctx, const int32_t ngenomes, cons
   if (!rc) {
     void *st = (void *)ctx->stream;
     const float *hx = lvc_array_mem_f32(herm_coefs), *hw = lvc_array_mem_f32(herm_weights);
-    float *lg = c.state + 10 * np;
+    const ic_state ps[2] = {population_of(&c, 0), population_of(&c, 1)};
+    float *lg = ps[1].logliks;
     const ic_move none = {0, 0, 0, 0};
     ic_dirvec dv;
     memset(&dv, 0, sizeof(dv));
@@ -573,8 +616,8 @@ int interestcalib_eval(struct futhark_context *ctx, const int32_t ngenomes, cons
                            c.nswap, IC_OUT_TERMS, c.terms, NULL);
     }
     if (!e)
-      e = ic_launch_step(st, ngenomes, c.nswap, c.terms, c.state, c.state + 5 * np, lg,
-                         lg + np, 1, 0, &none, &dv, -1, 0, NULL);
+      e = ic_launch_step(st, ngenomes, c.nswap, c.terms, &ps[0], &ps[1], 1, 0, &none, &dv,
+                         -1, 0, NULL);
     rc = lvc_check_hip(ctx, e, "InterestCalib kernels");
     if (!rc && ns > 0)
       rc = lvc_check_hip(ctx, hipMemcpyAsync(quotes, pq, np * ns * sizeof(float),

@@ -32,10 +32,11 @@ typedef struct {
   float tod1, tod2, fact, log_fact;
 } ic_period;
 
-/* One wavefront's work: a swaption and the first of the 64 / lanes genomes
- * it evaluates. */
+/* One wavefront's work: a swaption, the first of the 64 * pack / lanes genomes
+ * it evaluates and how many of the swaption's lanes a physical lane stands
+ * for (1, 2 or 4; 1 unless per_lane is 2). */
 typedef struct {
-  int32_t swaption, genome0;
+  int32_t swaption, genome0, pack, pad;
 } ic_work;
 
 /* The wavefronts of the evaluation launches: [0] swaptions of 1 or 2
@@ -60,6 +61,12 @@ typedef struct {
   int32_t type, base, dim, pad;
 } ic_move;
 
+/* The population: genomes and proposals [pop][5], log-likelihoods and the
+ * proposals' forward/backward ratios [pop]. */
+typedef struct {
+  float *genomes, *props, *logliks, *fb;
+} ic_state;
+
 /* Where ic_launch_step records the trajectory (NULL: not recorded):
  * genomes [conv+1][pop][5] and logliks [conv+1][pop] after the initial
  * evaluation and after each iteration's accept step; props [conv][pop][5],
@@ -72,7 +79,8 @@ typedef struct {
 enum { IC_OUT_TERMS = 0, IC_OUT_PRICES = 1, IC_OUT_SUMMARY = 2 };
 
 /* Genome-independent swaption data: nswap rows of `stride` floats at
- * swaptions; sw[s].n, off, lanes and per_lane set.  Returns 0 or a hipError_t value. */
+ * swaptions; sw[s].n, off, lanes and per_lane set.
+ * Returns 0 or a hipError_t value. */
 int ic_launch_setup(void *stream, const float *swaptions, int64_t stride, int32_t nswap,
                     ic_swaption *sw, ic_period *periods);
 
@@ -89,15 +97,16 @@ int ic_launch_eval(void *stream, const ic_swaption *sw, const ic_period *periods
                    const float *herm_x, const float *herm_w, int32_t nherm, int32_t nswap,
                    int mode, float *out0, float *out1);
 
-/* Two launches: the log-likelihood of each genome, the sum of its terms
- * over the swaptions in a fixed order (32 threads per genome each sum the
+/* One launch: the log-likelihood of each genome, the sum of its terms over
+ * the swaptions in a fixed order (32 threads per genome each sum the
  * swaptions t, t + 32, ... in order, and the partial sums are added
- * pairwise), then, with init, logliks := those sums, else the accept step
- * (:733-745) with draws from Sobol offset acc; then, unless next is no
- * move, the proposals of move `next` into props (ratios into fb).  it is
+ * pairwise); with init those become the log-likelihoods, else the accept step
+ * (:733-745) with draws from Sobol offset acc; then, unless next is no move,
+ * the proposals of move `next` and their ratios.  Reads `from`, writes `to`
+ * (genomes and logliks; props and fb with a move): separate buffers.  it is
  * the iteration whose accept step this is (-1 for init), for the trace. */
-int ic_launch_step(void *stream, int32_t pop, int32_t nswap, const float *terms, float *genomes,
-                   float *props, float *logliks, float *fb, int init, int32_t acc,
+int ic_launch_step(void *stream, int32_t pop, int32_t nswap, const float *terms,
+                   const ic_state *from, const ic_state *to, int init, int32_t acc,
                    const ic_move *next, const ic_dirvec *dv, int32_t it, int32_t conv,
                    const ic_trace *trace);
 

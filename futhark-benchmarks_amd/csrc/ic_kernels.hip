@@ -12,24 +12,35 @@
 // iteration over the schedule is a sum over the lane's K periods followed by
 // a butterfly within the group.  The butterfly hands every lane of the group
 // the same bits, so a group's control flow (the root finder's branches and
-// iteration counts) stays uniform within the group.  An iteration's
-// evaluations (25-50K on the datasets) fill only a few wavefronts per SIMD,
-// so a launch lasts about as long as its slowest wavefront: the host keeps
-// K at 2 (1 for one-period swaptions) up to 128 periods, which measured
-// faster than packing more periods into fewer, longer-running lanes, and
-// every class of such swaptions runs in one launch.
+// iteration counts) stays uniform within the group.  The lanes of a group are
+// virtual: a physical lane stands for V = 1, 2 or 4 of them, and the sums are
+// added in the butterfly's order whatever V, so every result has the same bits
+// for every V.  What a group does once (the root finder's own
+// arithmetic, the quadrature's terms without a period) is done by each of its
+// physical lanes, so fewer of them is less work, and the host packs as far as
+// enough wavefronts remain.
 //
 // What does not depend on the genome (dates, discount factors, the Black
 // quote, each period's c_i * zc(end) / zc(maturity)) is computed once per
 // call by ic_setup_kernel into per-swaption and per-period tables.  The
-// log-likelihood terms land in [swaption][genome] order; ic_accept_kernel
-// sums them per genome in a fixed order and accepts or rejects, and
-// ic_propose_kernel draws the next proposals, so an iteration is three
-// launches, each spread over the device.
+// log-likelihood terms land in [swaption][genome] order; ic_step_kernel sums
+// them per genome in a fixed order, accepts or rejects and draws the next
+// proposals, so an iteration is two launches, each spread over the device.
 //
 // Arithmetic is f32 in the reference's order of operations, compiled
 // without contraction; expf/logf/sqrtf are the device library's, so results
 // differ from a host libm in the last bits.
+//
+// Divisions.  An IEEE division is 11 instructions; half of the evaluation's
+// were that.  rcp_rn's v_rcp_f32 and one Newton step give the correctly
+// rounded reciprocal for every significand (checked over all 2^23), and
+// Markstein's theorem then makes q = a r corrected by one residual step the
+// correctly rounded quotient, in 7 instructions, where neither the reciprocal
+// nor the residual underflows: |b| and |a / b| within 2^+-125, |a| above
+// 2^-101 or 0.  v_div_fixup gives the quotients of zeros, infinities and NaN.
+// The evaluation's operands are far inside (root finder: |f| below 600, every
+// difference an ulp of 1 or more); beyond it a quotient may be off by one
+// denormal ulp.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -118,13 +129,31 @@ __device__ inline int32_t today() { return date_of_gregorian(2012, 1, 1, 12, 0);
 
 __device__ inline float zc(int32_t t) { return expf(-kR * act365(t, today())); }  // :48
 
+__device__ __forceinline__ float rcp_rn(float b) {
+  const float r = __builtin_amdgcn_rcpf(b);
+  return fmaf(fmaf(-b, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float quot(float a, float b) {
+  const float r = rcp_rn(b), q = a * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-b, q, a), r, q), b, a);
+}
+__device__ __forceinline__ float recip(float b) {
+  return __builtin_amdgcn_div_fixupf(rcp_rn(b), b, 1.0f);
+}
+// x / sqrt(2) (the divisor's correctly rounded reciprocal is a constant)
+__device__ __forceinline__ float over_sqrt2(float x) {
+  constexpr float c = 1.41421354f, r = 1.0f / c;  // sqrtf(2.0f)
+  const float q = x * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-c, q, x), r, q), c, x);
+}
+
 // ---- the math module (:56-101) --------------------------------------------
 // Abramowitz & Stegun 7.1.26 without its exp factor
 __device__ inline float erf_poly(float x) {
   const float p = 0.3275911f;
   const float a1 = 0.254829592f, a2 = -0.284496736f, a3 = 1.421413741f, a4 = -1.453152027f,
               a5 = 1.061405429f;
-  const float t = 1.0f / (1.0f + p * x);
+  const float t = recip(1.0f + p * x);
   const float t2 = t * t;
   const float t3 = t * t2;
   const float t4 = t2 * t2;
@@ -133,14 +162,14 @@ __device__ inline float erf_poly(float x) {
 }
 
 __device__ inline float ugaussian_P(float x) {  // :60-93
-  const float u = x / sqrtf(2.0f);
+  const float u = over_sqrt2(x);
   const float e = u < 0.0f ? -(1.0f - erf_poly(-u) * expf(-(u * u)))
                            : 1.0f - erf_poly(u) * expf(-(u * u));
   return 0.5f * (1.0f + e);
 }
 
 __device__ inline float ugaussian_P_exp(float x, float exp_factor) {  // :95-101
-  const float u = fabsf(x / sqrtf(2.0f));
+  const float u = fabsf(over_sqrt2(x));
   const float e = erf_poly(u);
   const float res = 0.5f * e * expf(exp_factor - u * u);
   return 0.0f <= x ? expf(exp_factor) - res : res;
@@ -148,8 +177,8 @@ __device__ inline float ugaussian_P_exp(float x, float exp_factor) {  // :95-101
 
 __device__ inline float log_likelihood(float y_ref, float y) {  // Cauchy, :606-625
   const float gamma = (fabsf(y_ref) / 50.0f) * kCauchyOffs + 0.01f;
-  const float x = (y - y_ref) / gamma;
-  const float pdf = 1.0f / (kPi * gamma * (1.0f + x * x));
+  const float x = quot(y - y_ref, gamma);
+  const float pdf = recip(kPi * gamma * (1.0f + x * x));
   return logf(pdf + 1.0e-20f);
 }
 
@@ -174,13 +203,15 @@ __device__ inline float gene_max(int j) { return j < 3 ? 1.0f - kEps0 : 0.2f; }
 constexpr float kAmplRatio = 0.005f;  // moves_unif_ampl_ratio, :248
 
 // ---- G2++ (:322-413) -------------------------------------------------------------
-__device__ inline float b_fun(float z, float tau) { return (1.0f - expf(-z * tau)) / z; }
+__device__ inline float b_fun(float z, float tau) {
+  return quot(1.0f - expf(-z * tau), z);
+}
 
 __device__ inline float t_fun(float sigma, float x, float tau) {
   const float expxtau = expf(-x * tau);
   const float exp2xtau = expxtau * expxtau;
-  return sigma * sigma / (x * x) *
-         (tau + 2.0f / x * expxtau - 1.0f / (2.0f * x) * exp2xtau - 3.0f / (2.0f * x));
+  return quot(sigma * sigma, x * x) *
+         (tau + quot(2.0f, x) * expxtau - recip(2.0f * x) * exp2xtau - quot(3.0f, 2.0f * x));
 }
 
 struct Genome {
@@ -194,7 +225,7 @@ __device__ inline float bigv(const Genome &g, float tau, float *ba, float *bb) {
   *bb = b_fun(g.b, tau);
   const float t1 = t_fun(sigma, g.a, tau);
   const float t2 = t_fun(g.nu, g.b, tau);
-  const float t3 = 2.0f * g.rho * g.nu * sigma / (g.a * g.b) *
+  const float t3 = quot(2.0f * g.rho * g.nu * sigma, g.a * g.b) *
                    (tau - *ba - *bb + b_fun(g.a + g.b, tau));
   return t1 + t2 + t3;
 }
@@ -204,10 +235,10 @@ __device__ inline float bigv(const Genome &g, float tau, float *ba, float *bb) {
 __device__ inline float bigmx(const Genome &g, float tmat0) {
   const float a = g.a, b = g.b, rho = g.rho, nu = g.nu, sigma = g.sigma;
   const float ts = tmat0, tmatt = 0.0f, tmats = tmat0, t0 = tmat0, s0 = 0.0f;
-  const float tmp1 = (sigma * sigma) / (a * a) + (sigma * rho * nu) / (a * b);
+  const float tmp1 = quot(sigma * sigma, a * a) + quot(sigma * rho * nu, a * b);
   const float tmp2 = 1.0f - expf(-a * ts);
-  const float tmp3 = sigma * sigma / (2.0f * a * a);
-  const float tmp4 = rho * sigma * nu / (b * (a + b));
+  const float tmp3 = quot(sigma * sigma, 2.0f * a * a);
+  const float tmp4 = quot(rho * sigma * nu, b * (a + b));
   const float tmp5 = expf(-a * tmatt) - expf(-a * (tmats + ts));
   const float tmp6 = expf(-b * tmatt) - expf(-b * tmat0 - a * t0 + (a + b) * s0);
   return tmp1 * tmp2 - (tmp3 * tmp5) - (tmp4 * tmp6);
@@ -216,53 +247,109 @@ __device__ inline float bigmx(const Genome &g, float tmat0) {
 __device__ inline float bigmy(const Genome &g, float tmat0) {
   const float a = g.a, b = g.b, rho = g.rho, nu = g.nu, sigma = g.sigma;
   const float ts = tmat0, tmatt = 0.0f, tmats = tmat0, t0 = tmat0, s0 = 0.0f;
-  const float tmp1 = nu * nu / (b * b) + sigma * rho * nu / (a * b);
+  const float tmp1 = quot(nu * nu, b * b) + quot(sigma * rho * nu, a * b);
   const float tmp2 = 1.0f - expf(-b * ts);
-  const float tmp3 = nu * nu / (2.0f * b * b);
-  const float tmp4 = sigma * rho * nu / (a * (a + b));
+  const float tmp3 = quot(nu * nu, 2.0f * b * b);
+  const float tmp4 = quot(sigma * rho * nu, a * (a + b));
   const float tmp5 = expf(-b * tmatt) - expf(-b * (tmats + ts));
   const float tmp6 = expf(-a * tmatt) - expf(-a * tmat0 - b * t0 + (a + b) * s0);
   return tmp1 * tmp2 - (tmp3 * tmp5) - (tmp4 * tmp6);
 }
 
 // ---- group reductions ---------------------------------------------------------------
-// Butterflies over the `lanes` lanes of an evaluation group (a power of two,
-// wave-uniform); every lane of the group ends with the same bits.
-__device__ inline float group_sum(float v, int lanes) {
-  for (int m = 1; m < lanes; m <<= 1) v += __shfl_xor(v, m, 64);
+// Butterflies over the `lanes` physical lanes of an evaluation group (a power
+// of two, wave-uniform); every lane of the group ends with the same bits.
+// Level m adds the lane j ^ m; the levels before it have left the same value
+// in m lanes each, so any lane of the partner's block does: mirrors within 8
+// and 16 lanes, row and half swaps past that, all VALU operands (the
+// ds_bpermute form waited for LDS at each level).
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <typename Op>
+__device__ __forceinline__ float group_all(float v, int lanes, Op op) {
+  if (lanes >= 2) v = op(v, dpp<0xB1>(v));   // quad_perm [1,0,3,2]
+  if (lanes >= 4) v = op(v, dpp<0x4E>(v));   // quad_perm [2,3,0,1]
+  if (lanes >= 8) v = op(v, dpp<0x141>(v));  // row_half_mirror
+  if (lanes >= 16) v = op(v, dpp<0x140>(v)); // row_mirror
+  if (lanes >= 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  if (lanes >= 64) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
   return v;
 }
-__device__ inline float group_max(float v, int lanes) {
-  for (int m = 1; m < lanes; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-  return v;
+__device__ __forceinline__ float group_max(float v, int lanes) {
+  return group_all(v, lanes, [](float a, float b) { return fmaxf(a, b); });
+}
+// The sum over the group of the V virtual lanes' sums on each lane, virtual
+// lane j + lanes * v on lane j: the physical lanes are the butterfly's first
+// levels, each v by itself, then the v.
+template <int V>
+__device__ __forceinline__ float group_sum(const float (&s)[V], int lanes) {
+  float t[V];
+#pragma unroll
+  for (int v = 0; v < V; v++) t[v] = group_all(s[v], lanes, [](float a, float b) { return a + b; });
+  if constexpr (V == 1) return t[0];
+  if constexpr (V == 2) return t[0] + t[1];
+  if constexpr (V == 4) return (t[0] + t[1]) + (t[2] + t[3]);
 }
 
-// One lane's schedule periods (K per lane) and their genome-dependent values.
-template <int K>
+// One lane's schedule periods (K for each of its V virtual lanes) and their
+// genome-dependent values.
+template <int K, int V>
 struct Periods {
-  float bai[K], bbi[K], aici[K], log_aici[K], scale[K], t1cs[K], cs[K];
-  bool valid[K];
+  float bai[K * V], bbi[K * V], aici[K * V], log_aici[K * V], scale[K * V], t1cs[K * V], cs[K * V];
+  bool valid[K * V];
+  int32_t n;  // the slots whose first period (slot0) is below n hold any: wave-uniform
+  int32_t slot0[K * V];
 };
 
-// sum over the group of scales * exp(-bbi * y), minus 1 (:108-117, fid 1)
-template <int K>
-__device__ inline float to_solve(const Periods<K> &P, const float (&ups)[K], float y, int lanes) {
-  float s = 0.0f;
+// expf(x) for |x| < 87: the exponent's integer part and the rest of
+// x log2(e), its product in two parts, by v_exp_f32; without expf's range
+// handling, a third of its instructions.  Equal to expf for every float of
+// that range (compared over all of them).
+__device__ __forceinline__ float exp_mid(float x) {
+  constexpr float c = 0x1.715476p+0f, cc = 0x1.4ae0bep-26f;  // log2(e)
+  const float t = x * c, n = __builtin_rintf(t);
+  const float r = (t - n) + fmaf(x, cc, fmaf(x, c, -t));
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(r), (int)n);
+}
+
+// sum over the group of scales * exp(-bbi * y), minus 1 (:108-117, fid 1).
+// MID: every |bbi * y| is below 87.
+template <bool MID, int K, int V>
+__device__ __forceinline__ float to_solve(const Periods<K, V> &P, const float (&ups)[K * V],
+                                          float y, int lanes) {
+  float s[V];
 #pragma unroll
-  for (int k = 0; k < K; k++)
-    if (P.valid[k]) s += ups[k] * expf(-P.bbi[k] * y);
-  return group_sum(s, lanes) - 1.0f;
+  for (int v = 0; v < V; v++) {
+    s[v] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      if (P.slot0[v * K + k] >= P.n) continue;
+      const float x = -P.bbi[v * K + k] * y;
+      const float t = ups[v * K + k] * (MID ? exp_mid(x) : expf(x));
+      s[v] += P.valid[v * K + k] ? t : 0.0f;
+    }
+  }
+  return group_sum<V>(s, lanes) - 1.0f;
 }
 
 // rootFinding_Brent (:124-185); the loop ends where the reference's
 // iterations stop changing its state
-template <int K>
-__device__ float brent(const Periods<K> &P, const float (&ups)[K], int lanes, float lb, float ub,
+template <bool MID, int K, int V>
+__device__ float brent(const Periods<K, V> &P, const float (&ups)[K * V], int lanes, float lb, float ub,
                        float tol, int32_t iter_max, float *err) {
   tol = tol <= 0.0f ? 1.0e-9f : tol;
   iter_max = iter_max <= 0 ? 10000 : iter_max;
   float a = lb, b = ub;
-  float fa = to_solve(P, ups, a, lanes), fb = to_solve(P, ups, b, lanes);
+  float fa = to_solve<MID>(P, ups, a, lanes), fb = to_solve<MID>(P, ups, b, lanes);
   if (0.0f <= fa * fb) {
     *err = 0.0f <= a ? INFINITY : -INFINITY;
     return 0.0f;
@@ -271,43 +358,40 @@ __device__ float brent(const Periods<K> &P, const float (&ups)[K], int lanes, fl
     float t = fa; fa = fb; fb = t;
     t = a; a = b; b = t;
   }
-  float c = a, fc = fa, d = 0.0f;
-  bool mflag = true;
+  // x: |b - c| after a bisection, |c - d| after an interpolation
+  float c = a, fc = fa, x = fabsf(b - c);
   for (int32_t i = 0; i < iter_max; i++) {
     if (fb == 0.0f || fabsf(b - a) < tol) break;
     float s;
     if (fa == fc || fb == fc) {
-      s = b - fb * (b - a) / (fb - fa);
+      s = b - quot(fb * (b - a), fb - fa);
     } else {
-      const float s1 = (a * fb * fc) / ((fa - fb) * (fa - fc));
-      const float s2 = (b * fa * fc) / ((fb - fa) * (fb - fc));
-      const float s3 = (c * fa * fb) / ((fc - fa) * (fc - fb));
+      // each difference once: negation is exact
+      const float ab = fa - fb, ac = fa - fc, bc = fb - fc;
+      const float s1 = quot(a * fb * fc, ab * ac);
+      const float s2 = quot(b * fa * fc, -ab * bc);
+      const float s3 = quot(c * fa * fb, ac * bc);
       s = s1 + s2 + s3;
     }
-    if (!((3.0f * a + b) / 4.0f <= s && s <= b) ||
-        (mflag && fabsf(b - c) / 2.0f <= fabsf(s - b)) ||
-        (!mflag && fabsf(c - d) / 2.0f <= fabsf(s - b)) ||
-        (mflag && fabsf(b - c) <= fabsf(tol)) || (!mflag && fabsf(c - d) <= fabsf(tol))) {
-      mflag = true;
-      s = (a + b) / 2.0f;
-    } else {
-      mflag = false;
-    }
-    const float fs = to_solve(P, ups, s, lanes);
-    d = c;
+    const bool bisect = !((3.0f * a + b) / 4.0f <= s && s <= b) || x / 2.0f <= fabsf(s - b) ||
+                        x <= fabsf(tol);
+    s = bisect ? (a + b) / 2.0f : s;
+    const float fs = to_solve<MID>(P, ups, s, lanes);
+    const float was_c = c;
     c = b;
     fc = fb;
-    if (fa * fs < 0.0f) {
-      b = s;
-      fb = fs;
-    } else {
-      a = s;
-      fa = fs;
-    }
-    if (fabsf(fa) < fabsf(fb)) {
-      float t = a; a = b; b = t;
-      t = fa; fa = fb; fb = t;
-    }
+    const bool left = fa * fs < 0.0f;
+    b = left ? s : b;
+    fb = left ? fs : fb;
+    a = left ? a : s;
+    fa = left ? fa : fs;
+    const bool swap = fabsf(fa) < fabsf(fb);
+    const float t = a, ft = fa;
+    a = swap ? b : a;
+    fa = swap ? fb : fa;
+    b = swap ? t : b;
+    fb = swap ? ft : fb;
+    x = fabsf(bisect ? b - c : c - was_c);
   }
   *err = fb;
   return b;
@@ -318,38 +402,51 @@ struct Scals {
 };
 
 // exactYhat (:418-481); bb_first and bb_last are bbi[0] and bbi[n-1]
-template <int K>
-__device__ float exact_yhat(const Periods<K> &P, int n, int lanes, const Scals &sc, float x) {
+template <int K, int V>
+__device__ float exact_yhat(const Periods<K, V> &P, int n, int lanes, const Scals &sc, float x) {
   const float k = -3.71901648545568f;
-  float ups[K];
-  float up = 0.0f, lo = -INFINITY;
+  float ups[K * V], part[V], lo = -INFINITY;
 #pragma unroll
-  for (int q = 0; q < K; q++) {
-    ups[q] = 0.0f;
-    if (P.valid[q]) {
-      const float baix = P.bai[q] * x;
-      ups[q] = P.aici[q] * expf(-baix);
-      up += ups[q];
-      lo = fmaxf(lo, (P.log_aici[q] - baix) / P.bbi[q]);
+  for (int v = 0; v < V; v++) {
+    part[v] = 0.0f;
+#pragma unroll
+    for (int q = v * K; q < (v + 1) * K; q++) {
+      ups[q] = 0.0f;
+      if (P.slot0[q] >= P.n) continue;
+      if (P.valid[q]) {
+        const float baix = P.bai[q] * x;
+        ups[q] = P.aici[q] * expf(-baix);
+        part[v] += ups[q];
+        lo = fmaxf(lo, quot(P.log_aici[q] - baix, P.bbi[q]));
+      }
     }
   }
-  up = group_sum(up, lanes);
+  const float up = group_sum<V>(part, lanes);
   lo = group_max(lo, lanes);
   if (n < 2) return lo;
   const float log_s = logf(up);
-  float tmp = log_s / sc.bb_last;
+  float tmp = quot(log_s, sc.bb_last);
   if (!(tmp <= 0.0f)) {
-    tmp = log_s / sc.bb_first;
+    tmp = quot(log_s, sc.bb_first);
     tmp = 0.0f <= tmp ? tmp : -INFINITY;
   }
   const float yl = lo - kEps, yu = tmp + kEps;
-  const float y0 = sc.sigmay * (sc.rhoxy * (x - sc.mux) / sc.sigmax + k * sc.rhoxycs) -
-                   sc.rhoxyc / sc.b + sc.muy;
-  const float y1 = sc.sigmay * (sc.rhoxy * (x - sc.mux) / sc.sigmax - k * sc.rhoxycs) + sc.muy;
+  const float rx = quot(sc.rhoxy * (x - sc.mux), sc.sigmax);
+  const float y0 = sc.sigmay * (rx + k * sc.rhoxycs) - quot(sc.rhoxyc, sc.b) + sc.muy;
+  const float y1 = sc.sigmay * (rx - k * sc.rhoxycs) + sc.muy;
   if (y1 <= yl) return y1 + 1.0f;
   if (yu <= y0) return y0 - 1.0f;
-  float err;
-  const float root = brent(P, ups, lanes, fmaxf(yl, y0), fminf(yu, y1), 1.0e-4f, 1000, &err);
+  const float ya = fmaxf(yl, y0), yb = fminf(yu, y1);
+  // every iterate lies between the two, so the wavefront knows its range of
+  // exponents (a NaN is in none)
+  float bb = 0.0f;
+#pragma unroll
+  for (int q = 0; q < K * V; q++) bb = fmaxf(bb, P.bbi[q]);
+  float err, root;
+  if (__ballot(!(bb * fabsf(ya) < 86.0f && bb * fabsf(yb) < 86.0f)) == 0)
+    root = brent<true>(P, ups, lanes, ya, yb, 1.0e-4f, 1000, &err);
+  else
+    root = brent<false>(P, ups, lanes, ya, yb, 1.0e-4f, 1000, &err);
   if (err == -INFINITY) return y0 - 1.0f;
   if (err == INFINITY) return y1 + 1.0f;
   return root;
@@ -444,13 +541,17 @@ struct EvalArgs {
   float *out0, *out1;
 };
 
-// One wavefront's evaluations, K schedule periods a lane.
-template <int K>
+// One wavefront's evaluations, K schedule periods for each of a lane's V
+// virtual lanes: period jv + S.lanes * k for virtual lane jv = j + lanes * v.
+// (With neighbouring virtual lanes on one physical lane the sums are shorter,
+// but a schedule of 20 periods on 16 lanes of 2 then keeps 8 slots busy for
+// lane 0's sake, where this needs 5.)
+template <int K, int V>
 __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, const ic_swaption S,
                                           const int lane) {
-  const int lanes = S.lanes;
+  const int lanes = S.lanes / V;  // physical lanes of a group
   const int n = S.n;
-  const int j = lane & (lanes - 1);
+  const int j = lane & (lanes - 1), group0 = lane & ~(lanes - 1);
   int32_t gi = wk.genome0 + lane / lanes;
   const bool store = gi < A.npop && j == 0;
   gi = gi < A.npop ? gi : A.npop - 1;
@@ -465,34 +566,36 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
   const float muy = 0.0f - bigmy(g, tmat0);
   const float sqrt_bfun_a = sqrtf(b_fun(2.0f * g.a, tmat0));
   const float sqrt_bfun_b = sqrtf(b_fun(2.0f * g.b, tmat0));
-  const float rhoxy = g.rho * b_fun(g.a + g.b, tmat0) / (sqrt_bfun_a * sqrt_bfun_b);
+  const float rhoxy = quot(g.rho * b_fun(g.a + g.b, tmat0), sqrt_bfun_a * sqrt_bfun_b);
   const float sigmax = g.sigma * sqrt_bfun_a;
   const float sigmay = g.nu * sqrt_bfun_b;
   const float rhoxyc = 1.0f - rhoxy * rhoxy;
   const float rhoxycs = sqrtf(rhoxyc);
   const float sigmay_rhoxycs = sigmay * rhoxycs;
-  const float t4 = (rhoxy * sigmay) / sigmax;
+  const float t4 = quot(rhoxy * sigmay, sigmax);
 
-  // the schedule's periods (:549-583), period j + lanes * k on this lane
-  Periods<K> P;
+  // the schedule's periods (:549-583)
+  Periods<K, V> P;
+  P.n = n;
 #pragma unroll
-  for (int k = 0; k < K; k++) {
-    const int i = j + lanes * k;
-    P.valid[k] = i < n;
-    P.bai[k] = P.bbi[k] = P.aici[k] = P.log_aici[k] = P.scale[k] = P.t1cs[k] = P.cs[k] = 0.0f;
-    if (P.valid[k]) {
+  for (int q = 0; q < K * V; q++) {
+    P.slot0[q] = lanes * (q / K) + S.lanes * (q % K);
+    const int i = P.slot0[q] + j;
+    P.valid[q] = i < n;
+    P.bai[q] = P.bbi[q] = P.aici[q] = P.log_aici[q] = P.scale[q] = P.t1cs[q] = P.cs[q] = 0.0f;
+    if (P.valid[q]) {
       const ic_period pe = A.per[S.off + i];
       float bai, bbi;
       const float v0_end = bigv(g, pe.tod1, &dum1, &dum2);
       const float vt_end = bigv(g, pe.tod2, &bai, &bbi);
       const float expo_aici = 0.5f * (vt_end - v0_end + v0_mat);
-      P.bai[k] = bai;
-      P.bbi[k] = bbi;
-      P.aici[k] = pe.fact * expf(expo_aici);
-      P.log_aici[k] = pe.log_fact + expo_aici;
-      P.scale[k] = 0.0f - (bai + bbi * t4);
-      P.cs[k] = pe.fact;
-      P.t1cs[k] = bbi * (mux * t4 - (muy - 0.5f * rhoxyc * sigmay * sigmay * bbi)) + expo_aici;
+      P.bai[q] = bai;
+      P.bbi[q] = bbi;
+      P.aici[q] = pe.fact * expf(expo_aici);
+      P.log_aici[q] = pe.log_fact + expo_aici;
+      P.scale[q] = 0.0f - (bai + bbi * t4);
+      P.cs[q] = pe.fact;
+      P.t1cs[q] = bbi * (mux * t4 - (muy - 0.5f * rhoxyc * sigmay * sigmay * bbi)) + expo_aici;
     }
   }
   Scals sc;
@@ -509,32 +612,63 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
 
   // :586-591
   const float eps = 0.5f * sigmax;
-  const float f = exact_yhat(P, n, lanes, sc, mux);
-  const float gg = exact_yhat(P, n, lanes, sc, mux + eps);
-  const float h = exact_yhat(P, n, lanes, sc, mux - eps);
-  const float df = 0.5f * (gg - h) / eps;
+  // one copy of the root search for the three: a launch's wavefronts run four
+  // instantiations of this function, which have to share the instruction cache
+  float f = 0.0f, gg = 0.0f, h = 0.0f;
+#pragma unroll 1
+  for (int r = 0; r < 3; r++) {
+    const float x = r == 0 ? mux : r == 1 ? mux + eps : mux - eps;
+    const float y = exact_yhat(P, n, lanes, sc, x);
+    f = r == 0 ? y : f;
+    gg = r == 1 ? y : gg;
+    h = r == 2 ? y : h;
+  }
+  const float df = quot(0.5f * (gg - h), eps);
   const float sqrt2sigmax = sqrtf(2.0f) * sigmax;
-  const float t2 = rhoxy / (sigmax * rhoxycs);
+  const float t2 = quot(rhoxy, sigmax * rhoxycs);
 
-  // Gauss-Hermite (:594-620)
+  // Gauss-Hermite (:594-620).  A point's terms without a period, h1 and
+  // P(-h1), are made by one lane of the group each, `lanes` points at a time,
+  // and its weight by one lane of the wavefront, 64 points at a time.
   float accum = 0.0f;
-  for (int q = 0; q < A.nherm; q++) {
-    const float x_quad = A.hx[q], w_quad = A.hw[q];
-    const float x = sqrt2sigmax * x_quad + mux;
-    const float yhat_x = f + df * (x - mux);
-    const float h1 = ((yhat_x - muy) / sigmay_rhoxycs) - t2 * (x - mux);
-    float part = 0.0f;
-#pragma unroll
-    for (int k = 0; k < K; k++)
-      if (P.valid[k]) {
-        const float h2 = h1 + P.bbi[k] * sigmay_rhoxycs;
-        const float expo_aici = P.t1cs[k] + P.scale[k] * x;
-        part += P.cs[k] * ugaussian_P_exp(-h2, expo_aici);
+  for (int q64 = 0; q64 < A.nherm; q64 += 64) {
+    const int end64 = A.nherm - q64 < 64 ? A.nherm - q64 : 64;
+    const int mine = q64 + (lane < end64 ? lane : 0);
+    const float hx = A.hx[mine];
+    const float tmp = sqrtf(2.0f) * hx;
+    const float hw = A.hw[mine] * expf(-0.5f * tmp * tmp);
+    for (int q0 = 0; q0 < end64; q0 += lanes) {
+      float own_h1, own_p;
+      {
+        const float x = sqrt2sigmax * __shfl(hx, q0 + j) + mux;
+        const float yhat_x = f + df * (x - mux);
+        own_h1 = quot(yhat_x - muy, sigmay_rhoxycs) - t2 * (x - mux);
+        own_p = ugaussian_P(-own_h1);
       }
-    const float accum1 = group_sum(part, lanes);
-    const float tmp = sqrtf(2.0f) * x_quad;
-    const float t1 = expf(-0.5f * tmp * tmp);
-    accum = accum + w_quad * t1 * (ugaussian_P(-h1) - accum1);
+      const int here = end64 - q0 < lanes ? end64 - q0 : lanes;
+      for (int t = 0; t < here; t++) {
+        const float h1 = __shfl(own_h1, group0 + t), p1 = __shfl(own_p, group0 + t);
+        const float x_quad = __int_as_float(
+            __builtin_amdgcn_readlane(__float_as_int(hx), q0 + t));
+        const float w_t1 = __int_as_float(
+            __builtin_amdgcn_readlane(__float_as_int(hw), q0 + t));
+        const float x = sqrt2sigmax * x_quad + mux;
+        float part[V];
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          part[v] = 0.0f;
+#pragma unroll
+          for (int q = v * K; q < (v + 1) * K; q++) {
+            if (P.slot0[q] >= n) continue;
+            const float h2 = h1 + P.bbi[q] * sigmay_rhoxycs;
+            const float expo_aici = P.t1cs[q] + P.scale[q] * x;
+            const float term = P.cs[q] * ugaussian_P_exp(-h2, expo_aici);
+            part[v] += P.valid[q] ? term : 0.0f;
+          }
+        }
+        accum = accum + w_t1 * (p1 - group_sum<V>(part, lanes));
+      }
+    }
   }
   const float price = S.zc_mat * (accum / sqrtf(kPi));
   if (!store) return;
@@ -552,17 +686,22 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
   }
 }
 
-// Swaptions of 1 or 2 periods a lane (up to 128 periods) in one launch, so
-// the classes share the device; a class is uniform per wavefront.
+// Swaptions of 1 or 2 periods a virtual lane (up to 128 periods) in one
+// launch, so the classes share the device; a class is uniform per wavefront.
 __global__ __launch_bounds__(256) void ic_eval_kernel(EvalArgs A) {
   const int32_t wv = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (wv >= A.nwork) return;  // wave-uniform
   const ic_work wk = A.work[wv];
   const ic_swaption S = A.sw[wk.swaption];
+  const int lane = threadIdx.x & 63;
   if (S.per_lane == 1)
-    eval_wave<1>(A, wk, S, threadIdx.x & 63);
+    eval_wave<1, 1>(A, wk, S, lane);
+  else if (wk.pack == 1)
+    eval_wave<2, 1>(A, wk, S, lane);
+  else if (wk.pack == 2)
+    eval_wave<2, 2>(A, wk, S, lane);
   else
-    eval_wave<2>(A, wk, S, threadIdx.x & 63);
+    eval_wave<2, 4>(A, wk, S, lane);
 }
 
 // Longer schedules (4 or 8 periods a lane, up to 512 periods): more registers.
@@ -572,136 +711,162 @@ __global__ __launch_bounds__(256) void ic_eval_long_kernel(EvalArgs A) {
   const ic_work wk = A.work[wv];
   const ic_swaption S = A.sw[wk.swaption];
   if (S.per_lane == 4)
-    eval_wave<4>(A, wk, S, threadIdx.x & 63);
+    eval_wave<4, 1>(A, wk, S, threadIdx.x & 63);
   else
-    eval_wave<8>(A, wk, S, threadIdx.x & 63);
+    eval_wave<8, 1>(A, wk, S, threadIdx.x & 63);
 }
 
 // ---- accept / propose ------------------------------------------------------------------
 struct StepArgs {
   int32_t pop, nswap;
   const float *terms;
-  float *genomes, *props, *logliks, *fb;
+  ic_state from, to;
   int32_t init, acc, it, conv;
   ic_move next;
   ic_dirvec dv;
   ic_trace trace;
 };
 
-constexpr int kSumLanes = 32;  // threads per genome of the accept kernel
+constexpr int kSumLanes = 32;  // threads per genome of the step kernel
 
-// The log-likelihood of each genome (:639-645) and the accept step
-// (:733-745).  Accepting needs only the genome's own terms, so the genomes
-// spread over the device: 32 lanes per genome, lane t summing the swaptions
-// t, t + 32, ... in order (one memory round trip on the datasets), the 32
-// partial sums added pairwise with the same bits on every lane.
-__global__ __launch_bounds__(256) void ic_accept_kernel(StepArgs A) {
-  const int32_t pop = A.pop;
-  const int t = threadIdx.x & (kSumLanes - 1);
-  const int32_t i = (int32_t)(blockIdx.x * (256 / kSumLanes) + threadIdx.x / kSumLanes);
-  float s = 0.0f;
-  if (i < pop) {
-    // this lane's terms w = t, t + kSumLanes, ... in that order, eight loads
-    // issued before their sums (a lane has ceil(nswap / kSumLanes) terms: 7
-    // for 196 swaptions, so one batch)
-    const float *col = A.terms + i;
-    for (int32_t w = t; w < A.nswap; w += 8 * kSumLanes) {
-      float v[8];
+// The log-likelihoods (:639-645) of N genomes ids[]: 32 lanes per genome, lane
+// t summing the swaptions t, t + 32, ... in order, the 32 partial sums added
+// pairwise with the same bits on every lane.  Eight terms of every genome are
+// loaded before their sums (a lane has ceil(nswap / 32) terms: 7 for 196
+// swaptions, so one memory round trip).
+template <int N>
+__device__ __forceinline__ void loglik_sums(const StepArgs &A, const int32_t (&ids)[N], int t,
+                                            float (&s)[N]) {
+#pragma unroll
+  for (int m = 0; m < N; m++) s[m] = 0.0f;
+  for (int32_t w = t; w < A.nswap; w += 8 * kSumLanes) {
+    float v[N][8];
+#pragma unroll
+    for (int m = 0; m < N; m++)
 #pragma unroll
       for (int k = 0; k < 8; k++) {
         const int32_t wk = w + k * kSumLanes;
-        v[k] = wk < A.nswap ? col[(int64_t)wk * pop] : 0.0f;
+        v[m][k] = wk < A.nswap ? A.terms[(int64_t)wk * A.pop + ids[m]] : 0.0f;
       }
 #pragma unroll
+    for (int m = 0; m < N; m++)
+#pragma unroll
       for (int k = 0; k < 8; k++)
-        if (w + k * kSumLanes < A.nswap) s += v[k];
-    }
+        if (w + k * kSumLanes < A.nswap) s[m] += v[m][k];
   }
-  for (int m = 1; m < kSumLanes; m <<= 1) s += __shfl_xor(s, m, 64);
-  if (i >= pop || t != 0) return;
-  if (A.init) {
-    A.logliks[i] = s;
-  } else {
-    const float acceptance = fminf(1.0f, expf(s - A.logliks[i]) * A.fb[i]);
-    const float r = sobol(A.dv, A.acc + i);
-    if (A.trace.newl) A.trace.newl[(int64_t)A.it * pop + i] = s;
-    if (r < acceptance) {
-      // genomes and proposals are separate arrays: the five loads first
-      float g[5];
-      for (int j = 0; j < 5; j++) g[j] = A.props[5 * i + j];
-      for (int j = 0; j < 5; j++) A.genomes[5 * i + j] = g[j];
-      A.logliks[i] = s;
-    }
-  }
-  if (A.trace.genomes) {
-    const int64_t row = (int64_t)(A.it + 1) * pop + i;
-    float g[5];
-    for (int j = 0; j < 5; j++) g[j] = A.genomes[5 * i + j];
-    for (int j = 0; j < 5; j++) A.trace.genomes[5 * row + j] = g[j];
-    A.trace.logliks[row] = A.logliks[i];
-  }
+#pragma unroll
+  for (int m = 0; m < N; m++)
+    for (int b = 1; b < kSumLanes; b <<= 1) s[m] += __shfl_xor(s[m], b, 64);
 }
 
-// The next iteration's proposals (:655-724), one thread per genome, after
-// every genome's accept step (differential evolution reads other genomes).
-__global__ __launch_bounds__(256) void ic_propose_kernel(StepArgs A) {
+// Whether genome i's proposal, of log-likelihood s, is accepted (:733-745).
+__device__ __forceinline__ bool accepted(const StepArgs &A, int32_t i, float s) {
+  const float acceptance = fminf(1.0f, expf(s - A.from.logliks[i]) * A.from.fb[i]);
+  return sobol(A.dv, A.acc + i) < acceptance;
+}
+
+// One step of the population: each genome's log-likelihood and acceptance,
+// then its next proposal (:655-724), 32 lanes per genome, a lane per gene.
+// Differential evolution reads two other genomes after their accept steps;
+// their log-likelihoods are summed here again, so that no second launch has
+// to wait for all of the first (which took 6 us of an iteration).  The old
+// state is only read and the new one only written: nothing races.
+__global__ __launch_bounds__(256) void ic_step_kernel(StepArgs A) {
   const int32_t pop = A.pop;
-  const int32_t i = (int32_t)(blockIdx.x * 256 + threadIdx.x);
-  if (i >= pop) return;
+  const int t = threadIdx.x & (kSumLanes - 1);
+  const int32_t at = (int32_t)(blockIdx.x * (256 / kSumLanes) + threadIdx.x / kSumLanes);
+  const int32_t i = at < pop ? at : pop - 1;  // spare lanes follow the last genome
   const ic_move mv = A.next;
-  float out[5], fb = 1.0f;
-  if (mv.type == 1 || mv.type == 2) {  // mutate_dims_all / mutate_dims_one (:278-306)
-    for (int j = 0; j < 5; j++) {
-      const float r01 = sobol(A.dv, 5 * i + mv.base + j);
-      const float ampl = mv.type == 1 || j == mv.dim ? kAmplRatio : 0.0f;
-      const float g_min = gene_min(j), g_max = gene_max(j);
-      const float gene = A.genomes[5 * i + j], prop = A.props[5 * i + j];
-      const float amplitude = fabsf((g_max - g_min) * ampl);  // mutateHelper, :250-266
-      const float semiamplitude = amplitude / 2.0f;
-      float tmp_min_max = fminf(g_max, gene + semiamplitude);
-      float tmp_max_min = fmaxf(g_min, gene - semiamplitude);
-      const float forward_range = tmp_min_max - tmp_max_min;
-      tmp_min_max = fminf(g_max, prop + semiamplitude);
-      tmp_max_min = fmaxf(g_min, prop - semiamplitude);
-      const float backward_range = tmp_min_max - tmp_max_min;
-      const float bf = 0.0f < semiamplitude ? backward_range / forward_range : 1.0f;
-      const float ng = gene + amplitude * r01 - semiamplitude;
-      out[j] = fmaxf(g_min, fminf(g_max, ng));  // constrainDim, :268-270
-      fb = j == 0 ? bf : fb * bf;
-    }
-  } else {  // DE (:700-723, mcmc_DE :309-320)
-    const int32_t kk = 8 * i + mv.base;
+  const bool de = mv.type == 3;
+  // DE's genomes k and l and its gamma (:700-712)
+  int32_t k = i, l = i;
+  float gamma1 = 0.0f;
+  const int32_t kk = 8 * i + mv.base;
+  if (de) {
     const float s1 = sobol(A.dv, kk);
-    int32_t k = (int32_t)(s1 * (float)(pop - 1));
+    k = (int32_t)(s1 * (float)(pop - 1));
     int32_t cand_ub = pop - 1;
     if (k == i) {
       k = pop - 1;
       cand_ub = pop - 2;
     }
     const float s2 = sobol(A.dv, kk + 1);
-    int32_t l = (int32_t)(s2 * (float)cand_ub);
+    l = (int32_t)(s2 * (float)cand_ub);
     if (l == i || l == k) l = cand_ub;
     const float s3 = sobol(A.dv, kk + 2);
     const float gamma_avg = 2.38f / sqrtf(2.0f * 5.0f);
-    const float ampl_ratio = 0.1f * kAmplRatio;
-    const float gamma1 = gamma_avg - 0.5f + s3;
-    for (int j = 0; j < 5; j++) {
-      const float r01 = sobol(A.dv, kk + 3 + j);
-      const float mm_diff = gene_max(j) - gene_min(j);
-      const float amplitude = fabsf(mm_diff * ampl_ratio);
-      const float semiamplitude = amplitude / 2.0f;
-      const float perturb = amplitude * r01 - semiamplitude;
-      const float ng = A.genomes[5 * i + j] + perturb +
-                       gamma1 * (A.genomes[5 * k + j] - A.genomes[5 * l + j]);
-      out[j] = fmaxf(gene_min(j), fminf(gene_max(j), ng));
-    }
+    gamma1 = gamma_avg - 0.5f + s3;
   }
-  for (int j = 0; j < 5; j++) A.props[5 * i + j] = out[j];
-  A.fb[i] = fb;
-  if (A.trace.props && A.it + 1 < A.conv) {
-    const int64_t row = (int64_t)(A.it + 1) * pop + i;
-    for (int j = 0; j < 5; j++) A.trace.props[5 * row + j] = out[j];
-    A.trace.fb[row] = fb;
+  float s;
+  bool take = false, take_k = false, take_l = false;
+  if (de) {
+    const int32_t ids[3] = {i, k, l};
+    float sums[3];
+    loglik_sums<3>(A, ids, t, sums);
+    s = sums[0];
+    if (!A.init) {
+      take = accepted(A, i, s);
+      take_k = accepted(A, k, sums[1]);
+      take_l = accepted(A, l, sums[2]);
+    }
+  } else {
+    const int32_t ids[1] = {i};
+    float sums[1];
+    loglik_sums<1>(A, ids, t, sums);
+    s = sums[0];
+    if (!A.init) take = accepted(A, i, s);
+  }
+  const int j = t < 5 ? t : 0;  // this lane's gene
+  auto gene_of = [&](int32_t g, bool taken) {
+    return taken ? A.from.props[5 * g + j] : A.from.genomes[5 * g + j];
+  };
+  const float gene = gene_of(i, take);
+  const float loglik = A.init || take ? s : A.from.logliks[i];
+  float out = 0.0f, bf = 1.0f;
+  if (mv.type == 1 || mv.type == 2) {  // mutate_dims_all / mutate_dims_one (:278-306)
+    const float r01 = sobol(A.dv, 5 * i + mv.base + j);
+    const float ampl = mv.type == 1 || j == mv.dim ? kAmplRatio : 0.0f;
+    const float g_min = gene_min(j), g_max = gene_max(j);
+    const float prop = A.from.props[5 * i + j];
+    const float amplitude = fabsf((g_max - g_min) * ampl);  // mutateHelper, :250-266
+    const float semiamplitude = amplitude / 2.0f;
+    float tmp_min_max = fminf(g_max, gene + semiamplitude);
+    float tmp_max_min = fmaxf(g_min, gene - semiamplitude);
+    const float forward_range = tmp_min_max - tmp_max_min;
+    tmp_min_max = fminf(g_max, prop + semiamplitude);
+    tmp_max_min = fmaxf(g_min, prop - semiamplitude);
+    const float backward_range = tmp_min_max - tmp_max_min;
+    bf = 0.0f < semiamplitude ? backward_range / forward_range : 1.0f;
+    const float ng = gene + amplitude * r01 - semiamplitude;
+    out = fmaxf(g_min, fminf(g_max, ng));  // constrainDim, :268-270
+  } else if (de) {  // :713-723, mcmc_DE :309-320
+    const float ampl_ratio = 0.1f * kAmplRatio;
+    const float r01 = sobol(A.dv, kk + 3 + j);
+    const float mm_diff = gene_max(j) - gene_min(j);
+    const float amplitude = fabsf(mm_diff * ampl_ratio);
+    const float semiamplitude = amplitude / 2.0f;
+    const float perturb = amplitude * r01 - semiamplitude;
+    const float ng = gene + perturb + gamma1 * (gene_of(k, take_k) - gene_of(l, take_l));
+    out = fmaxf(gene_min(j), fminf(gene_max(j), ng));
+  }
+  // the genes' ratios multiplied in order
+  const int first = threadIdx.x & 63 & ~(kSumLanes - 1);
+  float fb = __shfl(bf, first);
+  for (int m = 1; m < 5; m++) fb = fb * __shfl(bf, first + m);
+  if (at >= pop) return;
+  const int64_t row = (int64_t)(A.it + 1) * pop + i;
+  if (t < 5) {
+    A.to.genomes[5 * i + j] = gene;
+    if (mv.type) A.to.props[5 * i + j] = out;
+    if (A.trace.genomes) A.trace.genomes[5 * row + j] = gene;
+    if (mv.type && A.trace.props && A.it + 1 < A.conv) A.trace.props[5 * row + j] = out;
+  }
+  if (t == 0) {
+    A.to.logliks[i] = loglik;
+    if (mv.type) A.to.fb[i] = fb;
+    if (A.trace.newl && !A.init) A.trace.newl[(int64_t)A.it * pop + i] = s;
+    if (A.trace.genomes) A.trace.logliks[row] = loglik;
+    if (mv.type && A.trace.props && A.it + 1 < A.conv) A.trace.fb[row] = fb;
   }
 }
 
@@ -763,7 +928,7 @@ extern "C" int ic_launch_eval(void *stream, const ic_swaption *sw, const ic_peri
     if (wl->nwork[c] <= 0) continue;
     A.work = wl->work[c];
     A.nwork = wl->nwork[c];
-    const dim3 grid((wl->nwork[c] + 3) / 4), block(256);
+    const dim3 grid((A.nwork + 3) / 4), block(256);
     if (c == 0)
       hipLaunchKernelGGL(ic_eval_kernel, grid, block, 0, (hipStream_t)stream, A);
     else
@@ -773,17 +938,15 @@ extern "C" int ic_launch_eval(void *stream, const ic_swaption *sw, const ic_peri
 }
 
 extern "C" int ic_launch_step(void *stream, int32_t pop, int32_t nswap, const float *terms,
-                              float *genomes, float *props, float *logliks, float *fb, int init,
-                              int32_t acc, const ic_move *next, const ic_dirvec *dv, int32_t it,
-                              int32_t conv, const ic_trace *trace) {
+                              const ic_state *from, const ic_state *to, int init, int32_t acc,
+                              const ic_move *next, const ic_dirvec *dv, int32_t it, int32_t conv,
+                              const ic_trace *trace) {
   StepArgs A;
   A.pop = pop;
   A.nswap = nswap;
   A.terms = terms;
-  A.genomes = genomes;
-  A.props = props;
-  A.logliks = logliks;
-  A.fb = fb;
+  A.from = *from;
+  A.to = *to;
   A.init = init;
   A.acc = acc;
   A.it = it;
@@ -797,11 +960,8 @@ extern "C" int ic_launch_step(void *stream, int32_t pop, int32_t nswap, const fl
   }
   if (pop <= 0) return 0;
   const int64_t per_block = 256 / kSumLanes;
-  hipLaunchKernelGGL(ic_accept_kernel, dim3((unsigned)((pop + per_block - 1) / per_block)),
+  hipLaunchKernelGGL(ic_step_kernel, dim3((unsigned)((pop + per_block - 1) / per_block)),
                      dim3(256), 0, (hipStream_t)stream, A);
-  if (A.next.type != 0)
-    hipLaunchKernelGGL(ic_propose_kernel, dim3((unsigned)((pop + 255) / 256)), dim3(256), 0,
-                       (hipStream_t)stream, A);
   return (int)hipGetLastError();
 }
 
