@@ -101,7 +101,7 @@ int futhark_entry_main(struct futhark_context *ctx, struct futhark_f32_1d **out0
                   "has %lld", contract_number, (long long)cK, (long long)K);
     return 1;
   }
-  if (B > OP_DV_STRIDE) {
+  if (B > OP_MAX_BITS) {
     lvc_set_error(ctx, "main: %lld direction-vector bits (at most 32: testBit shifts "
                   "an i32, :17-18)", (long long)B);
     return 1;
@@ -112,13 +112,14 @@ int futhark_entry_main(struct futhark_context *ctx, struct futhark_f32_1d **out0
   }
   const int launch = priced && num_mc_it > 0 && M > 0;
   pthread_mutex_lock(&ctx->lock);
-  void *out = NULL, *dv = NULL, *partial = NULL;
-  /* the padded direction vectors, then the bridge check's flag */
-  const size_t dv_bytes = (size_t)(D * U) * OP_DV_STRIDE * sizeof(int32_t) + sizeof(int32_t);
-  const size_t part_bytes = (size_t)op_blocks(num_mc_it) * (size_t)M * sizeof(double);
+  void *out = NULL, *tables = NULL, *partial = NULL;
+  const size_t tab_bytes = op_table_bytes(contract_number);
+  const size_t part_bytes = (size_t)op_blocks(contract_number, num_mc_it) *
+                            (size_t)(M < OP_MAX_MODELS ? M : OP_MAX_MODELS) * sizeof(double);
   int rc = lvc_dev_alloc(ctx, (size_t)M * sizeof(float), &out);
   if (!rc && launch)
-    rc = lvc_dev_alloc(ctx, dv_bytes, &dv) || lvc_dev_alloc(ctx, part_bytes, &partial);
+    rc = (tab_bytes && lvc_dev_alloc(ctx, tab_bytes, &tables)) ||
+         lvc_dev_alloc(ctx, part_bytes, &partial);
   if (!rc && launch) {
     op_args a;
     memset(&a, 0, sizeof(a));
@@ -135,7 +136,7 @@ int futhark_entry_main(struct futhark_context *ctx, struct futhark_f32_1d **out0
     a.bbd = bb_data->a.mem;
     a.N = num_mc_it;
     int tok = lvc_prof_begin(ctx, "op_paths");
-    int e = op_launch((void *)ctx->stream, contract_number, &a, dir_vs->a.mem, dv,
+    int e = op_launch((void *)ctx->stream, contract_number, &a, dir_vs->a.mem, tables,
                       partial, out);
     lvc_prof_end(ctx, tok);
     rc = lvc_check_hip(ctx, e, "option pricing kernels");
@@ -155,8 +156,8 @@ int futhark_entry_main(struct futhark_context *ctx, struct futhark_f32_1d **out0
   }
   if (partial)
     lvc_dev_free(ctx, partial, part_bytes);
-  if (dv)
-    lvc_dev_free(ctx, dv, dv_bytes);
+  if (tables)
+    lvc_dev_free(ctx, tables, tab_bytes);
   struct futhark_f32_1d *arr = NULL;
   if (!rc) {
     arr = lvc_array_adopt_f32(out, M);

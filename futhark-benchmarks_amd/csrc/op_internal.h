@@ -3,11 +3,13 @@
 #ifndef OP_INTERNAL_H
 #define OP_INTERNAL_H
 
+#include <stddef.h>
 #include <stdint.h>
 
-#define OP_MAX_MODELS 8
-#define OP_MAX_BLOCKS 2048 /* workgroups of the path kernel at most */
-#define OP_DV_STRIDE 32    /* ints per padded direction-vector row */
+#define OP_MAX_BITS 32
+#define OP_MAX_MODELS 4     /* models that share a pass over the paths */
+#define OP_FEW_BLOCKS 1024  /* workgroups at most, contracts 1 and 2 */
+#define OP_MANY_BLOCKS 2048 /* and contract 3 */
 
 #ifdef __cplusplus
 extern "C" {
@@ -24,17 +26,19 @@ typedef struct {
   int64_t N;           /* paths */
 } op_args;
 
-/* Workgroups of the path kernel for N paths (OP_MAX_BLOCKS at most): the
- * f64 partial sums it writes are [op_blocks(N)][M]. */
-int op_blocks(int64_t paths);
+/* Workgroups of the path kernel for N paths: the f64 partial sums it writes
+ * are [op_blocks(contract, N)][models of the pass]. */
+int op_blocks(int contract, int64_t paths);
 
-/* Pads dir_vs ([dims][bits]) into dv ([dims][OP_DV_STRIDE] ints, then one
- * more: whether the bridge tables let the paths skip zeroing their rows),
- * runs the paths and writes the mean payoff per model to out[M]; every launch on
- * `stream` (a hipStream_t).  The contract fixes dims (1, 15 or 1101).
- * Returns 0 or a hipError_t value. */
+/* Bytes of the tables that op_launch makes for a contract (0: none). */
+size_t op_table_bytes(int contract);
+
+/* Makes the contract's tables, runs the paths and writes the mean payoff per
+ * model to out[M]; every launch on `stream` (a hipStream_t).  dir_vs
+ * [dims][bits]; the contract fixes dims (1, 15 or 1101).  Returns 0 or a
+ * hipError_t value. */
 int op_launch(void *stream, int contract, const op_args *A, const int32_t *dir_vs,
-              int32_t *dv, double *partial, float *out);
+              void *tables, double *partial, float *out);
 
 #ifdef __cplusplus
 }
