@@ -44,7 +44,8 @@ typedef struct lvc_problem {
   int32_t fac_src;         /* problem whose y factor table this one uses */
   int32_t grid32;          /* initGrid's scalars in f32 (the reference's f32 entry) */
   int32_t out_index;       /* where the gather writes this problem's price */
-  int32_t pad_;
+  int32_t fac_dt;          /* complement of the bits of the f32 time step whose y
+                            * factor the problem's table holds; 0: none */
   int64_t state_off;       /* element offset of R and Y */
   int64_t geo_off;         /* element offset into the f64 geometry buffer */
   double s0, strike, t, alpha, nu, beta;
