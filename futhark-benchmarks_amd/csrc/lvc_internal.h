@@ -154,10 +154,12 @@ int lvc_launch_gather_list(void *stream, int precision, lvc_problem *probs,
                            const int32_t *list, int nprob, const void *R, void *out,
                            int out_f64);
 /* Sets up problems list[0 .. nprob-1] from the descriptors src[0 .. nprob-1]
- * (stored to probs[list[i]]). */
+ * (stored to probs[list[i]]), and copies `bytes` (a multiple of 16) from copy_src
+ * to copy_dst.  src, list and copy_src may be pinned host memory. */
 int lvc_launch_setup_list(void *stream, int precision, lvc_problem *probs,
                           const lvc_problem *src, const int32_t *list, int nprob,
-                          double *geo, void *R);
+                          double *geo, void *R, const void *copy_src, void *copy_dst,
+                          int64_t bytes);
 
 /* ---- prices by separation of x (lvc_modes_kernels.hip) ---------------------- */
 

@@ -317,13 +317,21 @@ struct Taps {
 // Grid: (problems, row chunks); chunk 0 also writes the geometry and resets
 // the time index.  With `list`, block i sets up problem list[i] from the
 // descriptor src[i] (chunk 0 stores it, time index set, to probs[list[i]]).
+// Blocks past the problems copy ncopy 16-byte words: the server's tick takes its
+// new descriptors and tile list from pinned host memory in this one launch.
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void lvc_setup_kernel(lvc_problem *probs,
                                                         const lvc_problem *src,
-                                                        const int32_t *list,
-                                                        double *geo, T *R) {
+                                                        const int32_t *list, int nprob,
+                                                        double *geo, T *R, const uint4 *copy_src,
+                                                        uint4 *copy_dst, int ncopy) {
 #pragma clang fp contract(off)
+  if ((int)blockIdx.x >= nprob) {
+    const int i = ((blockIdx.x - nprob) * gridDim.y + blockIdx.y) * blockDim.x + threadIdx.x;
+    if (i < ncopy) copy_dst[i] = copy_src[i];
+    return;
+  }
   lvc_problem &dst = probs[list ? list[blockIdx.x] : blockIdx.x];
   const lvc_problem pr = list ? src[blockIdx.x] : dst;
   const int nx = pr.nx, ny = pr.ny;
@@ -1413,20 +1421,31 @@ int lvc_seg_supported(int seg, int ysweep) {
 
 int lvc_launch_setup_list(void *stream, int precision, lvc_problem *probs,
                           const lvc_problem *src, const int32_t *list, int nprob,
-                          double *geo, void *R) {
-  if (nprob <= 0) return 0;
+                          double *geo, void *R, const void *copy_src, void *copy_dst,
+                          int64_t bytes) {
+  constexpr int kRows = 8, kThreads = 256;
+  if (nprob < 0 || bytes < 0 || bytes % 16 != 0 || bytes / 16 > INT32_MAX)
+    return (int)hipErrorInvalidValue;
+  const int ncopy = (int)(bytes / 16), per = kRows * kThreads;
+  const int blocks = nprob + (ncopy + per - 1) / per;
+  if (blocks == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid(nprob, 8);
+  const dim3 grid(blocks, kRows);
   if (precision == LVC_FP64)
-    lvc_setup_kernel<double><<<grid, 256, 0, st>>>(probs, src, list, geo, (double *)R);
+    lvc_setup_kernel<double><<<grid, kThreads, 0, st>>>(probs, src, list, nprob, geo, (double *)R,
+                                                        (const uint4 *)copy_src,
+                                                        (uint4 *)copy_dst, ncopy);
   else
-    lvc_setup_kernel<float><<<grid, 256, 0, st>>>(probs, src, list, geo, (float *)R);
+    lvc_setup_kernel<float><<<grid, kThreads, 0, st>>>(probs, src, list, nprob, geo, (float *)R,
+                                                       (const uint4 *)copy_src, (uint4 *)copy_dst,
+                                                       ncopy);
   return (int)hipGetLastError();
 }
 
 int lvc_launch_setup(void *stream, int precision, lvc_problem *probs, int nprob,
                      double *geo, void *R) {
-  return lvc_launch_setup_list(stream, precision, probs, nullptr, nullptr, nprob, geo, R);
+  return lvc_launch_setup_list(stream, precision, probs, nullptr, nullptr, nprob, geo, R, nullptr,
+                               nullptr, 0);
 }
 
 int lvc_launch_xsweep(void *stream, int precision, int seg,

@@ -309,19 +309,16 @@ void lvc_dev_free(struct futhark_context *ctx, void *ptr, size_t bytes) {
 
 /* ---- staged uploads ----------------------------------------------------- */
 
-int lvc_upload(struct futhark_context *ctx, void *dst, const void *src,
-               size_t bytes) {
-  if (bytes == 0)
-    return 0;
-  /* The staging buffer is a bump arena: uploads take consecutive regions and
-   * only a wrap-around waits, for the copies enqueued so far (they run in
-   * stream order, so the event after the latest one covers them all). */
+/* The staging buffer is a bump arena of pinned memory: takers get consecutive
+ * regions and only a wrap-around waits, for what was enqueued so far to read
+ * them (in stream order, so the event after the latest covers all). */
+void *lvc_stage(struct futhark_context *ctx, size_t bytes) {
   const size_t need = (bytes + 255) & ~(size_t)255;
   if (ctx->stage_used + need > ctx->stage_size) {
     if (ctx->stage_pending) {
       if (lvc_check_hip(ctx, hipEventSynchronize(ctx->stage_done),
                         "hipEventSynchronize"))
-        return 1;
+        return NULL;
       ctx->stage_pending = 0;
     }
     ctx->stage_used = 0;
@@ -333,23 +330,36 @@ int lvc_upload(struct futhark_context *ctx, void *dst, const void *src,
       if (lvc_check_hip(ctx, hipHostMalloc(&ctx->stage, sz, hipHostMallocDefault),
                         "hipHostMalloc")) {
         ctx->stage_size = 0;
-        return 1;
+        return NULL;
       }
       ctx->stage_size = sz;
     }
   }
   char *region = (char *)ctx->stage + ctx->stage_used;
-  memcpy(region, src, bytes);
-  if (lvc_check_hip(ctx, hipMemcpyAsync(dst, region, bytes,
-                                        hipMemcpyHostToDevice, ctx->stream),
-                    "hipMemcpyAsync"))
-    return 1;
+  ctx->stage_used += need;
+  return region;
+}
+
+int lvc_stage_read(struct futhark_context *ctx) {
   if (lvc_check_hip(ctx, hipEventRecord(ctx->stage_done, ctx->stream),
                     "hipEventRecord"))
     return 1;
-  ctx->stage_used += need;
   ctx->stage_pending = 1;
   return 0;
+}
+
+int lvc_upload(struct futhark_context *ctx, void *dst, const void *src,
+               size_t bytes) {
+  if (bytes == 0)
+    return 0;
+  void *region = lvc_stage(ctx, bytes);
+  if (!region)
+    return 1;
+  memcpy(region, src, bytes);
+  return lvc_check_hip(ctx, hipMemcpyAsync(dst, region, bytes,
+                                           hipMemcpyHostToDevice, ctx->stream),
+                       "hipMemcpyAsync") ||
+         lvc_stage_read(ctx);
 }
 
 /* ---- profiling ---------------------------------------------------------- */

@@ -123,6 +123,11 @@ void lvc_dev_free(struct futhark_context *ctx, void *ptr, size_t bytes);
  * on ctx->stream and the host data may be reused on return */
 int lvc_upload(struct futhark_context *ctx, void *dst, const void *src,
                size_t bytes);
+/* a region of the pinned staging memory, which kernels on ctx->stream may read
+ * in place; the caller fills it, enqueues its readers and calls
+ * lvc_stage_read before the next region is taken.  NULL on failure. */
+void *lvc_stage(struct futhark_context *ctx, size_t bytes);
+int lvc_stage_read(struct futhark_context *ctx);
 
 /* the 1-D arrays' device memory and length; adopt wraps device memory from
  * lvc_dev_alloc as an array that futhark_free_*_1d returns to the pool */

@@ -15,12 +15,19 @@
  *   1. admits queued requests, in arrival order, while a slot is free and the
  *      arena has an extent for the request's grids (in-order: the first
  *      request that does not fit waits for memory, and the ones behind it
- *      with it); each admission uploads its descriptor and runs the setup
- *      kernel for that slot;
+ *      with it); one launch sets up the admitted slots;
  *   2. launches the x sweep and the y sweep once over every resident request
  *      (each advances one time step);
- *   3. gathers the price of every request that has just done its last step,
- *      copies those prices back and frees their slots.
+ *   3. gathers the price of every request that has just done its last step
+ *      and frees their slots.
+ * A tick of small requests is its launches' latency, and a copy between two
+ * kernels costs as much as a small kernel: so nothing is copied.  The setup
+ * kernel reads the admitted descriptors from pinned host memory and brings
+ * the tile list to the device; the gather kernel reads its list from there and
+ * writes the prices there; and a finished request's tiles stay in the list (its
+ * time index makes them return at once) until requests are admitted or half of
+ * the list is dead.  A burst of 96 requests of 32 .. 128 points and 16 .. 64
+ * steps on 64 slots: 3.55 ms with 2.4 copies a tick, 2.28 now.
  * Every kernel runs on the context's stream, so the slot reuse in step 1 is
  * ordered after the completed request's last use.  A request's arithmetic
  * depends only on its own inputs and the server's fixed segment lengths,
@@ -58,7 +65,7 @@ typedef struct {
 #define LVC_SRV_PENDING 4
 typedef struct {
   hipEvent_t done;
-  double *host;  /* pinned, max_slots prices */
+  double *host;  /* pinned, max_slots prices, then the slots they are of */
   int64_t *ids;  /* request ids, in gather order */
   int count;
   int64_t seq;
@@ -84,21 +91,19 @@ struct lvc_server {
   double *d_geo;
   void *d_R, *d_Y;
   void *d_yfac; /* y factor tables per slot (column y sweep only) */
-  int32_t *h_fprobs, *d_fprobs; /* resident slots (factor workgroups) */
+  int32_t *h_fprobs, *d_fprobs; /* resident slots (factor workgroups), after the tiles */
   int nfac;
-  double *d_out;
-  /* admission: the tick's new descriptors and their slots, staged on the
-   * device for one setup launch */
-  lvc_problem *h_adm, *d_adm;
-  int32_t *h_admslot, *d_admslot;
+  /* admission: the tick's new descriptors and their slots */
+  lvc_problem *h_adm;
+  int32_t *h_admslot;
   int nadm;
-  /* completions: the tick's finished slots, one gather launch */
-  int32_t *h_done, *d_done;
+  /* completions: the tick's finished slots */
+  int32_t *h_done;
   completion_batch pend[LVC_SRV_PENDING];
   int64_t pend_head, pend_tail; /* batches pend_head .. pend_tail-1 in flight */
   /* tiles of the resident set */
   lvc_tile *h_tiles, *d_tiles;
-  int nxt, nyt, tiles_cap, tiles_dirty, ylds;
+  int nxt, nyt, dead, tiles_cap, tiles_dirty, ylds;
   /* queue and results */
   queued_req *queue;
   int64_t qhead, qtail, qcap;
@@ -124,6 +129,20 @@ static int64_t slot_bytes(const struct lvc_server *s, int col) {
          (col ? LVC_YFAC_LEN * (int64_t)s->real + (int64_t)sizeof(int32_t) : 0) +
          (int64_t)sizeof(double) + SLOT_MAX_TILES * (int64_t)sizeof(lvc_tile) +
          2 * (int64_t)sizeof(int32_t);
+}
+
+static size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
+
+/* the device tile list and, after its tiles, the resident slots */
+static size_t tile_bytes(const struct lvc_server *s) {
+  return align16((size_t)s->tiles_cap * sizeof(lvc_tile)) +
+         align16((size_t)s->max_slots * sizeof(int32_t));
+}
+
+/* tiles of a request: x (rows per workgroup) and y */
+static int request_tiles(const struct lvc_server *s, const lvc_problem *q) {
+  const int rows = LVC_BLOCK / lvc_lanes_for(q->nx, s->seg_x);
+  return (q->ny + rows - 1) / rows + q->ytiles;
 }
 
 /* First-fit extent of `len` elements; -1 when none is free. */
@@ -243,7 +262,8 @@ struct lvc_server *lvc_server_new(struct futhark_context *ctx, int32_t max_slots
   }
   for (int b = 0; !rc && b < LVC_SRV_PENDING; b++)
     rc = lvc_check_hip(ctx, hipHostMalloc((void **)&s->pend[b].host,
-                                          (size_t)max_slots * sizeof(double),
+                                          (size_t)max_slots *
+                                              (sizeof(double) + sizeof(int32_t)),
                                           hipHostMallocDefault), "hipHostMalloc") ||
          lvc_check_hip(ctx, hipEventCreateWithFlags(&s->pend[b].done, hipEventDisableTiming),
                        "hipEventCreate");
@@ -252,14 +272,9 @@ struct lvc_server *lvc_server_new(struct futhark_context *ctx, int32_t max_slots
          lvc_dev_alloc(ctx, (size_t)max_slots * s->slot_geo * sizeof(double), (void **)&s->d_geo) ||
          lvc_dev_alloc(ctx, (size_t)arena * s->real, &s->d_R) ||
          lvc_dev_alloc(ctx, (size_t)arena * s->real, &s->d_Y) ||
-         lvc_dev_alloc(ctx, (size_t)max_slots * sizeof(double), (void **)&s->d_out) ||
-         lvc_dev_alloc(ctx, (size_t)s->tiles_cap * sizeof(lvc_tile), (void **)&s->d_tiles) ||
-         lvc_dev_alloc(ctx, (size_t)max_slots * sizeof(lvc_problem), (void **)&s->d_adm) ||
-         lvc_dev_alloc(ctx, (size_t)max_slots * sizeof(int32_t), (void **)&s->d_admslot) ||
-         lvc_dev_alloc(ctx, (size_t)max_slots * sizeof(int32_t), (void **)&s->d_done) ||
+         lvc_dev_alloc(ctx, tile_bytes(s), (void **)&s->d_tiles) ||
          (lvc_seg_is_col(s->seg_y) &&
-          (lvc_dev_alloc(ctx, (size_t)max_slots * LVC_YFAC_LEN * s->real, &s->d_yfac) ||
-           lvc_dev_alloc(ctx, (size_t)max_slots * sizeof(int32_t), (void **)&s->d_fprobs)));
+          lvc_dev_alloc(ctx, (size_t)max_slots * LVC_YFAC_LEN * s->real, &s->d_yfac));
   if (!rc)
     rc = lvc_upload(ctx, s->d_slots, s->h_slots, (size_t)max_slots * sizeof(lvc_problem));
   pthread_mutex_unlock(&ctx->lock);
@@ -280,16 +295,10 @@ void lvc_server_free(struct lvc_server *s) {
   lvc_dev_free(ctx, s->d_geo, (size_t)s->max_slots * s->slot_geo * sizeof(double));
   lvc_dev_free(ctx, s->d_R, (size_t)s->arena_elems * s->real);
   lvc_dev_free(ctx, s->d_Y, (size_t)s->arena_elems * s->real);
-  lvc_dev_free(ctx, s->d_out, (size_t)s->max_slots * sizeof(double));
   if (s->d_yfac)
     lvc_dev_free(ctx, s->d_yfac, (size_t)s->max_slots * LVC_YFAC_LEN * s->real);
-  if (s->d_fprobs)
-    lvc_dev_free(ctx, s->d_fprobs, (size_t)s->max_slots * sizeof(int32_t));
   if (s->d_tiles)
-    lvc_dev_free(ctx, s->d_tiles, (size_t)s->tiles_cap * sizeof(lvc_tile));
-  lvc_dev_free(ctx, s->d_adm, (size_t)s->max_slots * sizeof(lvc_problem));
-  lvc_dev_free(ctx, s->d_admslot, (size_t)s->max_slots * sizeof(int32_t));
-  lvc_dev_free(ctx, s->d_done, (size_t)s->max_slots * sizeof(int32_t));
+    lvc_dev_free(ctx, s->d_tiles, tile_bytes(s));
   for (int b = 0; b < LVC_SRV_PENDING; b++) {
     if (s->pend[b].host)
       (void)hipHostFree(s->pend[b].host);
@@ -411,15 +420,12 @@ static int rebuild_tiles(struct lvc_server *s) {
   }
   s->nxt = nx_t;
   s->nyt = ny_t;
+  s->dead = 0;
   s->tiles_dirty = 0;
-  if (s->d_fprobs && s->nfac &&
-      lvc_upload(ctx, s->d_fprobs, s->h_fprobs, (size_t)s->nfac * sizeof(int32_t)))
-    return 1;
-  return need ? lvc_upload(ctx, s->d_tiles, s->h_tiles, (size_t)need * sizeof(lvc_tile)) : 0;
+  return 0;
 }
 
-static int admit(struct lvc_server *s) {
-  struct futhark_context *ctx = s->ctx;
+static void admit(struct lvc_server *s) {
   int slot = 0;
   while (s->qhead < s->qtail && s->nresident < s->max_slots) {
     const queued_req *qr = &s->queue[s->qhead];
@@ -463,20 +469,36 @@ static int admit(struct lvc_server *s) {
     s->h_admslot[s->nadm] = slot;
     s->nadm++;
   }
-  /* the tick's admissions: their descriptors and slots in one upload each,
-   * set up by one launch (which also stores each descriptor to its slot) */
-  if (s->nadm > 0) {
-    const int n = s->nadm;
-    s->nadm = 0;
-    if (lvc_upload(ctx, s->d_adm, s->h_adm, (size_t)n * sizeof(lvc_problem)) ||
-        lvc_upload(ctx, s->d_admslot, s->h_admslot, (size_t)n * sizeof(int32_t)))
-      return 1;
-    const int e = lvc_launch_setup_list((void *)ctx->stream, s->precision, s->d_slots, s->d_adm,
-                                        s->d_admslot, n, s->d_geo, s->d_R);
-    if (lvc_check_hip(ctx, e, "setup kernel"))
-      return 1;
-  }
-  return 0;
+}
+
+/* Brings the tick's admissions and, if it changed, the tile list to the device:
+ * one region of pinned memory, read by one launch. */
+static int set_up(struct lvc_server *s) {
+  struct futhark_context *ctx = s->ctx;
+  if (s->tiles_dirty && rebuild_tiles(s))
+    return 1;
+  const int n = s->nadm;
+  s->nadm = 0;
+  const size_t desc = align16((size_t)n * sizeof(lvc_problem));
+  const size_t slots = align16((size_t)n * sizeof(int32_t));
+  const size_t tiles = align16((size_t)(s->nxt + s->nyt) * sizeof(lvc_tile));
+  const size_t fprobs = align16((size_t)s->nfac * sizeof(int32_t));
+  if (desc + tiles == 0)
+    return 0;
+  char *r = lvc_stage(ctx, desc + slots + tiles + fprobs);
+  if (!r)
+    return 1;
+  memcpy(r, s->h_adm, (size_t)n * sizeof(lvc_problem));
+  memcpy(r + desc, s->h_admslot, (size_t)n * sizeof(int32_t));
+  char *list = r + desc + slots;
+  memcpy(list, s->h_tiles, (size_t)(s->nxt + s->nyt) * sizeof(lvc_tile));
+  memcpy(list + tiles, s->h_fprobs, (size_t)s->nfac * sizeof(int32_t));
+  s->d_fprobs = (int32_t *)((char *)s->d_tiles + tiles);
+  const int e = lvc_launch_setup_list((void *)ctx->stream, s->precision, s->d_slots,
+                                      (const lvc_problem *)r, (const int32_t *)(r + desc), n,
+                                      s->d_geo, s->d_R, list, s->d_tiles,
+                                      (int64_t)(tiles + fprobs));
+  return lvc_check_hip(ctx, e, "setup kernel") || lvc_stage_read(ctx);
 }
 
 /* Publishes the completion batches whose price copies have landed, in
@@ -514,9 +536,9 @@ int32_t lvc_server_step(struct lvc_server *s) {
   pthread_mutex_lock(&ctx->lock);
   int rc = publish(s, -1);
   if (!rc)
-    rc = admit(s);
+    admit(s);
   if (!rc && s->tiles_dirty)
-    rc = rebuild_tiles(s);
+    rc = set_up(s);
   int32_t ndone = 0;
   if (!rc && s->nresident > 0) {
     void *st = (void *)ctx->stream;
@@ -535,7 +557,7 @@ int32_t lvc_server_step(struct lvc_server *s) {
       lvc_prof_end(ctx, tok);
       rc = lvc_check_hip(ctx, e, "y sweep kernel");
     }
-    /* completions: one gather over the finished slots, its prices copied
+    /* completions: one gather over the finished slots, its prices written
      * to a pinned buffer behind the launches and published once landed
      * (poll waits for them); the slots and arena extents are free at once,
      * since every later use of them runs after the gather in stream order */
@@ -551,15 +573,12 @@ int32_t lvc_server_step(struct lvc_server *s) {
       if (s->pend_tail - s->pend_head == LVC_SRV_PENDING)
         rc = publish(s, s->pend_head);            /* the ring is full: the oldest */
       cb = &s->pend[s->pend_tail % LVC_SRV_PENDING];
+      int32_t *list = (int32_t *)(cb->host + s->max_slots);
+      memcpy(list, s->h_done, (size_t)ndone * sizeof(int32_t));
       if (!rc)
-        rc = lvc_upload(ctx, s->d_done, s->h_done, (size_t)ndone * sizeof(int32_t));
-      if (!rc)
-        rc = lvc_check_hip(ctx, lvc_launch_gather_list(st, s->precision, s->d_slots, s->d_done,
-                                                       ndone, s->d_R, s->d_out, 1),
+        rc = lvc_check_hip(ctx, lvc_launch_gather_list(st, s->precision, s->d_slots, list, ndone,
+                                                       s->d_R, cb->host, 1),
                            "gather kernel") ||
-             lvc_check_hip(ctx, hipMemcpyAsync(cb->host, s->d_out, (size_t)ndone * sizeof(double),
-                                               hipMemcpyDeviceToHost, ctx->stream),
-                           "hipMemcpyAsync") ||
              lvc_check_hip(ctx, hipEventRecord(cb->done, ctx->stream), "hipEventRecord");
       if (!rc) {
         cb->count = ndone;
@@ -580,7 +599,9 @@ int32_t lvc_server_step(struct lvc_server *s) {
         s->h_slots[i].k = -1;
         s->nresident--;
         s->completed++;
-        s->tiles_dirty = 1;
+        s->dead += request_tiles(s, &s->h_slots[i]);
+        if (2 * s->dead > s->nxt + s->nyt)
+          s->tiles_dirty = 1;
       }
     }
   }
