@@ -2,12 +2,11 @@
 // test program (misc/ocean-sim/tridiag-test.fut:14-26), [n][m] f32 systems,
 // one system per row.
 //
-//   tridag_seq_kernel  tridagSeq (misc/ocean-sim/tridiag.fut:81-95): Thomas.
-//   tridag_par_kernel  tridagPar (tridiag.fut:4-79): the three recurrences
-//                      in the form of the reference's scans, evaluated left to
-//                      right.
+//   seq_system  tridagSeq (misc/ocean-sim/tridiag.fut:81-95): Thomas.
+//   par_system  tridagPar (tridiag.fut:4-79): the three recurrences in the form
+//               of the reference's scans, evaluated left to right.
 //   tridag_seq_aligned_kernel, tridag_par_staged_kernel: the same two for
-//                      systems of up to 128 unknowns, staged through LDS.
+//               systems of up to 128 unknowns, staged through LDS.
 //
 // One thread per system, in the reference's order of operations with IEEE
 // division and no contraction (the file is built with -ffp-contract=off), so
@@ -15,8 +14,8 @@
 // not diagonally dominant, and a reordered (partitioned or cyclic-reduction)
 // solve would meet pivots the reference's never does.  Systems of up to 128
 // unknowns go through the staged kernels below, which keep the forward
-// pass's per-row values in registers.  For longer ones the two kernels above
-// keep them in LDS (c' or the modified diagonal, one column per lane) when
+// pass's per-row values in registers.  For longer ones tridag_system_kernel
+// keeps them in LDS (c' or the modified diagonal, one column per lane) when
 // m <= kLdsRows, otherwise in a global scratch array; y' goes to the output
 // array in place.
 
@@ -36,19 +35,10 @@ struct RowStore {
   __device__ float &operator[](int i) const { return p[i * stride]; }
 };
 
-// tridiag.fut:81-95
-template <bool LDS>
-__global__ __launch_bounds__(kThreads) void tridag_seq_kernel(
-    const float *__restrict__ a, const float *__restrict__ b,
-    const float *__restrict__ c, const float *__restrict__ y,
-    float *__restrict__ out, float *__restrict__ scratch, int64_t n, int m) {
-  extern __shared__ float lds[];  // m * kThreads floats when LDS
-  const int64_t sys = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (sys >= n) return;
-  const int64_t off = sys * m;
-  const float *A = a + off, *B = b + off, *C = c + off, *Yv = y + off;
-  float *X = out + off;
-  const RowStore cp = LDS ? RowStore{lds + threadIdx.x, kThreads} : RowStore{scratch + off, 1};
+// tridiag.fut:81-95, one system
+__device__ __forceinline__ void seq_system(const float *__restrict__ A, const float *__restrict__ B,
+                                           const float *__restrict__ C, const float *__restrict__ Yv,
+                                           float *__restrict__ X, const RowStore cp, int m) {
   float cprev = C[0] / B[0];
   float yprev = Yv[0] / B[0];
   cp[0] = cprev;
@@ -68,21 +58,12 @@ __global__ __launch_bounds__(kThreads) void tridag_seq_kernel(
   }
 }
 
-// tridiag.fut:4-79: recurrence 1 as the scan of normalised 2x2 matrices,
-// recurrences 2 and 3 as scans of linear-function composition, in the
+// tridiag.fut:4-79, one system: recurrence 1 as the scan of normalised 2x2
+// matrices, recurrences 2 and 3 as scans of linear-function composition, in the
 // operator forms of the reference, accumulated left to right.
-template <bool LDS>
-__global__ __launch_bounds__(kThreads) void tridag_par_kernel(
-    const float *__restrict__ a, const float *__restrict__ b,
-    const float *__restrict__ c, const float *__restrict__ y,
-    float *__restrict__ out, float *__restrict__ scratch, int64_t n, int m) {
-  extern __shared__ float lds[];  // m * kThreads floats when LDS
-  const int64_t sys = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (sys >= n) return;
-  const int64_t off = sys * m;
-  const float *A = a + off, *B = b + off, *C = c + off, *Yv = y + off;
-  float *X = out + off;
-  const RowStore bb = LDS ? RowStore{lds + threadIdx.x, kThreads} : RowStore{scratch + off, 1};
+__device__ __forceinline__ void par_system(const float *__restrict__ A, const float *__restrict__ B,
+                                           const float *__restrict__ C, const float *__restrict__ Yv,
+                                           float *__restrict__ X, const RowStore bb, int m) {
   // Recurrence 1 (:8-31): b'_i = (t0*b0 + t1) / (t2*b0 + t3) from the scan
   // of (b_i, -a_i*c_{i-1}, 1, 0) under the normalised product.
   const float b0 = B[0];
@@ -130,6 +111,22 @@ __global__ __launch_bounds__(kThreads) void tridag_par_kernel(
   }
 }
 
+template <bool LDS, bool SEQ>
+__global__ __launch_bounds__(kThreads) void tridag_system_kernel(
+    const float *__restrict__ a, const float *__restrict__ b,
+    const float *__restrict__ c, const float *__restrict__ y,
+    float *__restrict__ out, float *__restrict__ scratch, int64_t n, int m) {
+  extern __shared__ float lds[];  // m * kThreads floats when LDS
+  const int64_t sys = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (sys >= n) return;
+  const int64_t off = sys * m;
+  const RowStore rows = LDS ? RowStore{lds + threadIdx.x, kThreads} : RowStore{scratch + off, 1};
+  if constexpr (SEQ)
+    seq_system(a + off, b + off, c + off, y + off, out + off, rows, m);
+  else
+    par_system(a + off, b + off, c + off, y + off, out + off, rows, m);
+}
+
 // Staged kernels for systems of up to kStagedRows unknowns: one wavefront
 // per 64 systems.  Chunks of CH columns of a, b, c, y are loaded into LDS
 // with coalesced row reads (each system's row is contiguous: CH * 4 bytes of
@@ -146,10 +143,10 @@ __global__ __launch_bounds__(kThreads) void tridag_par_kernel(
 // interleaving them changes no result).
 //
 // The scan form (tridag_par_staged_kernel) takes chunks of 16 columns
-// aligned to the systems' columns: with its more numerous carries and five
-// divisions a row it is bound by its division chain rather than its reads,
-// and 16 measured best (32, or 32-column chunks aligned to the arrays'
-// lines as Thomas takes them, were slower).
+// aligned to the systems' columns: with its more numerous carries it is
+// bound by its chains rather than its reads, and 16 measured best (32 is 1 us
+// faster at 115 and 128 unknowns and up to 7 slower below; 8, and chunks
+// aligned to the arrays' lines as Thomas takes them, are slower throughout).
 // Thomas (tridag_seq_aligned_kernel, below) takes 32-column chunks aligned
 // to the arrays' 128-byte lines instead.
 constexpr int kStagedRows = 128;
@@ -168,12 +165,15 @@ struct Stage {
   static constexpr int kLanesPerRow = CH / kVec;
   static constexpr int kRowStep = kThreads / kLanesPerRow;
   static constexpr int kQ = kThreads / kRowStep;
-  float v[4][kThreads][CH + 1];  // a, b, c, y; the solution through v[3]
+  union {
+    float v[4][kThreads][CH + 1];  // a, b, c, y; the solution through v[3]
+    float rows[kStagedRows * kThreads];  // a forward pass from memory
+  };
 };
 
 // The same rows and columns loaded into registers (this lane's slots), to be
 // written to LDS later: the next chunk's loads fly while this one computes.
-// Slots outside the systems (rows >= rows, columns >= m) hold 0.  A chunk
+// Slots outside the systems (rows >= rows, columns >= m) hold an identity row.  A chunk
 // wholly inside them (every chunk of a full workgroup but a ragged last one)
 // takes unguarded 16-byte loads; the test is made once for the four arrays,
 // so that their loads issue back to back.
@@ -210,7 +210,8 @@ __device__ __forceinline__ void fetch(Chunk<CH> &pa, Chunk<CH> &pb, Chunk<CH> &p
         const int r = q * St::kRowStep + sr;
 #pragma unroll
         for (int e = 0; e < kVec; ++e)
-          dst[k][q][e] = (r < rows && i + e < m) ? src[k][(s0 + r) * m + i + e] : 0.0f;
+          dst[k][q][e] = (r < rows && i + e < m) ? src[k][(s0 + r) * m + i + e]
+                                                 : k == 1 ? 1.0f : 0.0f;
       }
   }
 }
@@ -259,6 +260,51 @@ __device__ __forceinline__ void stage_out(const float (&st)[kThreads][CH + 1],
   }
 }
 
+// Divisions.  One wavefront per SIMD issues an instruction every four or five
+// cycles and waits for each of a chain, so the eleven dependent instructions
+// of an IEEE division are what the staged kernels spend their time on.  Where
+// nothing over- or underflows they are not needed: v_rcp_f32 and one Newton step
+// give the correctly rounded 1 / d (checked for every significand), and with it
+// n * r and one residual step the correctly rounded n / d (Markstein, "Computation
+// of elementary functions on the IBM RISC System/6000 processor", 1990), three
+// instructions for each further quotient by the same d.  The forward pass runs
+// on them and keeps the largest and smallest magnitudes that it met; if any
+// lane's left the range, the wave's systems are solved from memory with the
+// division operator instead, zeros, denormals and infinities included.  (A NaN
+// passes through both.)  That costs four times the call's time, so the
+// right-hand sides, which a caller scales as he likes, are divided by the operator
+// throughout and only the matrix can leave the range.  57600 systems: Thomas 38.7 -> 37.1 us at 115 unknowns,
+// the scan form, which has five divisions a row and three of them by the same
+// number, 57.1 -> 55.3 (and 49.4 -> 44.1 at 128).
+constexpr float kDivLow = 0x1p-40f, kDivHigh = 0x1p40f;
+// taps 0 or above 2^-80, as (bits << 1) - 1, where 0 is the largest
+constexpr uint32_t kNumLow = (uint32_t)(127 - 80) << 24;
+
+__device__ __forceinline__ float recip(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float quotient(float n, float d, float r) {
+  const float q = n * r;
+  return fmaf(fmaf(-d, q, n), r, q);
+}
+struct Range {
+  float high = 1.0f, low = 1.0f;
+  uint32_t num = 0xffffffffu;
+  // magnitudes that must be in range, without the compiler's quieting
+  __device__ __forceinline__ void divisors(float x, float y) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(high) : "v"(x), "v"(y));
+    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(low) : "v"(x), "v"(y));
+  }
+  __device__ __forceinline__ void numerators(float x, float y) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(high) : "v"(x), "v"(y));
+    num = min(num, min((__float_as_uint(x) << 1) - 1u, (__float_as_uint(y) << 1) - 1u));
+  }
+  __device__ __forceinline__ bool left() const {
+    return !(high <= kDivHigh && low >= kDivLow && num >= kNumLow);
+  }
+};
+
 template <int CH>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void tridag_par_staged_kernel(const float *__restrict__ a, const float *__restrict__ b,
@@ -275,10 +321,12 @@ void tridag_par_staged_kernel(const float *__restrict__ a, const float *__restri
   float t0 = 1.0f, t1 = 0.0f, t2 = 0.0f, t3 = 1.0f, b0 = 0.0f, bprev = 0.0f;
   float f0 = 0.0f, f1 = 1.0f, y0 = 0.0f;
   float yn = 0.0f;  // l0 of row m-1, recurrence 3's start
+  float rprev = 0.0f;  // 1 / bprev
+  Range range;
 
   // The row loops have no per-row branch, so that the scheduler can overlap
   // one row's LDS reads with the previous row's arithmetic: rows m..(the end
-  // of the last chunk) run on the zeros that fetch() leaves there, and what
+  // of the last chunk) run on the identity rows that fetch() leaves there, and what
   // they produce is never stored nor carried into rows below m (the forward
   // pass ends with them; the backward pass restarts at row m-1 by select).
   Chunk<CH> pa, pb, pc, py;  // the next chunk, in flight
@@ -305,7 +353,8 @@ void tridag_par_staged_kernel(const float *__restrict__ a, const float *__restri
         b0 = bi;
       } else {
         const float m0 = bi, m1 = 0.0f - ai * cprev, m2 = 1.0f, m3 = 0.0f;
-        const float value = 1.0f / (t0 * m0);
+        const float scale = t0 * m0;
+        const float value = recip(scale);
         const float n0 = (m0 * t0 + m1 * t2) * value;
         const float n1 = (m0 * t1 + m1 * t3) * value;
         const float n2 = (m2 * t0 + m3 * t2) * value;
@@ -314,28 +363,42 @@ void tridag_par_staged_kernel(const float *__restrict__ a, const float *__restri
         t1 = n1;
         t2 = n2;
         t3 = n3;
+        range.divisors(scale, scale);
       }
-      const float bb = (t0 * b0 + t1) / (t2 * b0 + t3);
+      const float num = t0 * b0 + t1, den = t2 * b0 + t3;
+      const float bb = quotient(num, den, recip(den)), rbb = recip(bb);
+      range.divisors(den, bb);  // and with them num
       // recurrence 2
       float yy;
       if (i == 0) {
         y0 = yi;
         yy = f0 + f1 * y0;
       } else {
-        const float l0 = yi, l1 = 0.0f - ai / bprev;
+        const float l0 = yi, l1 = 0.0f - quotient(ai, bprev, rprev);
         const float g0 = l0 + l1 * f0, g1 = f1 * l1;
         f0 = g0;
         f1 = g1;
         yy = f0 + f1 * y0;
       }
       // this row's element of recurrence 3
-      fw0[i] = yy / bb;
-      fw1[i] = 0.0f - ci / bb;
+      fw0[i] = yy / bb;  // a right-hand side may be of any size
+      fw1[i] = 0.0f - quotient(ci, bb, rbb);
+      range.numerators(ai, ci);
       bprev = bb;
+      rprev = rbb;
       cprev = ci;
       yn = i < m ? fw0[i] : yn;  // ends as y'_{m-1}/b'_{m-1}
     }
     __syncthreads();  // every lane has read the chunk before the next deposit
+  }
+
+  if (__any(range.left())) {
+    if (lane < rows) {
+      const int64_t off = (s0 + lane) * m;
+      par_system(a + off, b + off, c + off, y + off, out + off, RowStore{S.rows + lane, kThreads},
+                 m);
+    }
+    return;
   }
 
   // backward pass (recurrence 3) over the chunks in reverse, from registers
@@ -414,6 +477,7 @@ void tridag_seq_aligned_kernel(const float *__restrict__ a, const float *__restr
 
   float fw0[kSlots], fw1[kSlots];  // y' and c' by slot
   float cprev = 0.0f, yprev = 0.0f;
+  Range range;
 
   const float *__restrict__ src[4] = {a + s0 * m, b + s0 * m, c + s0 * m, y + s0 * m};
   float *__restrict__ dst = out + s0 * m;
@@ -435,7 +499,7 @@ void tridag_seq_aligned_kernel(const float *__restrict__ a, const float *__restr
         }
       }
     } else {
-      // the last workgroup: rows past n hold zeros; units stop at the end of
+      // the last workgroup: rows past n hold identity rows; units stop at the end of
       // the arrays (floats from src to there: tail), elementwise only in the
       // one 16-byte piece that crosses it
 #pragma unroll
@@ -444,7 +508,8 @@ void tridag_seq_aligned_kernel(const float *__restrict__ a, const float *__restr
         const int u = row_start(q) - row_shift(q) + k * CH + sc;
 #pragma unroll
         for (int arr = 0; arr < 4; ++arr) {
-          float4u v = {0.0f, 0.0f, 0.0f, 0.0f};
+          const float fill = arr == 1 ? 1.0f : 0.0f;
+          float4u v = {fill, fill, fill, fill};
           if (r < rows && u + kVec <= tail) {
             v = *(const float4u *)(src[arr] + u);
           } else if (r < rows) {
@@ -485,7 +550,9 @@ void tridag_seq_aligned_kernel(const float *__restrict__ a, const float *__restr
       const float ci = S.v[2][lane][j], yi = S.v[3][lane][j];
       // column 0 falls in chunk 0 (sh < CH); before it the carries hold
       // whatever the slots before produced, and they restart there (:82-88)
-      const float norm = 1.0f / (bi - ai * cprev);
+      const float pivot = bi - ai * cprev;
+      const float norm = recip(pivot);
+      range.divisors(pivot, pivot);
       float cn = ci * norm, yv = (yi - ai * yprev) * norm;
       if (k == 0) {
         const bool first = j == sh;
@@ -498,6 +565,15 @@ void tridag_seq_aligned_kernel(const float *__restrict__ a, const float *__restr
       fw0[s] = yprev;
     }
     __syncthreads();  // every lane has read the chunk before the next deposit
+  }
+
+  if (__any(range.left())) {
+    if (lane < rows) {
+      const int64_t off = (s0 + lane) * m;
+      seq_system(a + off, b + off, c + off, y + off, out + off, RowStore{S.rows + lane, kThreads},
+                 m);
+    }
+    return;
   }
 
   // backward pass over the chunks in reverse, from registers.  Slot s's
@@ -583,14 +659,14 @@ int lvc_launch_tridag(void *stream, int form, const float *a, const float *b,
   const size_t shm = lds ? (size_t)m * kThreads * sizeof(float) : 0;
   if (form == 1) {
     if (lds)
-      tridag_seq_kernel<true><<<(unsigned)blocks, kThreads, shm, st>>>(a, b, c, y, out, scratch, n, m);
+      tridag_system_kernel<true, true><<<(unsigned)blocks, kThreads, shm, st>>>(a, b, c, y, out, scratch, n, m);
     else
-      tridag_seq_kernel<false><<<(unsigned)blocks, kThreads, 0, st>>>(a, b, c, y, out, scratch, n, m);
+      tridag_system_kernel<false, true><<<(unsigned)blocks, kThreads, 0, st>>>(a, b, c, y, out, scratch, n, m);
   } else if (form == 0) {
     if (lds)
-      tridag_par_kernel<true><<<(unsigned)blocks, kThreads, shm, st>>>(a, b, c, y, out, scratch, n, m);
+      tridag_system_kernel<true, false><<<(unsigned)blocks, kThreads, shm, st>>>(a, b, c, y, out, scratch, n, m);
     else
-      tridag_par_kernel<false><<<(unsigned)blocks, kThreads, 0, st>>>(a, b, c, y, out, scratch, n, m);
+      tridag_system_kernel<false, false><<<(unsigned)blocks, kThreads, 0, st>>>(a, b, c, y, out, scratch, n, m);
   } else {
     return (int)hipErrorInvalidValue;
   }
