@@ -759,10 +759,20 @@ __device__ __forceinline__ void loglik_sums(const StepArgs &A, const int32_t (&i
     for (int b = 1; b < kSumLanes; b <<= 1) s[m] += __shfl_xor(s[m], b, 64);
 }
 
-// Whether genome i's proposal, of log-likelihood s, is accepted (:733-745).
-__device__ __forceinline__ bool accepted(const StepArgs &A, int32_t i, float s) {
-  const float acceptance = fminf(1.0f, expf(s - A.from.logliks[i]) * A.from.fb[i]);
-  return sobol(A.dv, A.acc + i) < acceptance;
+// What the step reads of a genome, gene j: all of it asked for beside the terms,
+// not after the sums and again after the decision (three memory round trips
+// of a launch that is little else: 8.9 us, and 8.2 with one).
+struct Member {
+  float loglik, fb, gene, prop;
+};
+__device__ __forceinline__ Member read_member(const StepArgs &A, int32_t i, int j) {
+  return {A.from.logliks[i], A.from.fb[i], A.from.genomes[5 * i + j], A.from.props[5 * i + j]};
+}
+
+// Whether the genome's proposal, of log-likelihood s, is accepted on its draw
+// (:733-745).
+__device__ __forceinline__ bool accepted(const Member &g, float s, float draw) {
+  return draw < fminf(1.0f, expf(s - g.loglik) * g.fb);
 }
 
 // One step of the population: each genome's log-likelihood and acceptance,
@@ -782,52 +792,56 @@ __global__ __launch_bounds__(256) void ic_step_kernel(StepArgs A) {
   int32_t k = i, l = i;
   float gamma1 = 0.0f;
   const int32_t kk = 8 * i + mv.base;
+  // The genome's Sobol numbers, a lane each (one after the other they were seven
+  // chains of 31 bits in DE's step, 8.2 us, and 6.4 with two): the genes' in
+  // lanes 0 .. 4, the accept step's, then DE's three.
+  const int first = threadIdx.x & 63 & ~(kSumLanes - 1);
+  const float draws =
+      sobol(A.dv, t < 5 ? (de ? kk + 3 : 5 * i + mv.base) + t : t == 5 ? A.acc + i : kk + t - 6);
+  const float draw = __shfl(draws, first + 5), s1 = __shfl(draws, first + 6);
+  const float s2 = __shfl(draws, first + 7), s3 = __shfl(draws, first + 8);
   if (de) {
-    const float s1 = sobol(A.dv, kk);
     k = (int32_t)(s1 * (float)(pop - 1));
     int32_t cand_ub = pop - 1;
     if (k == i) {
       k = pop - 1;
       cand_ub = pop - 2;
     }
-    const float s2 = sobol(A.dv, kk + 1);
     l = (int32_t)(s2 * (float)cand_ub);
     if (l == i || l == k) l = cand_ub;
-    const float s3 = sobol(A.dv, kk + 2);
     const float gamma_avg = 2.38f / sqrtf(2.0f * 5.0f);
     gamma1 = gamma_avg - 0.5f + s3;
   }
-  float s;
-  bool take = false, take_k = false, take_l = false;
+  const int j = t < 5 ? t : 0;  // this lane's gene
+  const Member own = read_member(A, i, j);
+  float s, gene_k = 0.0f, gene_l = 0.0f;
+  bool take = false;
   if (de) {
+    const Member gk = read_member(A, k, j), gl = read_member(A, l, j);
+    const float theirs = sobol(A.dv, A.acc + (t & 1 ? l : k));
+    const float draw_k = __shfl(theirs, first), draw_l = __shfl(theirs, first + 1);
     const int32_t ids[3] = {i, k, l};
     float sums[3];
     loglik_sums<3>(A, ids, t, sums);
     s = sums[0];
-    if (!A.init) {
-      take = accepted(A, i, s);
-      take_k = accepted(A, k, sums[1]);
-      take_l = accepted(A, l, sums[2]);
-    }
+    take = !A.init && accepted(own, s, draw);
+    gene_k = !A.init && accepted(gk, sums[1], draw_k) ? gk.prop : gk.gene;
+    gene_l = !A.init && accepted(gl, sums[2], draw_l) ? gl.prop : gl.gene;
   } else {
     const int32_t ids[1] = {i};
     float sums[1];
     loglik_sums<1>(A, ids, t, sums);
     s = sums[0];
-    if (!A.init) take = accepted(A, i, s);
+    take = !A.init && accepted(own, s, draw);
   }
-  const int j = t < 5 ? t : 0;  // this lane's gene
-  auto gene_of = [&](int32_t g, bool taken) {
-    return taken ? A.from.props[5 * g + j] : A.from.genomes[5 * g + j];
-  };
-  const float gene = gene_of(i, take);
-  const float loglik = A.init || take ? s : A.from.logliks[i];
+  const float gene = take ? own.prop : own.gene;
+  const float loglik = A.init || take ? s : own.loglik;
   float out = 0.0f, bf = 1.0f;
   if (mv.type == 1 || mv.type == 2) {  // mutate_dims_all / mutate_dims_one (:278-306)
-    const float r01 = sobol(A.dv, 5 * i + mv.base + j);
+    const float r01 = draws;
     const float ampl = mv.type == 1 || j == mv.dim ? kAmplRatio : 0.0f;
     const float g_min = gene_min(j), g_max = gene_max(j);
-    const float prop = A.from.props[5 * i + j];
+    const float prop = own.prop;
     const float amplitude = fabsf((g_max - g_min) * ampl);  // mutateHelper, :250-266
     const float semiamplitude = amplitude / 2.0f;
     float tmp_min_max = fminf(g_max, gene + semiamplitude);
@@ -841,16 +855,15 @@ __global__ __launch_bounds__(256) void ic_step_kernel(StepArgs A) {
     out = fmaxf(g_min, fminf(g_max, ng));  // constrainDim, :268-270
   } else if (de) {  // :713-723, mcmc_DE :309-320
     const float ampl_ratio = 0.1f * kAmplRatio;
-    const float r01 = sobol(A.dv, kk + 3 + j);
+    const float r01 = draws;
     const float mm_diff = gene_max(j) - gene_min(j);
     const float amplitude = fabsf(mm_diff * ampl_ratio);
     const float semiamplitude = amplitude / 2.0f;
     const float perturb = amplitude * r01 - semiamplitude;
-    const float ng = gene + perturb + gamma1 * (gene_of(k, take_k) - gene_of(l, take_l));
+    const float ng = gene + perturb + gamma1 * (gene_k - gene_l);
     out = fmaxf(gene_min(j), fminf(gene_max(j), ng));
   }
   // the genes' ratios multiplied in order
-  const int first = threadIdx.x & 63 & ~(kSumLanes - 1);
   float fb = __shfl(bf, first);
   for (int m = 1; m < 5; m++) fb = fb * __shfl(bf, first + m);
   if (at >= pop) return;
