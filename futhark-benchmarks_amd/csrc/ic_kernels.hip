@@ -883,17 +883,43 @@ __global__ __launch_bounds__(256) void ic_step_kernel(StepArgs A) {
   }
 }
 
-__global__ void ic_winner_kernel(int32_t pop, const float *__restrict__ genomes,
-                                 const float *__restrict__ logliks, float *__restrict__ out,
-                                 float *__restrict__ winner) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int32_t wi = 0;  // :752-756, the reduction read as a left fold
+// The winner (:752-756): the reduction read as a left fold, so the first of the
+// largest log-likelihoods (a NaN is never one, and genome 0 wins where nothing
+// is above -inf).  One workgroup: a lane folds its genomes in order, the lanes
+// are joined by value, then by the smaller index.  (One thread over them all
+// was 17.6 us at 256 genomes, 4.6 now.)
+constexpr int kWinnerThreads = 256;
+__global__ __launch_bounds__(kWinnerThreads) void ic_winner_kernel(
+    int32_t pop, const float *__restrict__ genomes, const float *__restrict__ logliks,
+    float *__restrict__ out, float *__restrict__ winner) {
+  __shared__ float values[kWinnerThreads / 64];
+  __shared__ int32_t indexes[kWinnerThreads / 64];
+  const int t = threadIdx.x;
+  int32_t wi = 0;
   float wv = -INFINITY;
-  for (int32_t i = 0; i < pop; i++)
-    if (wv < logliks[i]) {
+  for (int32_t i = t; i < pop; i += kWinnerThreads) {
+    const float v = logliks[i];
+    if (wv < v) {
       wi = i;
-      wv = logliks[i];
+      wv = v;
     }
+  }
+  auto join = [&](float v, int32_t i) {
+    if (wv < v || (wv == v && i < wi)) {
+      wi = i;
+      wv = v;
+    }
+  };
+#pragma unroll
+  for (int b = 1; b < 64; b <<= 1) join(__shfl_xor(wv, b), __shfl_xor(wi, b));
+  if ((t & 63) == 0) {
+    values[t >> 6] = wv;
+    indexes[t >> 6] = wi;
+  }
+  __syncthreads();
+  if (t != 0) return;
+#pragma unroll
+  for (int k = 1; k < kWinnerThreads / 64; k++) join(values[k], indexes[k]);
   const float *w = genomes + 5 * wi;
   out[0] = w[0];
   out[1] = w[1];
@@ -980,7 +1006,7 @@ extern "C" int ic_launch_step(void *stream, int32_t pop, int32_t nswap, const fl
 
 extern "C" int ic_launch_winner(void *stream, int32_t pop, const float *genomes,
                                 const float *logliks, float *out, float *winner) {
-  hipLaunchKernelGGL(ic_winner_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, pop, genomes,
+  hipLaunchKernelGGL(ic_winner_kernel, dim3(1), dim3(kWinnerThreads), 0, (hipStream_t)stream, pop, genomes,
                      logliks, out, winner);
   return (int)hipGetLastError();
 }
