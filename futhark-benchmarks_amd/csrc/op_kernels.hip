@@ -803,7 +803,9 @@ __global__ __launch_bounds__(kThreads) void op_many_kernel(
 }
 
 // Contract 3's tables, one launch: workgroup 0 makes the bridge's schedule,
-// the others the parts of the Sobol numbers.
+// the others the parts of the Sobol numbers and the models' dates.  It is the
+// schedule's chain of LDS and barriers, 8.9 us; the dates made at its end, and a
+// second search for the step before, were 1.2 us of it.
 //
 // The schedule: with the path kernel's clamped indexes step i (of D) writes
 // date l_i and, for i >= 1, reads dates k_i and (when li != 0) j_i.  Every date
@@ -835,7 +837,7 @@ __global__ __launch_bounds__(kTabThreads) void op_tables_kernel(
       for (int u = 0; u < 3; ++u) {
         int32_t x = 0;
         if (at < 63) {
-          #pragma unroll
+#pragma unroll
           for (int b = 0; b < 6; ++b) x ^= vec(t, u, b, g >> b & 1u);
         } else {
           x = vec(t, u, 5, true) ^ vec(t, u, 6 + at - 63, true);
@@ -850,6 +852,11 @@ __global__ __launch_bounds__(kTabThreads) void op_tables_kernel(
         for (int b = 0; b < 4; ++b) x ^= vec(t, u, 5 + row / 16 * 4 + b, row >> b & 1);
         tab->hi[row / 16][row % 16][t][u] = x;
       }
+    } else {
+      // the models' dates, and two zero ones that the path kernel reads past them
+      const int e = i - D * (kLo + 16 * groups), m = e / (D + 2), d = e % (D + 2);
+      const Market mk = {cs, vols, drifts, nullptr, nullptr, nullptr, 0};
+      if (m < M) tab->date[m][d] = d < D ? make_date<3>(mk, m, d) : Date{};
     }
     return;
   }
@@ -875,8 +882,6 @@ __global__ __launch_bounds__(kTabThreads) void op_tables_kernel(
     count[i] = 0;
     depth[0][i] = 0;
   }
-  if (i == D || i == D + 1)
-    for (int m = 0; m < M; ++m) tab->date[m][i] = Date{};
   for (int e = tid; e < kSlots * kWords; e += kTabThreads) (&uses[0][0])[e] = 0u;
   if (tid == 0) bad = 0;
   __syncthreads();
@@ -917,7 +922,11 @@ __global__ __launch_bounds__(kTabThreads) void op_tables_kernel(
   }
   if ((tid & 63) == 63) most[tid >> 6] = done;
   __syncthreads();
-  for (int w = 0; w < tid >> 6; ++w) done = max(done, most[w]);
+#pragma unroll
+  for (int w = 0; w < kTabThreads / 64; ++w) {
+    const int v = most[w];  // read whether it counts or not: the reads are independent
+    done = w < tid >> 6 ? max(done, v) : done;
+  }
   ready[tid] = done;
   if (bad) {
     if (tid == 0) tab->fits = 0;
@@ -933,22 +942,22 @@ __global__ __launch_bounds__(kTabThreads) void op_tables_kernel(
     while (left == 0u && ++word < kWords) left = m[word];
     return left ? word * 32 + __builtin_ctz(left) : D;
   };
+  // the dates complete after step i: ready is ascending
+  int upto = 0;
+  for (int hi = D; upto < hi;) {
+    const int mid = (upto + hi) >> 1;
+    if (ready[mid] <= i)
+      upto = mid + 1;
+    else
+      hi = mid;
+  }
+  if (on) count[i] = upto;
+  __syncthreads();
   if (on) {
     ok = next(first[i]) > done;
     if (i > 0) ok = ok && next(fk) >= i && (j == -1 || next(fj) >= i);
     if (!ok) bad = 1;
-    auto complete = [&](int step) {  // the dates after it: ready is ascending
-      int lo = 0, hi = D;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (ready[mid] <= step)
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
-      return lo;
-    };
-    const int upto = complete(i), from = complete(i - 1);
+    const int from = i > 0 ? count[i - 1] : 0;
     auto offset = [](int slot) { return (uint32_t)(slot * 64 * (int)sizeof(float4)); };
     auto slot_of = [&](int d) { return offset(d < D ? dep[first[d]] : kSlots); };
     // the half of a record that streams comes from the thread of the step before
@@ -967,10 +976,6 @@ __global__ __launch_bounds__(kTabThreads) void op_tables_kernel(
       st->stream = 0u;
     }
     tab->slot[i] = slot_of(i);
-    const Market mk = {cs, vols, drifts, nullptr, nullptr, nullptr, 0};
-    for (int m = 0; m < M; ++m) {
-      tab->date[m][i] = make_date<3>(mk, m, i);
-    }
   }
   __syncthreads();
   if (tid == 0) tab->fits = !bad;
@@ -1032,7 +1037,7 @@ int op_launch(void *stream, int contract, const op_args *A, const int32_t *dir_v
       // the groups of bits that a wave's base has
       int groups = 0;
       while (groups < kHi && (((uint32_t)A->N + 63u) >> 5) >> (4 * groups) != 0u) ++groups;
-      const int entries = kD3 * (kLo + 16 * groups);
+      const int entries = kD3 * (kLo + 16 * groups) + mc * (kD3 + 2);
       op_tables_kernel<<<1 + (entries + kTabThreads - 1) / kTabThreads, kTabThreads, 0, st>>>(
           dir_vs, A->bbi, A->bbd, A->cs + (int64_t)m0 * U * U, A->vols + (int64_t)m0 * D * U,
           A->drifts + (int64_t)m0 * D * U, A->bits, groups, mc, tab);
