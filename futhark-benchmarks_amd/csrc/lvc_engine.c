@@ -327,10 +327,12 @@ void lvc_batch_release(struct futhark_context *ctx, lvc_batch *b) {
   memset(b, 0, sizeof(*b));
 }
 
-/* One time step of every batch in bs that still runs: the x sweeps, then
- * the y sweeps (each batch is a set of problems sharing one segment pair). */
-static int launch_step(struct futhark_context *ctx, lvc_batch *bs, int nb, int64_t s) {
-  void *st = (void *)ctx->stream;
+/* One time step of every batch in bs that still runs, on `stream`: the x
+ * sweeps, then the y sweeps (each batch is a set of problems sharing one
+ * segment pair). */
+static int launch_step(struct futhark_context *ctx, hipStream_t stream, lvc_batch *bs,
+                       int nb, int64_t s) {
+  void *st = (void *)stream;
   for (int g = 0; g < nb; g++) {
     lvc_batch *b = &bs[g];
     if (s >= b->steps)
@@ -401,7 +403,7 @@ static int run_graph(struct futhark_context *ctx, lvc_batch *bs, int nb, int64_t
       return 1;
     int rc = 0;
     for (int64_t s = 0; !rc && s < steps; s++)
-      rc = launch_step(ctx, bs, nb, s);
+      rc = launch_step(ctx, ctx->stream, bs, nb, s);
     const int e = (int)hipStreamEndCapture(ctx->stream, &graph);
     if (rc || lvc_check_hip(ctx, e, "hipStreamEndCapture")) {
       if (graph)
@@ -436,9 +438,15 @@ static int run_graph(struct futhark_context *ctx, lvc_batch *bs, int nb, int64_t
                        "hipGraphLaunch");
 }
 
+static int profiling_on(const struct futhark_context *ctx) {
+  return ctx->cfg && ctx->cfg->profiling && !ctx->prof_paused;
+}
+
 /* Runs the batches in bs together: their setups, then the time steps, each
- * step every batch's x sweep then every batch's y sweep. */
-static int run_batches(struct futhark_context *ctx, lvc_batch *bs, int nb) {
+ * step every batch's x sweep then every batch's y sweep.  The batches from
+ * `split` on (none: split = nb) are independent of the others and step on the
+ * context's second stream. */
+static int run_batches(struct futhark_context *ctx, lvc_batch *bs, int nb, int split) {
   int64_t steps = 0;
   for (int g = 0; g < nb; g++) {
     lvc_batch *b = &bs[g];
@@ -453,17 +461,21 @@ static int run_batches(struct futhark_context *ctx, lvc_batch *bs, int nb) {
     if (b->steps > steps)
       steps = b->steps;
   }
-  const int profiling = ctx->cfg && ctx->cfg->profiling && !ctx->prof_paused;
-  if (nb > 0 && bs[0].graph && !profiling && steps > 0)
+  if (nb > 0 && bs[0].graph && !profiling_on(ctx) && steps > 0)
     return run_graph(ctx, bs, nb, steps);
-  for (int64_t s = 0; s < steps; s++)
-    if (launch_step(ctx, bs, nb, s))
-      return 1;
-  return 0;
+  if (split < nb && lvc_fork(ctx))
+    return 1;
+  int rc = 0;
+  for (int64_t s = 0; !rc && s < steps; s++)
+    rc = launch_step(ctx, ctx->stream, bs, split, s) ||
+         launch_step(ctx, ctx->stream2, bs + split, nb - split, s);
+  if (split < nb && lvc_join(ctx))
+    rc = 1;
+  return rc;
 }
 
 int lvc_batch_run(struct futhark_context *ctx, lvc_batch *b) {
-  return run_batches(ctx, b, 1);
+  return run_batches(ctx, b, 1, 1);
 }
 
 int lvc_batch_gather(struct futhark_context *ctx, lvc_batch *b, void *out,
@@ -480,14 +492,65 @@ int lvc_batch_gather(struct futhark_context *ctx, lvc_batch *b, void *out,
 static int download(struct futhark_context *ctx, void *dst, const void *src,
                     size_t bytes);
 
+/* The streams a batch of sweeps steps on.  A step is an x launch and a y
+ * launch that waits for all of it, and each alone leaves half of the vector
+ * ALUs' issue slots idle (2 to 3 waves per SIMD, each in a serial chain, and
+ * the launch's start and end): with the problems in two halves on two
+ * streams one half's x sweep runs beside the other's y sweep.  It costs two
+ * launches more a step, so it needs work enough to hide them: four x tiles
+ * per CU at the first step and three on the mean over the steps (problems
+ * drop out as they end).  Measured, FP32+refinement / FP32, ms on one stream
+ * -> two, by tiles per CU (first step, mean); numT uneven in 32..128:
+ *   512 of 32..256 points (14.2, 9.0)  5.17 -> 4.43 / 4.15 -> 3.54
+ *   256                   (7.0, 4.4)   3.89 -> 3.26 / 3.16 -> 2.68
+ *   192                   (5.0, 3.1)   3.29 -> 3.03 / 2.76 -> 2.55
+ *   1024 of 32..64        (5.0, 3.1)   3.46 -> 2.96 / 2.86 -> 2.47
+ *   16 of 512             (8.0, 5.4)   4.59 -> 4.13 / 3.48 -> 3.25
+ *   128 of 32..256        (3.3, 2.1)   2.86 -> 2.80 / 2.40 -> 2.33
+ *   8 of 512              (4.0, 2.8)   3.42 -> 3.18 / 2.66 -> 2.81
+ *   64 of 32..256         (2.2, 1.3)   2.52 -> 2.62 / 2.11 -> 2.14
+ * and equal numT of 64: 40 of 256 points (5, 5) 2.24 -> 2.05 / 1.93 -> 1.75,
+ * 24 (3, 3) 1.74 -> 1.76 / 1.51 -> 1.53.  Three streams and more are bound by
+ * the host's launches.  One stream also where problems share factorisations
+ * (batch_xshare sizes those workgroups for the whole chip), in FP64 (whose
+ * batches go by the modes), under a captured graph and while kernels are timed
+ * one by one; and past 2^20 tiles, where a launch's ends no longer matter. */
+static int sweep_streams(struct futhark_context *ctx, int n, const lvc_problem *probs,
+                         int precision) {
+  if (precision == LVC_FP64 || (ctx->cfg && ctx->cfg->graph) || profiling_on(ctx))
+    return 1;
+  int64_t tiles = 0, steps = 1;
+  double tile_steps = 0;
+  for (int p = 0; p < n; p++) {
+    const lvc_problem *q = &probs[p];
+    if (p && lvc_same_factor(q - 1, q))
+      return 1;
+    int sx, sy;
+    lvc_choose_segs(ctx, precision, q->nx, q->ny, &sx, &sy);
+    const int rows = LVC_BLOCK / lvc_lanes_for(q->nx, sx);
+    const int64_t t = (q->ny + rows - 1) / rows;
+    tiles += t;
+    tile_steps += (double)t * (q->nt - 1);
+    if (q->nt - 1 > steps)
+      steps = q->nt - 1;
+  }
+  const int64_t cus = ctx->num_cus;
+  return tiles <= 1 << 20 && tiles >= 4 * cus &&
+                 tile_steps >= 3.0 * (double)cus * (double)steps
+             ? 2
+             : 1;
+}
+
 /* Runs problems by the sweeps into out.  Each problem takes its own size
- * class's segment pair; the problems of each distinct pair form a sub-batch,
- * the sub-batches advance together, and each problem's price goes to its own
- * place in the output. */
+ * class's segment pair; the problems of each distinct pair (and stream) form
+ * a sub-batch, the sub-batches advance together, and each problem's price
+ * goes to its own place in the output. */
 #define LVC_MAX_GROUPS 16
 static int run_sweeps(struct futhark_context *ctx, int n, const lvc_problem *probs,
                       int precision, int out_f64, void *out) {
-  int gsx[LVC_MAX_GROUPS], gsy[LVC_MAX_GROUPS], gcnt[LVC_MAX_GROUPS] = {0}, ng = 0;
+  int gsx[LVC_MAX_GROUPS], gsy[LVC_MAX_GROUPS], gcnt[2 * LVC_MAX_GROUPS] = {0}, ng = 0;
+  const int streams = sweep_streams(ctx, n, probs, precision);
+  double load[2] = {0, 0};
   int *grp = malloc((size_t)(n ? n : 1) * sizeof(int));
   lvc_problem *sub = malloc((size_t)(n ? n : 1) * sizeof(lvc_problem));
   if (!grp || !sub) {
@@ -512,24 +575,32 @@ static int run_sweeps(struct futhark_context *ctx, int n, const lvc_problem *pro
       gsy[ng] = sy;
       ng++;
     }
-    grp[p] = g;
-    gcnt[g]++;
+    /* each problem to the stream with the lesser load so far */
+    const int l = streams == 2 && load[1] < load[0];
+    load[l] += (double)(probs[p].nx * probs[p].ny) * (probs[p].nt - 1);
+    grp[p] = l * LVC_MAX_GROUPS + g;
+    gcnt[l * LVC_MAX_GROUPS + g]++;
   }
-  lvc_batch bs[LVC_MAX_GROUPS];
+  lvc_batch bs[2 * LVC_MAX_GROUPS];
   memset(bs, 0, sizeof(bs));
-  int rc = 0;
-  for (int g = 0; !rc && g < ng; g++) {
+  int rc = 0, nb = 0, split = 0;
+  for (int g = 0; !rc && g < 2 * LVC_MAX_GROUPS; g++) {
+    if (g == LVC_MAX_GROUPS)
+      split = nb;
+    if (gcnt[g] == 0)
+      continue;
     int m = 0;
     for (int p = 0; p < n; p++)
       if (grp[p] == g)
         sub[m++] = probs[p];
-    rc = lvc_batch_build(ctx, &bs[g], m, sub, precision, gsx[g], gsy[g]);
+    rc = lvc_batch_build(ctx, &bs[nb++], m, sub, precision, gsx[g % LVC_MAX_GROUPS],
+                         gsy[g % LVC_MAX_GROUPS]);
   }
   if (!rc)
-    rc = run_batches(ctx, bs, ng);
-  for (int g = 0; !rc && g < ng; g++)
+    rc = run_batches(ctx, bs, nb, split);
+  for (int g = 0; !rc && g < nb; g++)
     rc = lvc_batch_gather(ctx, &bs[g], out, out_f64);
-  for (int g = 0; g < ng; g++)
+  for (int g = 0; g < nb; g++)
     lvc_batch_release(ctx, &bs[g]);
   free(grp);
   free(sub);

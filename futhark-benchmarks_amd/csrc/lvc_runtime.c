@@ -161,6 +161,41 @@ struct futhark_context *futhark_context_new(struct futhark_context_config *cfg) 
   return ctx;
 }
 
+int lvc_fork(struct futhark_context *ctx) {
+  if (!ctx->stream2) {
+    /* default priority; kept only when all three exist */
+    hipStream_t st = NULL;
+    hipEvent_t f = NULL, j = NULL;
+    if (lvc_check_hip(ctx, hipStreamCreateWithFlags(&st, hipStreamNonBlocking),
+                      "hipStreamCreate") ||
+        lvc_check_hip(ctx, hipEventCreateWithFlags(&f, hipEventDisableTiming),
+                      "hipEventCreate") ||
+        lvc_check_hip(ctx, hipEventCreateWithFlags(&j, hipEventDisableTiming),
+                      "hipEventCreate")) {
+      if (f)
+        (void)hipEventDestroy(f);
+      if (st)
+        (void)hipStreamDestroy(st);
+      return 1;
+    }
+    ctx->stream2 = st;
+    ctx->forked = f;
+    ctx->joined = j;
+  }
+  return lvc_check_hip(ctx, hipEventRecord(ctx->forked, ctx->stream), "hipEventRecord") ||
+         lvc_check_hip(ctx, hipStreamWaitEvent(ctx->stream2, ctx->forked, 0),
+                       "hipStreamWaitEvent");
+}
+
+int lvc_join(struct futhark_context *ctx) {
+  if (!lvc_check_hip(ctx, hipEventRecord(ctx->joined, ctx->stream2), "hipEventRecord") &&
+      !lvc_check_hip(ctx, hipStreamWaitEvent(ctx->stream, ctx->joined, 0),
+                     "hipStreamWaitEvent"))
+    return 0;
+  (void)hipStreamSynchronize(ctx->stream2);
+  return 1;
+}
+
 void lvc_graph_release(struct futhark_context *ctx) {
   if (ctx->graph_exec)
     (void)hipGraphExecDestroy((hipGraphExec_t)ctx->graph_exec);
@@ -192,6 +227,11 @@ void futhark_context_free(struct futhark_context *ctx) {
     for (int i = 0; i < ctx->nevents; i++)
       (void)hipEventDestroy(ctx->event_pool[i]);
     (void)hipEventDestroy(ctx->stage_done);
+    if (ctx->stream2) {
+      (void)hipEventDestroy(ctx->forked);
+      (void)hipEventDestroy(ctx->joined);
+      (void)hipStreamDestroy(ctx->stream2);
+    }
     (void)hipStreamDestroy(ctx->stream);
   }
   free(ctx->pool);

@@ -55,6 +55,10 @@ struct futhark_context {
   int device;
   int ok; /* device opened */
   hipStream_t stream;
+  /* second stream for independent halves of one call (lvc_fork), made at its
+   * first use, and the events that order it with `stream` */
+  hipStream_t stream2;
+  hipEvent_t forked, joined;
   pthread_mutex_t lock;
   char *error;
   FILE *log;
@@ -111,6 +115,13 @@ extern const lvc_program lvc_prog;
 void lvc_set_error(struct futhark_context *ctx, const char *fmt, ...);
 int lvc_check_hip(struct futhark_context *ctx, int err, const char *what);
 int lvc_ready(struct futhark_context *ctx);
+
+/* lvc_fork lets ctx->stream2 work on what ctx->stream has been given so far;
+ * lvc_join, which every successful lvc_fork is followed by, makes ctx->stream
+ * wait for ctx->stream2, so that freeing, reading and synchronising stay
+ * matters of ctx->stream alone. */
+int lvc_fork(struct futhark_context *ctx);
+int lvc_join(struct futhark_context *ctx);
 
 /* drops the kept graph (its launches name pool memory) */
 void lvc_graph_release(struct futhark_context *ctx);
