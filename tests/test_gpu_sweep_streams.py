@@ -52,3 +52,24 @@ def test_two_streams_keep_the_bits(sizes, n, precision):
         got = ctx.main_batch(**c, precision=precision)
     assert np.array_equal(got[:n], want_a)
     assert got[n] == want_a[n - 2] and got[n + 1] == want_a[n - 2]
+
+
+@pytest.mark.parametrize("precision", [lvc.PRECISION_FP32, lvc.PRECISION_FP32_REFINE])
+def test_equal_problems_apart_in_the_list(precision):
+    """Equal problems with one of another segment class between them: they are
+    neighbours in their class's list, and may come to lie on either stream."""
+    print(f"case: equal problems in turn with others, precision {precision}", flush=True)
+    one = problems((256,), 30, 3)
+    pr = {k: np.repeat(v, 2) for k, v in one.items()}
+    pr["numX"][1::2] = 600
+    pr["numY"][1::2] = 40
+    pr = {k: np.concatenate([np.tile(v[:2], 8), v]) for k, v in pr.items()}
+    pr["strike"] = np.linspace(0.0, 0.04, len(pr["strike"]))
+    with lvc.LocVolCalib(tuning={"lvc.graph": 1}) as ctx:
+        want = ctx.main_batch(**pr, precision=precision)
+    with lvc.LocVolCalib() as ctx:
+        for _ in range(3):
+            assert np.array_equal(ctx.main_batch(**pr, precision=precision), want)
+        for i in (0, 1, 2, 15, len(want) - 1):
+            alone = {k: v[i:i + 1] for k, v in pr.items()}
+            assert ctx.main_batch(**alone, precision=precision)[0] == want[i]
