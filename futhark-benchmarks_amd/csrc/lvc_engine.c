@@ -617,9 +617,10 @@ static void note_index(struct futhark_context *ctx, const lvc_problem *q) {
 }
 
 /* Runs a batch end to end into a new device array of n prices: in FP64 the
- * problems whose x direction separates (lvc_modes_fit) by their modes, the
- * others, and the FP32 forms, whose FP64 prices show the arithmetic that was
- * asked for, by the sweeps.  A problem's way depends on the precision and its
+ * problems whose x direction separates (lvc_modes_fit) and whose price the
+ * modes do not lose (lvc_modes_strike) by their modes, the others, and the FP32
+ * forms, whose FP64 prices show the arithmetic that was asked for, by the
+ * sweeps.  A problem's way depends on the precision and its
  * own sizes and parameters only, so its price has the same bits alone and in
  * any batch. */
 static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *probs,
@@ -638,7 +639,7 @@ static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *prob
     q.out_index = p;
     if (p == 0)
       note_index(ctx, &q);
-    if (precision == LVC_FP64 && lvc_modes_fit(&q)) {
+    if (precision == LVC_FP64 && lvc_modes_fit(&q) && lvc_modes_strike(&q, q.strike, 1)) {
       by[nm++] = q;
       /* "lvc.autotune" asks for every class's sweeps to be timed */
       int sx, sy;
@@ -664,21 +665,20 @@ static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *prob
   return rc;
 }
 
-static void fill_main(lvc_problem *probs, int outer, int nx, int ny, int nt,
-                      double s0, double t, double alpha, double nu, double beta,
-                      int grid32) {
-  memset(probs, 0, (size_t)outer * sizeof(*probs));
-  for (int i = 0; i < outer; i++) {
-    probs[i].nx = nx;
-    probs[i].ny = ny;
-    probs[i].nt = nt;
-    probs[i].s0 = s0;
-    probs[i].t = t;
-    probs[i].alpha = alpha;
-    probs[i].nu = nu;
-    probs[i].beta = beta;
-    probs[i].grid32 = grid32;
-  }
+static lvc_problem main_problem(int nx, int ny, int nt, double s0, double t,
+                                double alpha, double nu, double beta, int f32) {
+  lvc_problem q;
+  memset(&q, 0, sizeof(q));
+  q.nx = nx;
+  q.ny = ny;
+  q.nt = nt;
+  q.s0 = s0;
+  q.t = t;
+  q.alpha = alpha;
+  q.nu = nu;
+  q.beta = beta;
+  lvc_grid_scalars(&q, f32);
+  return q;
 }
 
 /* The price index of main's options (all share initGrid's scalars): the
@@ -706,15 +706,32 @@ static int check_main_index(struct futhark_context *ctx, int outer, int nx, int 
   return 1;
 }
 
+/* main's options first .. first + n - 1 as problems, each with its strike and
+ * its place in main's output. */
+static lvc_problem *main_problems(struct futhark_context *ctx, const lvc_problem *one,
+                                  int first, int n, int f32) {
+  lvc_problem *probs = malloc((size_t)(n ? n : 1) * sizeof(*probs));
+  if (!probs) {
+    lvc_set_error(ctx, "host allocation failed");
+    return NULL;
+  }
+  for (int i = 0; i < n; i++) {
+    probs[i] = *one;
+    probs[i].strike = lvc_main_strike(first + i, f32);
+    probs[i].out_index = first + i;
+  }
+  return probs;
+}
+
 /* main's options into a new device array: one grid with strikes 0.001 * i
  * (:247; f32 = the reference's f32 entry, strikes and initGrid's scalars in
- * f32), by its modes where it separates, else as a batch. */
+ * f32), by its modes where it separates (and the strikes too far for them by
+ * the sweeps, over the modes' prices), else as a batch. */
 static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int nt,
                     double s0, double t, double alpha, double nu, double beta,
                     int f32, int precision, void **mem) {
-  lvc_problem q;
-  fill_main(&q, 1, nx, ny, nt, s0, t, alpha, nu, beta, f32);
-  lvc_grid_scalars(&q, f32);
+  const lvc_problem q = main_problem(nx, ny, nt, s0, t, alpha, nu, beta, f32);
+  lvc_problem *probs;
   int rc = 0;
   *mem = NULL;
   if (outer > 0 && lvc_modes_fit(&q)) {
@@ -726,6 +743,14 @@ static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int 
     rc = lvc_dev_alloc(ctx, ob, mem) || lvc_dev_alloc(ctx, wb, (void **)&work) ||
          lvc_modes_main(ctx, &q, outer, f32, work, *mem, !f32);
     lvc_dev_free(ctx, work, wb);
+    int first = 0, end = 0;
+    if (!rc)
+      lvc_modes_far(&q, outer, f32, &first, &end);
+    if (first < end) {
+      probs = main_problems(ctx, &q, first, end - first, f32);
+      rc = !probs || run_sweeps(ctx, end - first, probs, precision, !f32, *mem);
+      free(probs);
+    }
     if (rc) {
       lvc_dev_free(ctx, *mem, ob);
       *mem = NULL;
@@ -733,14 +758,9 @@ static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int 
     pthread_mutex_unlock(&ctx->lock);
     return rc;
   }
-  lvc_problem *probs = malloc((size_t)(outer ? outer : 1) * sizeof(*probs));
-  if (!probs) {
-    lvc_set_error(ctx, "host allocation failed");
+  probs = main_problems(ctx, &q, 0, outer, f32);
+  if (!probs)
     return 1;
-  }
-  fill_main(probs, outer, nx, ny, nt, s0, t, alpha, nu, beta, f32);
-  for (int i = 0; i < outer; i++)
-    probs[i].strike = f32 ? (double)(0.001f * (float)(int64_t)i) : 0.001 * (double)(int64_t)i;
   pthread_mutex_lock(&ctx->lock);
   rc = run_batch(ctx, outer, probs, precision, !f32, mem);
   pthread_mutex_unlock(&ctx->lock);
@@ -812,6 +832,80 @@ void lvc_context_ready(struct futhark_context *ctx) {
 
 static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
+/* The static scratch of the allocation-free entry as main's options first ..
+ * first + n - 1 use it, in the order of the offsets: descriptors, tiles,
+ * leaders, geometry, R, Y, y factors.  With the same xshare (0: the batch's
+ * choice), fewer options take no more of it. */
+typedef struct {
+  lvc_main_layout lay;
+  int64_t tiles, lead, geo, R, Y, fac, end;
+  int64_t nxt, nyt;
+} noalloc_layout;
+
+static noalloc_layout noalloc_place(struct futhark_context *ctx, int precision, int first, int n,
+                                    int nx, int ny, int sx, int sy, int xshare) {
+  const int64_t real = precision == LVC_FP64 ? 8 : 4;
+  noalloc_layout L;
+  memset(&L, 0, sizeof(L));
+  lvc_main_layout *lay = &L.lay;
+  lay->first = first;
+  lay->outer = n;
+  lay->gx = lvc_lanes_for(nx, sx);
+  lay->rows = LVC_BLOCK / lay->gx;
+  lay->xtpg = (ny + lay->rows - 1) / lay->rows;
+  lvc_ytile_shape(ny, sy, (int)real, &lay->gy, &lay->ycpl, &lay->cols);
+  lay->ytpo = (nx + lay->cols - 1) / lay->cols;
+  if (xshare <= 0)
+    xshare = lvc_xshare(ctx, precision);
+  if (xshare <= 0) {
+    const int runs[1] = {n}, tiles[1] = {lay->xtpg};
+    xshare = batch_xshare(ctx, precision, 1, runs, tiles);
+  }
+  lay->xshare = xshare;
+  lay->groups = (n + xshare - 1) / xshare;
+  lay->strike_f32 = 1;
+  lay->geo_stride = align64(LVC_GEO_LEN(nx, ny));
+  lay->state_stride = align64((int64_t)nx * ny);
+  L.nxt = (int64_t)lay->groups * lay->xtpg;
+  L.nyt = (int64_t)n * lay->ytpo;
+  L.tiles = align256((int64_t)n * (int64_t)sizeof(lvc_problem));
+  L.lead = L.tiles + align256((L.nxt + L.nyt) * (int64_t)sizeof(lvc_tile));
+  L.geo = L.lead + align256((int64_t)lay->groups * 4);
+  L.R = L.geo + align256((int64_t)n * lay->geo_stride * 8);
+  L.Y = L.R + align256((int64_t)n * lay->state_stride * real);
+  L.fac = L.Y + align256((int64_t)n * lay->state_stride * real);
+  L.end = L.fac + (lvc_seg_is_col(sy) ? align256((int64_t)n * LVC_YFAC_LEN * real) : 0);
+  return L;
+}
+
+/* The sweeps of the options of layout L, prices to out[0 .. n-1]. */
+static int noalloc_sweeps(struct futhark_context *ctx, const lvc_problem *tmpl,
+                          const noalloc_layout *L, int precision, int sx, int sy, float *out) {
+  const int n = L->lay.outer, col = lvc_seg_is_col(sy);
+  char *base = (char *)ctx->scratch;
+  lvc_problem *probs = (lvc_problem *)base;
+  lvc_tile *tl = (lvc_tile *)(base + L->tiles);
+  int32_t *lead = (int32_t *)(base + L->lead);
+  double *geo = (double *)(base + L->geo);
+  void *R = base + L->R, *Y = base + L->Y, *yfac = col ? base + L->fac : NULL;
+  const int ylds = lvc_ytile_lds(tmpl->ny, sy, precision == LVC_FP64 ? 8 : 4);
+  const int xshared = (L->lay.xshare < n ? L->lay.xshare : n) > 1;
+  void *st = (void *)ctx->stream;
+  int e = lvc_launch_main_init(st, tmpl, &L->lay, probs, tl, lead);
+  if (!e)
+    e = lvc_launch_setup(st, precision, probs, n, geo, R);
+  for (int s = 0; !e && s < tmpl->nt - 1; s++) {
+    e = lvc_launch_xsweep(st, precision, sx, probs, tl, (int)L->nxt, geo, R, Y, yfac,
+                          col ? sy : 0, lead, L->lay.groups, xshared);
+    if (!e)
+      e = lvc_launch_ysweep(st, precision, sy, probs, tl + L->nxt, (int)L->nyt, geo, Y, R, ylds,
+                            yfac);
+  }
+  if (!e)
+    e = lvc_launch_gather(st, precision, probs, n, R, out, 0);
+  return lvc_check_hip(ctx, e, "main_noalloc kernel launch");
+}
+
 /* futhark_entry_main without device allocation: the same options, segment
  * lengths, tiles and kernels as futhark_entry_main (so the same bits), with
  * every buffer carved from the static device scratch and the descriptors and
@@ -842,84 +936,34 @@ int futhark_entry_main_noalloc(struct futhark_context *ctx, float *out,
     return 1;
   }
   const int precision = ctx->cfg ? ctx->cfg->precision : LVC_FP32_REFINE;
-  const int64_t real = precision == LVC_FP64 ? 8 : 4;
   int sx = ctx->cfg ? ctx->cfg->seg_x : 0, sy = ctx->cfg ? ctx->cfg->seg_y : 0, tx = 0, ty = 0;
   if (!sx || !sy)
     lvc_tune_peek(ctx, precision, numX, numY, &tx, &ty); /* never times (that allocates) */
   sx = fit_seg(numX, sx ? sx : tx, 0);
   sy = fit_seg(numY, sy ? sy : ty, 1);
 
-  lvc_problem tmpl;
-  memset(&tmpl, 0, sizeof(tmpl));
-  fill_main(&tmpl, 1, numX, numY, numT, s0, t, alpha, nu, beta, 1);
-  lvc_grid_scalars(&tmpl, 1);
-  lvc_main_layout lay;
-  memset(&lay, 0, sizeof(lay));
-  lay.outer = outer;
-  lay.gx = lvc_lanes_for(numX, sx);
-  lay.rows = LVC_BLOCK / lay.gx;
-  lay.xtpg = (numY + lay.rows - 1) / lay.rows;
-  lvc_ytile_shape(numY, sy, (int)real, &lay.gy, &lay.ycpl, &lay.cols);
-  lay.ytpo = (numX + lay.cols - 1) / lay.cols;
-  int xshare = lvc_xshare(ctx, precision);
-  if (xshare <= 0) {
-    const int runs[1] = {outer}, tiles[1] = {lay.xtpg};
-    xshare = batch_xshare(ctx, precision, 1, runs, tiles);
-  }
-  lay.xshare = xshare;
-  lay.groups = (outer + xshare - 1) / xshare;
-  lay.strike_f32 = 1;
-  lay.geo_stride = align64(LVC_GEO_LEN(numX, numY));
-  lay.state_stride = align64((int64_t)numX * numY);
-  const int64_t nxt = (int64_t)lay.groups * lay.xtpg, nyt = (int64_t)outer * lay.ytpo;
-  const int col = lvc_seg_is_col(sy);
-
-  /* the scratch, in order: descriptors, tiles, leaders, geometry, R, Y, y factors */
-  const int64_t o_tiles = align256((int64_t)outer * (int64_t)sizeof(lvc_problem));
-  const int64_t o_lead = o_tiles + align256((nxt + nyt) * (int64_t)sizeof(lvc_tile));
-  const int64_t o_geo = o_lead + align256((int64_t)lay.groups * 4);
-  const int64_t o_R = o_geo + align256((int64_t)outer * lay.geo_stride * 8);
-  const int64_t o_Y = o_R + align256((int64_t)outer * lay.state_stride * real);
-  const int64_t o_fac = o_Y + align256((int64_t)outer * lay.state_stride * real);
-  const int64_t need = o_fac + (col ? align256((int64_t)outer * LVC_YFAC_LEN * real) : 0);
-  if (need > LVC_SCRATCH_BYTES) {
+  const lvc_problem tmpl = main_problem(numX, numY, numT, s0, t, alpha, nu, beta, 1);
+  noalloc_layout L = noalloc_place(ctx, precision, 0, outer, numX, numY, sx, sy, 0);
+  if (L.end > LVC_SCRATCH_BYTES) {
     lvc_set_error(ctx, "main_noalloc: main(%d, %d, %d, %d) needs %lld bytes of device scratch; "
                        "the static scratch holds %lld",
-                  outer, numX, numY, numT, (long long)need, (long long)LVC_SCRATCH_BYTES);
+                  outer, numX, numY, numT, (long long)L.end, (long long)LVC_SCRATCH_BYTES);
     return 1;
   }
+  pthread_mutex_lock(&ctx->lock);
+  int rc = 0, first = 0, end = outer;
   if (lvc_modes_fit(&tmpl)) {
     /* the work memory (lambda, f and a row of coefficients per option) is
      * less than the geometry above */
-    pthread_mutex_lock(&ctx->lock);
-    const int rc = lvc_modes_main(ctx, &tmpl, outer, 1, (double *)ctx->scratch, out, 0);
-    pthread_mutex_unlock(&ctx->lock);
-    return rc;
+    rc = lvc_modes_main(ctx, &tmpl, outer, 1, (double *)ctx->scratch, out, 0);
+    lvc_modes_far(&tmpl, outer, 1, &first, &end);
   }
-  char *base = (char *)ctx->scratch;
-  lvc_problem *probs = (lvc_problem *)base;
-  lvc_tile *tl = (lvc_tile *)(base + o_tiles);
-  int32_t *lead = (int32_t *)(base + o_lead);
-  double *geo = (double *)(base + o_geo);
-  void *R = base + o_R, *Y = base + o_Y, *yfac = col ? base + o_fac : NULL;
-  const int ylds = lvc_ytile_lds(numY, sy, (int)real);
-  const int xshared = (xshare < outer ? xshare : outer) > 1;
-
-  void *st = (void *)ctx->stream;
-  pthread_mutex_lock(&ctx->lock);
-  int e = lvc_launch_main_init(st, &tmpl, &lay, probs, tl, lead);
-  if (!e)
-    e = lvc_launch_setup(st, precision, probs, outer, geo, R);
-  for (int s = 0; !e && s < numT - 1; s++) {
-    e = lvc_launch_xsweep(st, precision, sx, probs, tl, (int)nxt, geo, R, Y, yfac,
-                          col ? sy : 0, lead, lay.groups, xshared);
-    if (!e)
-      e = lvc_launch_ysweep(st, precision, sy, probs, tl + nxt, (int)nyt, geo, Y, R, ylds,
-                            yfac);
+  if (!rc && first < end) {
+    if (end - first < outer)
+      L = noalloc_place(ctx, precision, first, end - first, numX, numY, sx, sy,
+                        L.lay.xshare);
+    rc = noalloc_sweeps(ctx, &tmpl, &L, precision, sx, sy, out + first);
   }
-  if (!e)
-    e = lvc_launch_gather(st, precision, probs, outer, R, out, 0);
-  const int rc = lvc_check_hip(ctx, e, "main_noalloc kernel launch");
   pthread_mutex_unlock(&ctx->lock);
   return rc;
 }

@@ -92,7 +92,7 @@ typedef struct lvc_main_layout {
   int32_t ytpo, cols, gy, ycpl;  /* y: tiles per option, columns per tile, lanes
                                     (segments) per column, columns per lane (groups) */
   int32_t strike_f32;            /* strikes 0.001f*i in f32 (else 0.001*i in f64) */
-  int32_t pad_;
+  int32_t first;                 /* option 0 is main's option `first` */
   int64_t geo_stride, state_stride; /* per option, in doubles / in reals */
 } lvc_main_layout;
 

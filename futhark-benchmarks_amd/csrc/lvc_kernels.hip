@@ -1281,7 +1281,8 @@ __global__ __launch_bounds__(256) void lvc_main_init_kernel(const lvc_problem tm
     const int p = (int)i;
     lvc_problem q = tmpl;
     // LocVolCalib.fut:247, strike_i = 0.001 * i (in f32 for the f32 entry)
-    q.strike = lay.strike_f32 ? (double)(0.001f * (float)p) : 0.001 * (double)p;
+    const int k = lay.first + p;
+    q.strike = lay.strike_f32 ? (double)(0.001f * (float)k) : 0.001 * (double)k;
     q.geo_off = (int64_t)p * lay.geo_stride;
     q.state_off = (int64_t)p * lay.state_stride;
     q.k = -1;

@@ -207,6 +207,9 @@ int lvc_same_factor(const lvc_problem *a, const lvc_problem *b);
 
 /* prices by separation of x (lvc_modes.c) */
 int lvc_modes_fit(const lvc_problem *q);
+int lvc_modes_strike(const lvc_problem *q, double strike, int out_f64);
+double lvc_main_strike(int i, int f32);
+void lvc_modes_far(const lvc_problem *q, int outer, int f32, int *first, int *end);
 int64_t lvc_modes_main_work(int outer, int nx);
 int lvc_modes_main(struct futhark_context *ctx, const lvc_problem *q, int outer,
                    int strike_f32, double *work, void *out, int out_f64);
