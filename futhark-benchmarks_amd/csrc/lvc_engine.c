@@ -617,10 +617,10 @@ static void note_index(struct futhark_context *ctx, const lvc_problem *q) {
 }
 
 /* Runs a batch end to end into a new device array of n prices: in FP64 the
- * problems whose x direction separates (lvc_modes_fit) and whose price the
- * modes do not lose (lvc_modes_strike) by their modes, the others, and the FP32
- * forms, whose FP64 prices show the arithmetic that was asked for, by the
- * sweeps.  A problem's way depends on the precision and its
+ * problems whose x direction separates (lvc_modes_fit), whose price the modes
+ * do not lose (lvc_modes_strike) and which cost less that way (lvc_modes_pay) by
+ * their modes, the others, and the FP32 forms, whose FP64 prices show the
+ * arithmetic that was asked for, by the sweeps.  A problem's way depends on the precision and its
  * own sizes and parameters only, so its price has the same bits alone and in
  * any batch. */
 static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *probs,
@@ -639,7 +639,8 @@ static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *prob
     q.out_index = p;
     if (p == 0)
       note_index(ctx, &q);
-    if (precision == LVC_FP64 && lvc_modes_fit(&q) && lvc_modes_strike(&q, q.strike, 1)) {
+    if (precision == LVC_FP64 && lvc_modes_fit(&q) && lvc_modes_pay(&q) &&
+        lvc_modes_strike(&q, q.strike, 1)) {
       by[nm++] = q;
       /* "lvc.autotune" asks for every class's sweeps to be timed */
       int sx, sy;

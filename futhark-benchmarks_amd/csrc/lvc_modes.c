@@ -42,6 +42,30 @@ int lvc_modes_fit(const lvc_problem *q) {
   return 2.0 * beta * log(xn / x1) < log(1e8) && beta * log(s0 / x1) < log(256.0);
 }
 
+/* Whether a problem of a batch costs less by its modes than by the sweeps.  A
+ * grid's modes are numX / 4 waves that each pass over numX nodes some seven
+ * times whatever numY and the steps are (and from 512 nodes on their LDS leaves
+ * few waves per CU), and its sweeps numX numY points per step.  Measured, ms
+ * by the sweeps / by the modes, numX x numY x steps:
+ *   512 problems   192 x 16 x 8 0.68 / 0.83, 192 x 8 x 31 1.15 / 0.84,
+ *                  256 x 64 x 8 1.03 / 1.15, 256 x 128 x 8 1.64 / 1.20,
+ *                  512 x 128 x 8 3.15 / 3.44, 512 x 32 x 63 5.78 / 4.46,
+ *                  768 x 128 x 8 6.8 / 8.3, 768 x 32 x 63 13.2 / 9.5,
+ *                  1024 x 16 x 8 1.5 / 16.2, 1024 x 32 x 63 15.4 / 18.1,
+ *                  1024 x 64 x 63 28.9 / 19.1
+ *   8192 problems  64 x 16 x 8 2.10 / 2.11, 128 x 16 x 8 2.95 / 4.41,
+ *                  128 x 8 x 31 5.93 / 4.30, 256 x 8 x 31 8.4 / 11.2,
+ *                  256 x 16 x 31 12.2 / 11.7
+ * A few problems alone, which two launches a step leave waiting, are faster by
+ * the modes everywhere (16 of 256 x 8 x 31 0.80 / 0.37); the rule is on the
+ * problem's own sizes, so that its price does not depend on its batch.  main's
+ * strikes share one grid's modes, which are faster at every size (one strike on
+ * 1024 x 4 x 7 0.18 / 0.12). */
+int lvc_modes_pay(const lvc_problem *q) {
+  const double nx = q->nx, rows = (double)q->ny * (double)(q->nt - 1);
+  return nx <= 64.0 || (rows >= 2.25 * (nx - 48.0) && rows >= nx * nx / 300.0);
+}
+
 /* The normal call price in units of the standard deviation, struck d above
  * the mean (less than 1e-20 past 9). */
 static double normal_call(double d) {

@@ -207,6 +207,7 @@ int lvc_same_factor(const lvc_problem *a, const lvc_problem *b);
 
 /* prices by separation of x (lvc_modes.c) */
 int lvc_modes_fit(const lvc_problem *q);
+int lvc_modes_pay(const lvc_problem *q);
 int lvc_modes_strike(const lvc_problem *q, double strike, int out_f64);
 double lvc_main_strike(int i, int f32);
 void lvc_modes_far(const lvc_problem *q, int outer, int f32, int *first, int *end);

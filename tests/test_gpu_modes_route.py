@@ -1,0 +1,52 @@
+"""Which problems of an FP64 batch go by the modes and which by the sweeps: by
+the kernels that the profiling report counts, the prices on both sides of the
+line against the FP64 oracle.  Tolerance: the FP64 form's bar of 1e-10.
+"""
+import json
+
+import numpy as np
+import pytest
+
+from oracle import oracle
+import locvolcalib as lvc
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("numX", "numY", "numT", "s0", "strike", "t", "alpha", "nu", "beta")
+MARKET = (0.03, 5.0, 0.2, 0.6, 0.5)
+
+
+def route(ctx, call):
+    """The call's result and the kernels it launched."""
+    before = json.loads(ctx.report())
+    out = call()
+    after = json.loads(ctx.report())
+    count = {k: v["count"] - before.get(k, {"count": 0})["count"] for k, v in after.items()
+             if isinstance(v, dict)}
+    return out, {k for k, c in count.items() if c}
+
+
+def problem(nx, ny, nt, strike):
+    s0, t, alpha, nu, beta = MARKET
+    return dict(numX=[nx], numY=[ny], numT=[nt], s0=[s0], strike=[strike], t=[t], alpha=[alpha],
+                nu=[nu], beta=[beta])
+
+
+# (numX, numY, numT), by the modes: narrow grids always; wide ones where
+# numY (numT - 1) reaches 2.25 (numX - 48) and numX^2 / 300
+@pytest.mark.parametrize("shape,modes", [
+    ((64, 3, 7), True), ((65, 6, 7), False), ((65, 7, 7), True), ((256, 18, 27), True),
+    ((256, 18, 26), False), ((512, 58, 19), True), ((512, 58, 18), False),
+    ((1024, 16, 8), False), ((1024, 583, 7), True), ((1024, 582, 7), False)])
+def test_batch_by_size(shape, modes):
+    print(f"case: route of {shape}", flush=True)
+    p = problem(*shape, 0.02)
+    with lvc.LocVolCalib(profiling=True) as ctx:
+        got, kernels = route(ctx, lambda: ctx.main_batch(**p, precision=lvc.PRECISION_FP64))
+        assert ("lvc_modes" in kernels) == modes and ("lvc_xsweep" in kernels) != modes
+        # main's strikes share one grid's modes at every size
+        by_main, kernels = route(ctx, lambda: ctx.main_f64(21, *shape, *MARKET))
+        assert "lvc_modes" in kernels and "lvc_xsweep" not in kernels
+    ref = oracle.batch(*[p[k] for k in KEYS], dtype=np.float64, thomas=True, nthreads=8)
+    assert abs(got[0] - ref[0]) < 1e-10 * ref[0]
+    assert abs(by_main[20] - ref[0]) < 1e-10 * ref[0]
