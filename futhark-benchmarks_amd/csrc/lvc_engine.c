@@ -616,6 +616,14 @@ static void note_index(struct futhark_context *ctx, const lvc_problem *q) {
   ctx->dbg_index_valid = 1;
 }
 
+/* "lvc.autotune" asks for the sweeps of every class that a call meets to be
+ * timed, also of one that goes by the modes. */
+static void autotune_class(struct futhark_context *ctx, int precision, const lvc_problem *q) {
+  int sx, sy;
+  if (ctx->cfg && ctx->cfg->autotune)
+    lvc_choose_segs(ctx, precision, q->nx, q->ny, &sx, &sy);
+}
+
 /* Runs a batch end to end into a new device array of n prices: in FP64 the
  * problems whose x direction separates (lvc_modes_fit), whose price the modes
  * do not lose (lvc_modes_strike) and which cost less that way (lvc_modes_pay) by
@@ -642,10 +650,7 @@ static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *prob
     if (precision == LVC_FP64 && lvc_modes_fit(&q) && lvc_modes_pay(&q) &&
         lvc_modes_strike(&q, q.strike, 1)) {
       by[nm++] = q;
-      /* "lvc.autotune" asks for every class's sweeps to be timed */
-      int sx, sy;
-      if (ctx->cfg && ctx->cfg->autotune)
-        lvc_choose_segs(ctx, precision, q.nx, q.ny, &sx, &sy);
+      autotune_class(ctx, precision, &q);
     } else {
       by[n - ++ns] = q;
     }
@@ -741,6 +746,7 @@ static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int 
     double *work = NULL;
     pthread_mutex_lock(&ctx->lock);
     note_index(ctx, &q);
+    autotune_class(ctx, precision, &q);
     rc = lvc_dev_alloc(ctx, ob, mem) || lvc_dev_alloc(ctx, wb, (void **)&work) ||
          lvc_modes_main(ctx, &q, outer, f32, work, *mem, !f32);
     lvc_dev_free(ctx, work, wb);

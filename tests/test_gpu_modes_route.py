@@ -50,3 +50,22 @@ def test_batch_by_size(shape, modes):
     ref = oracle.batch(*[p[k] for k in KEYS], dtype=np.float64, thomas=True, nthreads=8)
     assert abs(got[0] - ref[0]) < 1e-10 * ref[0]
     assert abs(by_main[20] - ref[0]) < 1e-10 * ref[0]
+
+
+@pytest.mark.parametrize("precision", [lvc.PRECISION_FP32_REFINE, lvc.PRECISION_FP64])
+def test_main_autotunes_its_class(tmp_path, precision):
+    """With "lvc.autotune" a call of main leaves its class's segment lengths in
+    the cache file, for the sweeps of the batch, the server and the
+    allocation-free entry, whichever way main itself goes."""
+    print(f"case: main autotunes, precision {precision}", flush=True)
+    cache = tmp_path / "lvc.tuning"
+    with lvc.LocVolCalib(cache_file=str(cache), precision=precision,
+                         tuning={"lvc.autotune": 1}) as ctx:
+        got = ctx.main(3, 40, 36, 20, *MARKET)
+        if precision == lvc.PRECISION_FP64:
+            ctx.main_f64(3, 48, 36, 20, *MARKET)
+    lines = [tuple(int(v) for v in line.split()[:3]) for line in cache.read_text().splitlines()]
+    want = [(precision, 40, 36)] + [(precision, 48, 36)] * (precision == lvc.PRECISION_FP64)
+    assert lines == want
+    with lvc.LocVolCalib(precision=precision) as ctx:
+        assert np.array_equal(got, ctx.main(3, 40, 36, 20, *MARKET))
