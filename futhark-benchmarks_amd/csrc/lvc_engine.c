@@ -960,9 +960,14 @@ int futhark_entry_main_noalloc(struct futhark_context *ctx, float *out,
   pthread_mutex_lock(&ctx->lock);
   int rc = 0, first = 0, end = outer;
   if (lvc_modes_fit(&tmpl)) {
-    /* the work memory (lambda, f and a row of coefficients per option) is
-     * less than the geometry above */
+    /* The work memory, lambda and f (16 KB at most) and a row of coefficients
+     * per option (a third of its states at most), is within the scratch where
+     * the layout is.  No events among the launches: making them allocates, and
+     * the caller may be capturing. */
+    const int paused = ctx->prof_paused;
+    ctx->prof_paused = 1;
     rc = lvc_modes_main(ctx, &tmpl, outer, 1, (double *)ctx->scratch, out, 0);
+    ctx->prof_paused = paused;
     lvc_modes_far(&tmpl, outer, 1, &first, &end);
   }
   if (!rc && first < end) {

@@ -69,3 +69,15 @@ def test_main_autotunes_its_class(tmp_path, precision):
     assert lines == want
     with lvc.LocVolCalib(precision=precision) as ctx:
         assert np.array_equal(got, ctx.main(3, 40, 36, 20, *MARKET))
+
+
+def test_noalloc_is_not_profiled():
+    """Profiling does not cover the allocation-free entry (an event made for it
+    would be an allocation, and its caller may be capturing)."""
+    print("case: main_noalloc with profiling", flush=True)
+    with lvc.LocVolCalib(profiling=True) as ctx:
+        got, kernels = route(ctx, lambda: ctx.main_noalloc(5, 40, 36, 20, *MARKET))
+        assert not kernels
+        want, kernels = route(ctx, lambda: ctx.main(5, 40, 36, 20, *MARKET))
+        assert kernels == {"lvc_modes", "lvc_evolve", "lvc_price"}
+        assert np.array_equal(got, want)
