@@ -649,7 +649,10 @@ __global__ __launch_bounds__(kThreads) void op_many_kernel(
     };
     asm volatile("" ::"v"(seen));
     float pay[MC];
-    bool good = false;
+    // the models whose payoff stands: a model's path is repriced for its own
+    // prices' sake only, so its mean does not depend on which share the pass
+    const uint32_t all = (1u << M) - 1u;
+    uint32_t good = 0u;
     if (fits) {
       LogPath<3> path[MC];
 #pragma unroll
@@ -739,12 +742,11 @@ __global__ __launch_bounds__(kThreads) void op_many_kernel(
       static_assert(D % 2 == 1, "a last step");
       step(D - 1, even);
       stream_rest(date_at, D * sizeof(Date));
-      good = true;
 #pragma unroll
       for (int m = 0; m < MC; ++m)
-        if (m < M) good = path[m].pay(discts + m * K, &pay[m]) && good;
+        if (m < M && path[m].pay(discts + m * K, &pay[m])) good |= 1u << m;
     }
-    if (__any(!good)) {
+    if (__any(good != all)) {
       // any tables, any values: all rows in private memory, starting at zero
       // (:153), indexes clamped to the row so that no input makes an access out
       // of bounds (the reference reads bb_inds unchecked, :156)
@@ -779,7 +781,7 @@ __global__ __launch_bounds__(kThreads) void op_many_kernel(
       for (int m = 0; m < MC; ++m) {
         if (m < M) {
           const float p = product_payoff<3>(mk, m, [&](int u, int d) { return rows[u][d]; });
-          if (!good) pay[m] = p;
+          if (!(good >> m & 1u)) pay[m] = p;
         }
       }
     }
