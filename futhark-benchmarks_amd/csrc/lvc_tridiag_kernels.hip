@@ -273,7 +273,9 @@ __device__ __forceinline__ void stage_out(const float (&st)[kThreads][CH + 1],
 // division operator instead, zeros, denormals and infinities included.  (A NaN
 // passes through both.)  That costs four times the call's time, so the
 // right-hand sides, which a caller scales as he likes, are divided by the operator
-// throughout and only the matrix can leave the range.  57600 systems: Thomas 38.7 -> 37.1 us at 115 unknowns,
+// throughout and only the matrix can leave the range: its entries, not a_0 and
+// c_(m-1), where a caller may leave anything and which the kernels take as 0.
+// 57600 systems: Thomas 38.7 -> 37.1 us at 115 unknowns,
 // the scan form, which has five divisions a row and three of them by the same
 // number, 57.1 -> 55.3 (and 49.4 -> 44.1 at 128).
 constexpr float kDivLow = 0x1p-40f, kDivHigh = 0x1p40f;
@@ -343,6 +345,7 @@ void tridag_par_staged_kernel(const float *__restrict__ a, const float *__restri
     if (ch + 1 < nch) {
       fetch<CH>(pa, pb, pc, py, a, b, c, y, s0, rows, m, i0 + CH, lane);
     }
+    S.v[2][lane][min(m - 1 - i0, CH)] = 0.0f;  // column CH is padding
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const int i = i0 + j;
@@ -383,7 +386,7 @@ void tridag_par_staged_kernel(const float *__restrict__ a, const float *__restri
       // this row's element of recurrence 3
       fw0[i] = yy / bb;  // a right-hand side may be of any size
       fw1[i] = 0.0f - quotient(ci, bb, rbb);
-      range.numerators(ai, ci);
+      range.numerators(i == 0 ? 0.0f : ai, ci);
       bprev = bb;
       rprev = rbb;
       cprev = ci;
@@ -526,6 +529,8 @@ void tridag_seq_aligned_kernel(const float *__restrict__ a, const float *__restr
     }
   };
 
+  // the next slot where a system starts, this lane's own or another in its slots
+  int start = sh % m;
   fetch_chunk(0);
 #pragma unroll
   for (int k = 0; k < kChunks; ++k) {
@@ -534,6 +539,7 @@ void tridag_seq_aligned_kernel(const float *__restrict__ a, const float *__restr
     for (int arr = 0; arr < 4; ++arr) deposit<CH>(S.v[arr], pf[arr], lane);
     __syncthreads();
     if (k + 1 < nch) fetch_chunk(k + 1);
+    for (; start < (k + 1) * CH; start += m) S.v[0][lane][start - k * CH] = 0.0f;
     // Thomas' first row (tridiag.fut:82-83), c_0/b_0 and y_0/b_0, from this
     // lane's column 0 (slot sh, in chunk 0), divided once here rather than
     // at every step of the chunk
