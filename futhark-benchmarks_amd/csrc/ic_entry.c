@@ -345,7 +345,7 @@ static int run_calibration(struct futhark_context *ctx, ic_call *c, int32_t conv
   if (!e) {
     tok = lvc_prof_begin(ctx, "ic_eval");
     e = ic_launch_eval(st, c->sw, c->per, &c->pop_lists, ps[0].genomes, pop, hx, hw, c->nherm,
-                       c->nswap, IC_OUT_TERMS, c->terms, NULL);
+                       c->nswap, IC_OUT_TERMS, 0, c->terms, NULL);
     lvc_prof_end(ctx, tok);
   }
   if (!e) {
@@ -358,7 +358,7 @@ static int run_calibration(struct futhark_context *ctx, ic_call *c, int32_t conv
   for (int32_t it = 0; !e && it < conv; it++) {
     tok = lvc_prof_begin(ctx, "ic_eval");
     e = ic_launch_eval(st, c->sw, c->per, &c->pop_lists, ps[at].props, pop, hx, hw, c->nherm,
-                       c->nswap, IC_OUT_TERMS, c->terms, NULL);
+                       c->nswap, IC_OUT_TERMS, 0, c->terms, NULL);
     lvc_prof_end(ctx, tok);
     if (!e) {
       tok = lvc_prof_begin(ctx, "ic_step");
@@ -372,7 +372,7 @@ static int run_calibration(struct futhark_context *ctx, ic_call *c, int32_t conv
   if (!e) e = ic_launch_winner(st, pop, ps[at].genomes, ps[at].logliks, out, winner);
   if (!e && c->nswap > 0)
     e = ic_launch_eval(st, c->sw, c->per, &c->one_lists, winner, 1, hx, hw, c->nherm, c->nswap,
-                       IC_OUT_SUMMARY, summary, NULL);
+                       IC_OUT_SUMMARY, 0, summary, NULL);
   lvc_prof_end(ctx, tok);
   return lvc_check_hip(ctx, e, "InterestCalib kernels");
 }
@@ -562,6 +562,18 @@ int interestcalib_trace(struct futhark_context *ctx, const int32_t pop, const in
   return rc;
 }
 
+/* Whether the evaluation's divisions stay in the range of their short form:
+ * the genes 1e-3 .. 1 of the calibration, with room to spare. */
+static int short_range(const float *genomes, size_t n) {
+  for (size_t i = 0; i < n; i++, genomes += 5)
+    for (int j = 0; j < 5; j++) {
+      const float g = fabsf(genomes[j]);
+      if (!(g <= 0x1p4f && (j == 2 || genomes[j] >= 0x1p-12f)))
+        return 0;
+    }
+  return 1;
+}
+
 int interestcalib_eval(struct futhark_context *ctx, const int32_t ngenomes, const float *genomes,
                        const struct futhark_f32_2d *swaptions,
                        const struct futhark_f32_1d *herm_coefs,
@@ -591,6 +603,7 @@ int interestcalib_eval(struct futhark_context *ctx, const int32_t ngenomes, cons
   ic_call c;
   float *pq = NULL;
   const size_t np = (size_t)ngenomes;
+  const int ieee = !short_range(genomes, np);
   size_t pq_bytes = 0;
   int rc = call_prepare(ctx, &c, &swaptions->a, ngenomes, (int32_t)nh) || alloc_state(ctx, &c);
   const size_t ns = (size_t)c.nswap;
@@ -610,10 +623,10 @@ int interestcalib_eval(struct futhark_context *ctx, const int32_t ngenomes, cons
     int e = 0;
     if (ns > 0) {
       e = ic_launch_eval(st, c.sw, c.per, &c.pop_lists, c.state, ngenomes, hx, hw, c.nherm,
-                         c.nswap, IC_OUT_PRICES, pq, pq + np * ns);
+                         c.nswap, IC_OUT_PRICES, ieee, pq, pq + np * ns);
       if (!e)
         e = ic_launch_eval(st, c.sw, c.per, &c.pop_lists, c.state, ngenomes, hx, hw, c.nherm,
-                           c.nswap, IC_OUT_TERMS, c.terms, NULL);
+                           c.nswap, IC_OUT_TERMS, ieee, c.terms, NULL);
     }
     if (!e)
       e = ic_launch_step(st, ngenomes, c.nswap, c.terms, &ps[0], &ps[1], 1, 0, &none, &dv,

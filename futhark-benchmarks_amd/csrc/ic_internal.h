@@ -91,11 +91,13 @@ int ic_launch_init(void *stream, int32_t pop, const ic_dirvec *dv, float *genome
  * work lists.
  * IC_OUT_TERMS: out0 [nswap][npop] the log-likelihood terms (:606-625);
  * IC_OUT_PRICES: out0, out1 [npop][nswap] quotes and prices;
- * IC_OUT_SUMMARY (npop 1): out0 [nswap][3] makeSummary's rows (:205-213). */
+ * IC_OUT_SUMMARY (npop 1): out0 [nswap][3] makeSummary's rows (:205-213).
+ * ieee: divisions by the operator, for genomes whose values may leave the range
+ * of the short form; the same bits where they do not. */
 int ic_launch_eval(void *stream, const ic_swaption *sw, const ic_period *periods,
                    const ic_worklists *wl, const float *genomes, int32_t npop,
                    const float *herm_x, const float *herm_w, int32_t nherm, int32_t nswap,
-                   int mode, float *out0, float *out1);
+                   int mode, int ieee, float *out0, float *out1);
 
 /* One launch: the log-likelihood of each genome, the sum of its terms over
  * the swaptions in a fixed order (32 threads per genome each sum the

@@ -38,9 +38,10 @@
 // correctly rounded quotient, in 7 instructions, where neither the reciprocal
 // nor the residual underflows: |b| and |a / b| within 2^+-125, |a| above
 // 2^-101 or 0.  v_div_fixup gives the quotients of zeros, infinities and NaN.
-// The evaluation's operands are far inside (root finder: |f| below 600, every
-// difference an ulp of 1 or more); beyond it a quotient may be off by one
-// denormal ulp.
+// With the calibration's genomes (1e-3 .. 1) the evaluation's operands are far
+// inside (root finder: |f| below 600, every difference an ulp of 1 or more).
+// interestcalib_eval takes any genome: where one is outside 2^-12 .. 2^4
+// (ic_entry.c) the kernels divide by the operator.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -129,31 +130,41 @@ __device__ inline int32_t today() { return date_of_gregorian(2012, 1, 1, 12, 0);
 
 __device__ inline float zc(int32_t t) { return expf(-kR * act365(t, today())); }  // :48
 
-__device__ __forceinline__ float rcp_rn(float b) {
-  const float r = __builtin_amdgcn_rcpf(b);
-  return fmaf(fmaf(-b, r, 1.0f), r, r);
-}
-__device__ __forceinline__ float quot(float a, float b) {
-  const float r = rcp_rn(b), q = a * r;
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-b, q, a), r, q), b, a);
-}
-__device__ __forceinline__ float recip(float b) {
-  return __builtin_amdgcn_div_fixupf(rcp_rn(b), b, 1.0f);
-}
-// x / sqrt(2) (the divisor's correctly rounded reciprocal is a constant)
-__device__ __forceinline__ float over_sqrt2(float x) {
-  constexpr float c = 1.41421354f, r = 1.0f / c;  // sqrtf(2.0f)
-  const float q = x * r;
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-c, q, x), r, q), c, x);
-}
+// The two forms of the divisions: by these steps where every operand is in
+// range (Short), and IEEE's (Ieee).
+struct Short {
+  static __device__ __forceinline__ float rcp_rn(float b) {
+    const float r = __builtin_amdgcn_rcpf(b);
+    return fmaf(fmaf(-b, r, 1.0f), r, r);
+  }
+  static __device__ __forceinline__ float quot(float a, float b) {
+    const float r = rcp_rn(b), q = a * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-b, q, a), r, q), b, a);
+  }
+  static __device__ __forceinline__ float recip(float b) {
+    return __builtin_amdgcn_div_fixupf(rcp_rn(b), b, 1.0f);
+  }
+  // x / sqrt(2) (the divisor's correctly rounded reciprocal is a constant)
+  static __device__ __forceinline__ float over_sqrt2(float x) {
+    constexpr float c = 1.41421354f, r = 1.0f / c;  // sqrtf(2.0f)
+    const float q = x * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-c, q, x), r, q), c, x);
+  }
+};
+struct Ieee {
+  static __device__ __forceinline__ float quot(float a, float b) { return a / b; }
+  static __device__ __forceinline__ float recip(float b) { return 1.0f / b; }
+  static __device__ __forceinline__ float over_sqrt2(float x) { return x / sqrtf(2.0f); }
+};
 
 // ---- the math module (:56-101) --------------------------------------------
 // Abramowitz & Stegun 7.1.26 without its exp factor
+template <typename D>
 __device__ inline float erf_poly(float x) {
   const float p = 0.3275911f;
   const float a1 = 0.254829592f, a2 = -0.284496736f, a3 = 1.421413741f, a4 = -1.453152027f,
               a5 = 1.061405429f;
-  const float t = recip(1.0f + p * x);
+  const float t = D::recip(1.0f + p * x);
   const float t2 = t * t;
   const float t3 = t * t2;
   const float t4 = t2 * t2;
@@ -161,24 +172,27 @@ __device__ inline float erf_poly(float x) {
   return a1 * t + a2 * t2 + a3 * t3 + a4 * t4 + a5 * t5;
 }
 
+template <typename D>
 __device__ inline float ugaussian_P(float x) {  // :60-93
-  const float u = over_sqrt2(x);
-  const float e = u < 0.0f ? -(1.0f - erf_poly(-u) * expf(-(u * u)))
-                           : 1.0f - erf_poly(u) * expf(-(u * u));
+  const float u = D::over_sqrt2(x);
+  const float e = u < 0.0f ? -(1.0f - erf_poly<D>(-u) * expf(-(u * u)))
+                           : 1.0f - erf_poly<D>(u) * expf(-(u * u));
   return 0.5f * (1.0f + e);
 }
 
+template <typename D>
 __device__ inline float ugaussian_P_exp(float x, float exp_factor) {  // :95-101
-  const float u = fabsf(over_sqrt2(x));
-  const float e = erf_poly(u);
+  const float u = fabsf(D::over_sqrt2(x));
+  const float e = erf_poly<D>(u);
   const float res = 0.5f * e * expf(exp_factor - u * u);
   return 0.0f <= x ? expf(exp_factor) - res : res;
 }
 
+template <typename D>
 __device__ inline float log_likelihood(float y_ref, float y) {  // Cauchy, :606-625
   const float gamma = (fabsf(y_ref) / 50.0f) * kCauchyOffs + 0.01f;
-  const float x = quot(y - y_ref, gamma);
-  const float pdf = recip(kPi * gamma * (1.0f + x * x));
+  const float x = D::quot(y - y_ref, gamma);
+  const float pdf = D::recip(kPi * gamma * (1.0f + x * x));
   return logf(pdf + 1.0e-20f);
 }
 
@@ -203,15 +217,17 @@ __device__ inline float gene_max(int j) { return j < 3 ? 1.0f - kEps0 : 0.2f; }
 constexpr float kAmplRatio = 0.005f;  // moves_unif_ampl_ratio, :248
 
 // ---- G2++ (:322-413) -------------------------------------------------------------
+template <typename D>
 __device__ inline float b_fun(float z, float tau) {
-  return quot(1.0f - expf(-z * tau), z);
+  return D::quot(1.0f - expf(-z * tau), z);
 }
 
+template <typename D>
 __device__ inline float t_fun(float sigma, float x, float tau) {
   const float expxtau = expf(-x * tau);
   const float exp2xtau = expxtau * expxtau;
-  return quot(sigma * sigma, x * x) *
-         (tau + quot(2.0f, x) * expxtau - recip(2.0f * x) * exp2xtau - quot(3.0f, 2.0f * x));
+  return D::quot(sigma * sigma, x * x) *
+         (tau + D::quot(2.0f, x) * expxtau - D::recip(2.0f * x) * exp2xtau - D::quot(3.0f, 2.0f * x));
 }
 
 struct Genome {
@@ -219,38 +235,41 @@ struct Genome {
 };
 
 // bigv (:336-352): V(tau) and B_a(tau), B_b(tau)
+template <typename D>
 __device__ inline float bigv(const Genome &g, float tau, float *ba, float *bb) {
   const float sigma = g.sigma == 0.0f ? 1.0e-10f : g.sigma;
-  *ba = b_fun(g.a, tau);
-  *bb = b_fun(g.b, tau);
-  const float t1 = t_fun(sigma, g.a, tau);
-  const float t2 = t_fun(g.nu, g.b, tau);
-  const float t3 = quot(2.0f * g.rho * g.nu * sigma, g.a * g.b) *
-                   (tau - *ba - *bb + b_fun(g.a + g.b, tau));
+  *ba = b_fun<D>(g.a, tau);
+  *bb = b_fun<D>(g.b, tau);
+  const float t1 = t_fun<D>(sigma, g.a, tau);
+  const float t2 = t_fun<D>(g.nu, g.b, tau);
+  const float t3 = D::quot(2.0f * g.rho * g.nu * sigma, g.a * g.b) *
+                   (tau - *ba - *bb + b_fun<D>(g.a + g.b, tau));
   return t1 + t2 + t3;
 }
 
 // bigmx / bigmy (:364-413) over (today, maturity, today, maturity): ts =
 // tmat0 = tmats = t0, tmatt = s0 = 0
+template <typename D>
 __device__ inline float bigmx(const Genome &g, float tmat0) {
   const float a = g.a, b = g.b, rho = g.rho, nu = g.nu, sigma = g.sigma;
   const float ts = tmat0, tmatt = 0.0f, tmats = tmat0, t0 = tmat0, s0 = 0.0f;
-  const float tmp1 = quot(sigma * sigma, a * a) + quot(sigma * rho * nu, a * b);
+  const float tmp1 = D::quot(sigma * sigma, a * a) + D::quot(sigma * rho * nu, a * b);
   const float tmp2 = 1.0f - expf(-a * ts);
-  const float tmp3 = quot(sigma * sigma, 2.0f * a * a);
-  const float tmp4 = quot(rho * sigma * nu, b * (a + b));
+  const float tmp3 = D::quot(sigma * sigma, 2.0f * a * a);
+  const float tmp4 = D::quot(rho * sigma * nu, b * (a + b));
   const float tmp5 = expf(-a * tmatt) - expf(-a * (tmats + ts));
   const float tmp6 = expf(-b * tmatt) - expf(-b * tmat0 - a * t0 + (a + b) * s0);
   return tmp1 * tmp2 - (tmp3 * tmp5) - (tmp4 * tmp6);
 }
 
+template <typename D>
 __device__ inline float bigmy(const Genome &g, float tmat0) {
   const float a = g.a, b = g.b, rho = g.rho, nu = g.nu, sigma = g.sigma;
   const float ts = tmat0, tmatt = 0.0f, tmats = tmat0, t0 = tmat0, s0 = 0.0f;
-  const float tmp1 = quot(nu * nu, b * b) + quot(sigma * rho * nu, a * b);
+  const float tmp1 = D::quot(nu * nu, b * b) + D::quot(sigma * rho * nu, a * b);
   const float tmp2 = 1.0f - expf(-b * ts);
-  const float tmp3 = quot(nu * nu, 2.0f * b * b);
-  const float tmp4 = quot(sigma * rho * nu, a * (a + b));
+  const float tmp3 = D::quot(nu * nu, 2.0f * b * b);
+  const float tmp4 = D::quot(sigma * rho * nu, a * (a + b));
   const float tmp5 = expf(-b * tmatt) - expf(-b * (tmats + ts));
   const float tmp6 = expf(-a * tmatt) - expf(-a * tmat0 - b * t0 + (a + b) * s0);
   return tmp1 * tmp2 - (tmp3 * tmp5) - (tmp4 * tmp6);
@@ -343,7 +362,7 @@ __device__ __forceinline__ float to_solve(const Periods<K, V> &P, const float (&
 
 // rootFinding_Brent (:124-185); the loop ends where the reference's
 // iterations stop changing its state
-template <bool MID, int K, int V>
+template <typename D, bool MID, int K, int V>
 __device__ float brent(const Periods<K, V> &P, const float (&ups)[K * V], int lanes, float lb, float ub,
                        float tol, int32_t iter_max, float *err) {
   tol = tol <= 0.0f ? 1.0e-9f : tol;
@@ -364,13 +383,13 @@ __device__ float brent(const Periods<K, V> &P, const float (&ups)[K * V], int la
     if (fb == 0.0f || fabsf(b - a) < tol) break;
     float s;
     if (fa == fc || fb == fc) {
-      s = b - quot(fb * (b - a), fb - fa);
+      s = b - D::quot(fb * (b - a), fb - fa);
     } else {
       // each difference once: negation is exact
       const float ab = fa - fb, ac = fa - fc, bc = fb - fc;
-      const float s1 = quot(a * fb * fc, ab * ac);
-      const float s2 = quot(b * fa * fc, -ab * bc);
-      const float s3 = quot(c * fa * fb, ac * bc);
+      const float s1 = D::quot(a * fb * fc, ab * ac);
+      const float s2 = D::quot(b * fa * fc, -ab * bc);
+      const float s3 = D::quot(c * fa * fb, ac * bc);
       s = s1 + s2 + s3;
     }
     const bool bisect = !((3.0f * a + b) / 4.0f <= s && s <= b) || x / 2.0f <= fabsf(s - b) ||
@@ -402,7 +421,7 @@ struct Scals {
 };
 
 // exactYhat (:418-481); bb_first and bb_last are bbi[0] and bbi[n-1]
-template <int K, int V>
+template <typename D, int K, int V>
 __device__ float exact_yhat(const Periods<K, V> &P, int n, int lanes, const Scals &sc, float x) {
   const float k = -3.71901648545568f;
   float ups[K * V], part[V], lo = -INFINITY;
@@ -417,7 +436,7 @@ __device__ float exact_yhat(const Periods<K, V> &P, int n, int lanes, const Scal
         const float baix = P.bai[q] * x;
         ups[q] = P.aici[q] * expf(-baix);
         part[v] += ups[q];
-        lo = fmaxf(lo, quot(P.log_aici[q] - baix, P.bbi[q]));
+        lo = fmaxf(lo, D::quot(P.log_aici[q] - baix, P.bbi[q]));
       }
     }
   }
@@ -425,14 +444,14 @@ __device__ float exact_yhat(const Periods<K, V> &P, int n, int lanes, const Scal
   lo = group_max(lo, lanes);
   if (n < 2) return lo;
   const float log_s = logf(up);
-  float tmp = quot(log_s, sc.bb_last);
+  float tmp = D::quot(log_s, sc.bb_last);
   if (!(tmp <= 0.0f)) {
-    tmp = quot(log_s, sc.bb_first);
+    tmp = D::quot(log_s, sc.bb_first);
     tmp = 0.0f <= tmp ? tmp : -INFINITY;
   }
   const float yl = lo - kEps, yu = tmp + kEps;
-  const float rx = quot(sc.rhoxy * (x - sc.mux), sc.sigmax);
-  const float y0 = sc.sigmay * (rx + k * sc.rhoxycs) - quot(sc.rhoxyc, sc.b) + sc.muy;
+  const float rx = D::quot(sc.rhoxy * (x - sc.mux), sc.sigmax);
+  const float y0 = sc.sigmay * (rx + k * sc.rhoxycs) - D::quot(sc.rhoxyc, sc.b) + sc.muy;
   const float y1 = sc.sigmay * (rx - k * sc.rhoxycs) + sc.muy;
   if (y1 <= yl) return y1 + 1.0f;
   if (yu <= y0) return y0 - 1.0f;
@@ -444,9 +463,9 @@ __device__ float exact_yhat(const Periods<K, V> &P, int n, int lanes, const Scal
   for (int q = 0; q < K * V; q++) bb = fmaxf(bb, P.bbi[q]);
   float err, root;
   if (__ballot(!(bb * fabsf(ya) < 86.0f && bb * fabsf(yb) < 86.0f)) == 0)
-    root = brent<true>(P, ups, lanes, ya, yb, 1.0e-4f, 1000, &err);
+    root = brent<D, true>(P, ups, lanes, ya, yb, 1.0e-4f, 1000, &err);
   else
-    root = brent<false>(P, ups, lanes, ya, yb, 1.0e-4f, 1000, &err);
+    root = brent<D, false>(P, ups, lanes, ya, yb, 1.0e-4f, 1000, &err);
   if (err == -INFINITY) return y0 - 1.0f;
   if (err == INFINITY) return y1 + 1.0f;
   return root;
@@ -494,7 +513,7 @@ __global__ __launch_bounds__(kSetupThreads) void ic_setup_kernel(
     const float strike = (zc(t0) - zc(tn)) / lvl;
     const float d1 = 0.5f * row[3] * tmat0;
     ic_swaption S = S0;
-    S.quote = lvl * strike * (ugaussian_P(d1) - ugaussian_P(-d1));
+    S.quote = lvl * strike * (ugaussian_P<Ieee>(d1) - ugaussian_P<Ieee>(-d1));
     S.tmat0 = tmat0;
     S.zc_mat = zc(maturity);
     sw[s] = S;
@@ -546,7 +565,7 @@ struct EvalArgs {
 // (With neighbouring virtual lanes on one physical lane the sums are shorter,
 // but a schedule of 20 periods on 16 lanes of 2 then keeps 8 slots busy for
 // lane 0's sake, where this needs 5.)
-template <int K, int V>
+template <typename D, int K, int V>
 __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, const ic_swaption S,
                                           const int lane) {
   const int lanes = S.lanes / V;  // physical lanes of a group
@@ -561,18 +580,18 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
 
   // :528-546
   float dum1, dum2;
-  const float v0_mat = bigv(g, tmat0, &dum1, &dum2);
-  const float mux = 0.0f - bigmx(g, tmat0);
-  const float muy = 0.0f - bigmy(g, tmat0);
-  const float sqrt_bfun_a = sqrtf(b_fun(2.0f * g.a, tmat0));
-  const float sqrt_bfun_b = sqrtf(b_fun(2.0f * g.b, tmat0));
-  const float rhoxy = quot(g.rho * b_fun(g.a + g.b, tmat0), sqrt_bfun_a * sqrt_bfun_b);
+  const float v0_mat = bigv<D>(g, tmat0, &dum1, &dum2);
+  const float mux = 0.0f - bigmx<D>(g, tmat0);
+  const float muy = 0.0f - bigmy<D>(g, tmat0);
+  const float sqrt_bfun_a = sqrtf(b_fun<D>(2.0f * g.a, tmat0));
+  const float sqrt_bfun_b = sqrtf(b_fun<D>(2.0f * g.b, tmat0));
+  const float rhoxy = D::quot(g.rho * b_fun<D>(g.a + g.b, tmat0), sqrt_bfun_a * sqrt_bfun_b);
   const float sigmax = g.sigma * sqrt_bfun_a;
   const float sigmay = g.nu * sqrt_bfun_b;
   const float rhoxyc = 1.0f - rhoxy * rhoxy;
   const float rhoxycs = sqrtf(rhoxyc);
   const float sigmay_rhoxycs = sigmay * rhoxycs;
-  const float t4 = quot(rhoxy * sigmay, sigmax);
+  const float t4 = D::quot(rhoxy * sigmay, sigmax);
 
   // the schedule's periods (:549-583)
   Periods<K, V> P;
@@ -586,8 +605,8 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
     if (P.valid[q]) {
       const ic_period pe = A.per[S.off + i];
       float bai, bbi;
-      const float v0_end = bigv(g, pe.tod1, &dum1, &dum2);
-      const float vt_end = bigv(g, pe.tod2, &bai, &bbi);
+      const float v0_end = bigv<D>(g, pe.tod1, &dum1, &dum2);
+      const float vt_end = bigv<D>(g, pe.tod2, &bai, &bbi);
       const float expo_aici = 0.5f * (vt_end - v0_end + v0_mat);
       P.bai[q] = bai;
       P.bbi[q] = bbi;
@@ -607,8 +626,8 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
   sc.rhoxycs = rhoxycs;
   sc.mux = mux;
   sc.muy = muy;
-  sc.bb_first = n > 0 ? b_fun(g.b, A.per[S.off].tod2) : 0.0f;
-  sc.bb_last = n > 0 ? b_fun(g.b, A.per[S.off + n - 1].tod2) : 0.0f;
+  sc.bb_first = n > 0 ? b_fun<D>(g.b, A.per[S.off].tod2) : 0.0f;
+  sc.bb_last = n > 0 ? b_fun<D>(g.b, A.per[S.off + n - 1].tod2) : 0.0f;
 
   // :586-591
   const float eps = 0.5f * sigmax;
@@ -618,14 +637,14 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
 #pragma unroll 1
   for (int r = 0; r < 3; r++) {
     const float x = r == 0 ? mux : r == 1 ? mux + eps : mux - eps;
-    const float y = exact_yhat(P, n, lanes, sc, x);
+    const float y = exact_yhat<D>(P, n, lanes, sc, x);
     f = r == 0 ? y : f;
     gg = r == 1 ? y : gg;
     h = r == 2 ? y : h;
   }
-  const float df = quot(0.5f * (gg - h), eps);
+  const float df = D::quot(0.5f * (gg - h), eps);
   const float sqrt2sigmax = sqrtf(2.0f) * sigmax;
-  const float t2 = quot(rhoxy, sigmax * rhoxycs);
+  const float t2 = D::quot(rhoxy, sigmax * rhoxycs);
 
   // Gauss-Hermite (:594-620).  A point's terms without a period, h1 and
   // P(-h1), are made by one lane of the group each, `lanes` points at a time,
@@ -642,8 +661,8 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
       {
         const float x = sqrt2sigmax * __shfl(hx, q0 + j) + mux;
         const float yhat_x = f + df * (x - mux);
-        own_h1 = quot(yhat_x - muy, sigmay_rhoxycs) - t2 * (x - mux);
-        own_p = ugaussian_P(-own_h1);
+        own_h1 = D::quot(yhat_x - muy, sigmay_rhoxycs) - t2 * (x - mux);
+        own_p = ugaussian_P<D>(-own_h1);
       }
       const int here = end64 - q0 < lanes ? end64 - q0 : lanes;
       for (int t = 0; t < here; t++) {
@@ -662,7 +681,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
             if (P.slot0[q] >= n) continue;
             const float h2 = h1 + P.bbi[q] * sigmay_rhoxycs;
             const float expo_aici = P.t1cs[q] + P.scale[q] * x;
-            const float term = P.cs[q] * ugaussian_P_exp(-h2, expo_aici);
+            const float term = P.cs[q] * ugaussian_P_exp<D>(-h2, expo_aici);
             part[v] += P.valid[q] ? term : 0.0f;
           }
         }
@@ -674,7 +693,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
   if (!store) return;
   const int32_t s = wk.swaption;
   if (A.mode == IC_OUT_TERMS) {
-    A.out0[(int64_t)s * A.npop + gi] = log_likelihood(S.quote, price);
+    A.out0[(int64_t)s * A.npop + gi] = log_likelihood<D>(S.quote, price);
   } else if (A.mode == IC_OUT_PRICES) {
     A.out0[(int64_t)gi * A.nswap + s] = S.quote;
     A.out1[(int64_t)gi * A.nswap + s] = price;
@@ -688,6 +707,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs &A, const ic_work wk, c
 
 // Swaptions of 1 or 2 periods a virtual lane (up to 128 periods) in one
 // launch, so the classes share the device; a class is uniform per wavefront.
+template <typename D>
 __global__ __launch_bounds__(256) void ic_eval_kernel(EvalArgs A) {
   const int32_t wv = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (wv >= A.nwork) return;  // wave-uniform
@@ -695,25 +715,26 @@ __global__ __launch_bounds__(256) void ic_eval_kernel(EvalArgs A) {
   const ic_swaption S = A.sw[wk.swaption];
   const int lane = threadIdx.x & 63;
   if (S.per_lane == 1)
-    eval_wave<1, 1>(A, wk, S, lane);
+    eval_wave<D, 1, 1>(A, wk, S, lane);
   else if (wk.pack == 1)
-    eval_wave<2, 1>(A, wk, S, lane);
+    eval_wave<D, 2, 1>(A, wk, S, lane);
   else if (wk.pack == 2)
-    eval_wave<2, 2>(A, wk, S, lane);
+    eval_wave<D, 2, 2>(A, wk, S, lane);
   else
-    eval_wave<2, 4>(A, wk, S, lane);
+    eval_wave<D, 2, 4>(A, wk, S, lane);
 }
 
 // Longer schedules (4 or 8 periods a lane, up to 512 periods): more registers.
+template <typename D>
 __global__ __launch_bounds__(256) void ic_eval_long_kernel(EvalArgs A) {
   const int32_t wv = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (wv >= A.nwork) return;
   const ic_work wk = A.work[wv];
   const ic_swaption S = A.sw[wk.swaption];
   if (S.per_lane == 4)
-    eval_wave<4, 1>(A, wk, S, threadIdx.x & 63);
+    eval_wave<D, 4, 1>(A, wk, S, threadIdx.x & 63);
   else
-    eval_wave<8, 1>(A, wk, S, threadIdx.x & 63);
+    eval_wave<D, 8, 1>(A, wk, S, threadIdx.x & 63);
 }
 
 // ---- accept / propose ------------------------------------------------------------------
@@ -950,7 +971,7 @@ extern "C" int ic_launch_init(void *stream, int32_t pop, const ic_dirvec *dv, fl
 extern "C" int ic_launch_eval(void *stream, const ic_swaption *sw, const ic_period *periods,
                               const ic_worklists *wl, const float *genomes, int32_t npop,
                               const float *herm_x, const float *herm_w, int32_t nherm,
-                              int32_t nswap, int mode, float *out0, float *out1) {
+                              int32_t nswap, int mode, int ieee, float *out0, float *out1) {
   EvalArgs A;
   A.sw = sw;
   A.per = periods;
@@ -968,10 +989,10 @@ extern "C" int ic_launch_eval(void *stream, const ic_swaption *sw, const ic_peri
     A.work = wl->work[c];
     A.nwork = wl->nwork[c];
     const dim3 grid((A.nwork + 3) / 4), block(256);
-    if (c == 0)
-      hipLaunchKernelGGL(ic_eval_kernel, grid, block, 0, (hipStream_t)stream, A);
-    else
-      hipLaunchKernelGGL(ic_eval_long_kernel, grid, block, 0, (hipStream_t)stream, A);
+    void (*const kernel)(EvalArgs) = c == 0 ? (ieee ? ic_eval_kernel<Ieee> : ic_eval_kernel<Short>)
+                                     : ieee ? ic_eval_long_kernel<Ieee>
+                                            : ic_eval_long_kernel<Short>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, A);
   }
   return (int)hipGetLastError();
 }
