@@ -122,21 +122,20 @@ static int64_t request_bytes(const struct lvc_server *s, int nx, int ny) {
   return 2 * request_elems(nx, ny) * (int64_t)s->real;
 }
 
-/* device bytes of the per-slot tables: descriptor, geometry, y factor
- * table, output, factor list and tiles */
-static int64_t slot_bytes(const struct lvc_server *s, int col) {
-  return 2 * (int64_t)sizeof(lvc_problem) + s->slot_geo * (int64_t)sizeof(double) +
-         (col ? LVC_YFAC_LEN * (int64_t)s->real + (int64_t)sizeof(int32_t) : 0) +
-         (int64_t)sizeof(double) + SLOT_MAX_TILES * (int64_t)sizeof(lvc_tile) +
-         2 * (int64_t)sizeof(int32_t);
-}
-
 static size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
 
 /* the device tile list and, after its tiles, the resident slots */
 static size_t tile_bytes(const struct lvc_server *s) {
   return align16((size_t)s->tiles_cap * sizeof(lvc_tile)) +
          align16((size_t)s->max_slots * sizeof(int32_t));
+}
+
+/* device bytes of the tables of all slots: descriptors, geometry, y factor
+ * tables, tile list */
+static int64_t table_bytes(const struct lvc_server *s, int col) {
+  const int64_t each = (int64_t)sizeof(lvc_problem) + s->slot_geo * (int64_t)sizeof(double) +
+                       (col ? LVC_YFAC_LEN * (int64_t)s->real : 0);
+  return s->max_slots * each + (int64_t)tile_bytes(s);
 }
 
 /* tiles of a request: x (rows per workgroup) and y */
@@ -215,7 +214,8 @@ struct lvc_server *lvc_server_new(struct futhark_context *ctx, int32_t max_slots
   /* the budget: the slot tables first, the grid arena from the rest, at most
    * what max_slots grids of the largest size take */
   const int col = lvc_seg_is_col(s->seg_y);
-  const int64_t fixed = (int64_t)max_slots * slot_bytes(s, col);
+  s->tiles_cap = max_slots * SLOT_MAX_TILES;
+  const int64_t fixed = table_bytes(s, col);
   int64_t arena = (int64_t)max_slots * request_elems(SLOT_MAX_N, SLOT_MAX_N);
   if (s->budget > 0) {
     const int64_t fit = (s->budget - fixed) / (2 * (int64_t)s->real) & ~(int64_t)63;
@@ -238,7 +238,6 @@ struct lvc_server *lvc_server_new(struct futhark_context *ctx, int32_t max_slots
   s->h_fprobs = calloc((size_t)max_slots, sizeof(int32_t));
   s->slot_len = calloc((size_t)max_slots, sizeof(int64_t));
   s->free_ext = malloc(((size_t)max_slots + 1) * sizeof(extent));
-  s->tiles_cap = max_slots * SLOT_MAX_TILES;
   s->h_tiles = malloc((size_t)s->tiles_cap * sizeof(lvc_tile));
   s->h_adm = malloc((size_t)max_slots * sizeof(lvc_problem));
   s->h_admslot = malloc((size_t)max_slots * sizeof(int32_t));
