@@ -489,9 +489,6 @@ int lvc_batch_gather(struct futhark_context *ctx, lvc_batch *b, void *out,
   return lvc_check_hip(ctx, e, "gather kernel");
 }
 
-static int download(struct futhark_context *ctx, void *dst, const void *src,
-                    size_t bytes);
-
 /* The streams a batch of sweeps steps on.  A step is an x launch and a y
  * launch that waits for all of it, and each alone leaves half of the vector
  * ALUs' issue slots idle (2 to 3 waves per SIMD, each in a serial chain, and
@@ -540,6 +537,15 @@ static int sweep_streams(struct futhark_context *ctx, int n, const lvc_problem *
              ? 2
              : 1;
 }
+
+/* debugging: the index that the price of problem 0 is taken at */
+void lvc_note_index(struct futhark_context *ctx, int yindex, int xindex) {
+  ctx->dbg_index[0] = yindex;
+  ctx->dbg_index[1] = xindex;
+  ctx->dbg_index_valid = 1;
+}
+
+int lvc_debugging(const struct futhark_context *ctx) { return ctx->cfg && ctx->cfg->debugging; }
 
 /* Runs problems by the sweeps into out.  Each problem takes its own size
  * class's segment pair; the problems of each distinct pair (and stream) form
@@ -600,20 +606,18 @@ static int run_sweeps(struct futhark_context *ctx, int n, const lvc_problem *pro
     rc = run_batches(ctx, bs, nb, split);
   for (int g = 0; !rc && g < nb; g++)
     rc = lvc_batch_gather(ctx, &bs[g], out, out_f64);
+  if (!rc && lvc_debugging(ctx) && probs[0].out_index == 0) {
+    /* the index the gather read: the first descriptor of the first sub-batch */
+    lvc_problem q;
+    rc = lvc_download(ctx, &q, bs[0].d_probs, sizeof(q));
+    if (!rc)
+      lvc_note_index(ctx, q.yindex, q.xindex);
+  }
   for (int g = 0; g < nb; g++)
     lvc_batch_release(ctx, &bs[g]);
   free(grp);
   free(sub);
   return rc;
-}
-
-/* debugging: the index the prices are taken at (problem 0's) */
-static void note_index(struct futhark_context *ctx, const lvc_problem *q) {
-  if (!ctx->cfg || !ctx->cfg->debugging)
-    return;
-  ctx->dbg_index[0] = q->yindex;
-  ctx->dbg_index[1] = q->xindex;
-  ctx->dbg_index_valid = 1;
 }
 
 /* "lvc.autotune" asks for the sweeps of every class that a call meets to be
@@ -645,8 +649,6 @@ static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *prob
     lvc_problem q = probs[p];
     lvc_grid_scalars(&q, q.grid32);
     q.out_index = p;
-    if (p == 0)
-      note_index(ctx, &q);
     if (precision == LVC_FP64 && lvc_modes_fit(&q) && lvc_modes_pay(&q) &&
         lvc_modes_strike(&q, q.strike, 1)) {
       by[nm++] = q;
@@ -745,7 +747,8 @@ static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int 
     const size_t wb = (size_t)lvc_modes_main_work(outer, nx) * sizeof(double);
     double *work = NULL;
     pthread_mutex_lock(&ctx->lock);
-    note_index(ctx, &q);
+    if (lvc_debugging(ctx)) /* the kernels take the index as an argument */
+      lvc_note_index(ctx, q.yindex, q.xindex);
     autotune_class(ctx, precision, &q);
     rc = lvc_dev_alloc(ctx, ob, mem) || lvc_dev_alloc(ctx, wb, (void **)&work) ||
          lvc_modes_main(ctx, &q, outer, f32, work, *mem, !f32);
@@ -980,8 +983,7 @@ int futhark_entry_main_noalloc(struct futhark_context *ctx, float *out,
   return rc;
 }
 
-static int download(struct futhark_context *ctx, void *dst, const void *src,
-                    size_t bytes) {
+int lvc_download(struct futhark_context *ctx, void *dst, const void *src, size_t bytes) {
   if (bytes == 0)
     return 0;
   if (lvc_check_hip(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost,
@@ -1044,11 +1046,11 @@ int futhark_entry_main_batch(struct futhark_context *ctx,
   }
   pthread_mutex_lock(&ctx->lock);
   int rc = 0;
-  rc = rc || download(ctx, iv, lvc_array_mem_i32(numX), (size_t)n * 4);
-  rc = rc || download(ctx, iv + n, lvc_array_mem_i32(numY), (size_t)n * 4);
-  rc = rc || download(ctx, iv + 2 * n, lvc_array_mem_i32(numT), (size_t)n * 4);
+  rc = rc || lvc_download(ctx, iv, lvc_array_mem_i32(numX), (size_t)n * 4);
+  rc = rc || lvc_download(ctx, iv + n, lvc_array_mem_i32(numY), (size_t)n * 4);
+  rc = rc || lvc_download(ctx, iv + 2 * n, lvc_array_mem_i32(numT), (size_t)n * 4);
   for (int k = 0; k < 6 && !rc; k++)
-    rc = download(ctx, rv + k * n, lvc_array_mem_f64(reals[k]), (size_t)n * 8);
+    rc = lvc_download(ctx, rv + k * n, lvc_array_mem_f64(reals[k]), (size_t)n * 8);
   for (int64_t p = 0; p < n && !rc; p++) {
     probs[p].nx = iv[p];
     probs[p].ny = iv[n + p];

@@ -328,6 +328,12 @@ int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs
     a.f = w + align64(modes);
     a.coef = w + 2 * align64(modes);
     rc = launch(ctx, &a, (int)nmode, max_nx, tiles, n, out, out_f64);
+    if (!rc && lvc_debugging(ctx) && probs[0].out_index == 0) {
+      lvc_mgrid g;
+      rc = lvc_download(ctx, &g, a.grids, sizeof(g));
+      if (!rc)
+        lvc_note_index(ctx, g.yindex, g.xindex);
+    }
   }
   lvc_dev_free(ctx, d, up);
   lvc_dev_free(ctx, w, work);

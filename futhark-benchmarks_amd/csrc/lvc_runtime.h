@@ -205,6 +205,12 @@ int lvc_xshare(struct futhark_context *ctx, int precision);
 /* everything but the strike (and the state) equal */
 int lvc_same_factor(const lvc_problem *a, const lvc_problem *b);
 
+/* device memory to the host, after what ctx->stream was given; waits */
+int lvc_download(struct futhark_context *ctx, void *dst, const void *src, size_t bytes);
+/* the debugging report's price index */
+int lvc_debugging(const struct futhark_context *ctx);
+void lvc_note_index(struct futhark_context *ctx, int yindex, int xindex);
+
 /* prices by separation of x (lvc_modes.c) */
 int lvc_modes_fit(const lvc_problem *q);
 int lvc_modes_pay(const lvc_problem *q);

@@ -81,3 +81,20 @@ def test_noalloc_is_not_profiled():
         want, kernels = route(ctx, lambda: ctx.main(5, 40, 36, 20, *MARKET))
         assert kernels == {"lvc_modes", "lvc_evolve", "lvc_price"}
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("shape,strike,precision", [
+    ((40, 36, 5), 0.02, lvc.PRECISION_FP64), ((40, 36, 20), 0.02, lvc.PRECISION_FP64),
+    ((40, 36, 20), 0.0998, lvc.PRECISION_FP64), ((40, 36, 20), 0.02, lvc.PRECISION_FP32)])
+def test_the_index_read(shape, strike, precision):
+    """The debugging report's index is problem 0's by whichever way it goes,
+    the others another."""
+    print(f"case: price index of {shape}, strike {strike}, precision {precision}", flush=True)
+    p = {k: v * 3 for k, v in problem(*shape, strike).items()}
+    p["numX"], p["numY"], p["strike"] = [shape[0], 64, 30], [shape[1], 20, 24], [strike, .01, .03]
+    t, alpha = MARKET[1:3]
+    with lvc.LocVolCalib(debugging=True) as ctx:
+        ctx.main_batch(**p, precision=precision)
+        assert ctx.price_index() == (18, int(40 / (20 * alpha * np.sqrt(t))))
+        ctx.main_f64(3, 64, 20, shape[2], *MARKET)
+        assert ctx.price_index() == (10, int(64 / (20 * alpha * np.sqrt(t))))
