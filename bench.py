@@ -8,17 +8,19 @@ result left in device memory.
 
 Reported:
   value       options/s of futhark_entry_main in its default form (f32
-              prices, to the accuracy of FP32 sweeps with an FP64-residual
-              refinement or better: computed in FP64);
-  fp64        options/s of the FP64 form (futhark_entry_main_f64) and the
-              ratio; p50/p99 per-call latency of both;
+              prices, at least to the accuracy of FP32 sweeps with an
+              FP64-residual refinement: here computed in FP64, by the modes);
+  fp64        options/s of the FP64 form (futhark_entry_main_f64), whose far
+              strikes go by FP64 sweeps, and the ratio; p50/p99 per-call
+              latency of both;
   roofline    the kernel with the largest share of a call's GPU time: the
               bytes it has to move (kernel_bytes) over its mean launch
-              duration, against 8 TB/s, and `fp64` beside it, the call's FP64
-              operations per second against the vector peak.  Neither is
-              near: a call's work is one grid's modes, a few hundred
-              wavefronts, so it lasts as long as one wavefront's chain of
-              dependent operations.  The duration: the event-free timed
+              duration, against 8 TB/s, and `fp64` beside it, the FP64
+              operations per second of the call's time steps against the
+              vector peak.  Neither is near: a call's work is one grid's
+              modes, a few hundred wavefronts, so it lasts as long as one
+              wavefront's chain of dependent operations, and the bound is
+              named "latency".  The duration: the event-free timed
               calls' time per call times the kernel's share of the GPU time
               per call, the share from HIP events recorded around every
               launch on the library's stream in a second pass of the same
@@ -111,7 +113,7 @@ def bench_main_workload(lvc, outer, nx, ny, nt, params=PARAMS, reps=10, check=Tr
     out = {"workload": f"main({outer}, {nx}, {ny}, {nt})"}
     res = {}
     with lvc.LocVolCalib(device=0) as ctx:
-        for key, raw, free, get in (("fp32refine", ctx.main_raw, ctx.free_f32, ctx.main),
+        for key, raw, free, get in (("f32", ctx.main_raw, ctx.free_f32, ctx.main),
                                     ("fp64", ctx.main_f64_raw, ctx.free_f64, ctx.main_f64)):
             for _ in range(2):
                 free(raw(outer, nx, ny, nt, *params))
@@ -126,13 +128,13 @@ def bench_main_workload(lvc, outer, nx, ny, nt, params=PARAMS, reps=10, check=Tr
             res[key] = get(outer, nx, ny, nt, *params)
             out[key] = {"ms_per_call": round(1e3 * float(np.median(lat)), 4),
                         "options_per_s": round(outer / float(np.median(lat)), 1)}
-    out["ratio_fp32refine_vs_fp64"] = round(out["fp32refine"]["options_per_s"] /
-                                            out["fp64"]["options_per_s"], 3)
-    log(f"{out['workload']}: {out['fp32refine']['ms_per_call']} / {out['fp64']['ms_per_call']} ms")
+    out["ratio_f32_vs_fp64"] = round(out["f32"]["options_per_s"] /
+                                     out["fp64"]["options_per_s"], 3)
+    log(f"{out['workload']}: {out['f32']['ms_per_call']} / {out['fp64']['ms_per_call']} ms")
     if check:
         log(f"{out['workload']}: FP64 oracle")
-        out["fp32refine"]["accuracy_vs_fp64_oracle"] = accuracy(
-            res["fp32refine"], oracle_main(outer, nx, ny, nt, params, True))
+        out["f32"]["accuracy_vs_fp64_oracle"] = accuracy(
+            res["f32"], oracle_main(outer, nx, ny, nt, params, True))
         out["fp64"]["accuracy_vs_fp64_oracle"] = accuracy(
             res["fp64"], oracle_main(outer, nx, ny, nt, params, False))
     return out
@@ -507,7 +509,7 @@ def main():
     ap.add_argument("--serve-rates", default="100,250,500,1000,2500,5000",
                     help="Poisson arrival rates (req/s) of the serving runs")
     ap.add_argument("--only-fp32refine", action="store_true",
-                    help="run only the FP32+refinement calls (for profiling)")
+                    help="run only the headline's calls of the f32 entry (for profiling)")
     ap.add_argument("--only-ocean", action="store_true",
                     help="run only the ocean-sim tridiagonal entries (for profiling)")
     ap.add_argument("--copy-calibration", action="store_true",
@@ -538,7 +540,7 @@ def main():
         return
 
     with lvc.LocVolCalib(device=0, profiling=True) as ctx:
-        # FP32 + refinement (headline): timed calls without per-launch events
+        # the f32 entry (headline): timed calls without per-launch events
         ctx.pause_profiling()
         total32, lat32 = time_calls(ctx, ctx.main_raw, ctx.free_f32, args.steps,
                                     args.warmup)
@@ -573,8 +575,9 @@ def main():
     avg_us = (1e6 * total32 / args.steps) * share / max(launches_per_call, 1e-9)
     bytes_launch = kernel_bytes(dom_name)
     achieved = bytes_launch / (avg_us * 1e-6) / 1e9 if avg_us > 0 else 0.0
-    # 18 FP64 operations per mode, row and step (fused multiply-adds as two)
-    flops_call = 26.0 * (NX - 2) * NY * (NT - 1)
+    # lvc_evolve's FP64 operations (fused multiply-adds as two): 24 per mode, row
+    # and step, and 29 per lane of four rows for the reduced system
+    flops_call = (24 + 29 / 4) * (NX - 2) * NY * (NT - 1)
     rel = float(np.max(np.abs(p32 - p64) / np.abs(p64)))
 
     out = {
@@ -599,12 +602,12 @@ def main():
         "fp64": {"value": round(v64, 2), "unit": "options/s",
                  "ms_per_step": round(1e3 * total64 / args.steps, 4),
                  "p50_ms": round(pct(lat64, 50), 4), "p99_ms": round(pct(lat64, 99), 4)},
-        "ratio_fp32refine_vs_fp64": round(v32 / v64, 3),
-        "max_rel_err_fp32refine_vs_fp64": rel,
+        "ratio_f32_vs_fp64": round(v32 / v64, 3),
+        "max_rel_err_f32_vs_fp64": rel,
         "kernels_us_per_launch_with_events": {k: round(v["total_us"] / max(v["count"], 1), 3)
                                               for k, v in rep32.items()},
         "ms_per_step_with_events": round(1e3 * total32p / args.steps, 4),
-        "roofline": {"bound": "hbm", "kernel": dom_name,
+        "roofline": {"bound": "latency", "kernel": dom_name,
                      "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 10),
                      "bytes_per_launch": bytes_launch, "avg_launch_us": round(avg_us, 3),
@@ -614,13 +617,13 @@ def main():
                      "fp64": {"tflops": round(flops_call / (total32 / args.steps) / 1e12, 3),
                               "peak": FP64_VECTOR_TFLOPS}},
     }
-    log(f"headline: {out['ms_per_step']} ms per call (FP32+refine), "
+    log(f"headline: {out['ms_per_step']} ms per call (f32 entry), "
         f"{out['fp64']['ms_per_step']} ms (FP64)")
     check = not args.no_cpu_baseline
     if check:
         log("headline: FP64 oracle")
         out["accuracy_vs_fp64_oracle"] = {
-            "fp32refine": accuracy(p32, oracle_main(OUTER, NX, NY, NT, PARAMS, True)),
+            "f32": accuracy(p32, oracle_main(OUTER, NX, NY, NT, PARAMS, True)),
             "fp64": accuracy(p64, oracle_main(OUTER, NX, NY, NT, PARAMS, False))}
     if not args.no_forms:
         out["plain_small"] = bench_main_workload(lvc, 16, 32, 256, 256, check=check)
