@@ -329,9 +329,9 @@ struct Periods {
   int32_t slot0[K * V];
 };
 
-// expf(x) for |x| < 87: the exponent's integer part and the rest of
-// x log2(e), its product in two parts, by v_exp_f32; without expf's range
-// handling, a third of its instructions.  Equal to expf for every float of
+// expf(x) for |x| < 87 by the device library's method, so as to have its bits:
+// the exponent's integer part and the rest of x log2(e), its product in two
+// parts, by v_exp_f32; without the range handling, a third of the instructions.  Equal to expf for every float of
 // that range (compared over all of them).
 __device__ __forceinline__ float exp_mid(float x) {
   constexpr float c = 0x1.715476p+0f, cc = 0x1.4ae0bep-26f;  // log2(e)

@@ -29,8 +29,9 @@
 // The work is one grid's point steps in FP64 for any number of strikes, at
 // one launch for all time steps, in place of two launches per step that each
 // move every option's grid (63 steps, 128 options of 256 x 256: 126 launches,
-// 8.5 GB).  The host takes this path where the scalars allow it and the
-// steps are worth three launches (lvc_modes_fit).
+// 8.5 GB).  The price is what is left of the chord, with the chord's rounding.
+// The host takes this path where the scalars allow it, the steps are worth three
+// launches (lvc_modes_fit) and the price is not lost that way (lvc_modes_strike).
 //
 // Three kernels: lvc_modes_kernel (eigenvalues, eigenvectors, the options'
 // coefficients), lvc_evolve_kernel (f_k: every time step), lvc_price_kernel

@@ -55,7 +55,8 @@ void futhark_context_config_set_cache_file(struct futhark_context_config *cfg,
  *   "main.suff_intra_par_0", "main.suff_intra_par_1"  accepted, no effect on
  *       results (the reference's version-selection thresholds);
  *   "lvc.precision"  0 = FP32, 1 = FP32 + one FP64-residual refinement per
- *       implicit solve (default), 2 = FP64 (for futhark_entry_main);
+ *       implicit solve (default), 2 = FP64 (for futhark_entry_main where it
+ *       sweeps: see there);
  *   "lvc.seg_x"  unknowns per lane of the x sweep's row systems: 4, 8 or
  *       16 (0 = tuned per size class);
  *   "lvc.seg_y"  the y sweep's solver: lane segments 4, 8, 16 (PCR across

@@ -31,9 +31,16 @@ extern "C" {
  * 0.001*i, i = 0..outer-1, all sharing the grid sizes and parameters.
  * initGrid's scalars (stdX, dx, myXindex = i32.f32(s0/dx): :15-20) are
  * formed in f32 from the f32 arguments, as the reference does, so the price
- * index is the reference's; the rest is computed in the precision set by
- * "lvc.precision" (default FP32 with one FP64-residual refinement per
- * implicit solve, on an FP64 grid).  Errors: numX or numY < 3 or numT < 2
+ * index is the reference's.  From 7 time points on, where the x direction
+ * separates (positive grid nodes, beta >= 0, moderate parameters), the rest is
+ * computed in FP64 by the modes of the x operator; "lvc.precision" and the
+ * sweeps' other tuning parameters then have no effect on these prices.
+ * Elsewhere, and for strikes whose price is too small a part of the spot for the
+ * modes (less than about 1e-6), it is computed by time-stepping sweeps in the
+ * precision set by "lvc.precision" (default FP32 with one FP64-residual
+ * refinement per implicit solve, on an FP64 grid).  So a call of 6 time points
+ * and one of 7 differ in their arithmetic.  "lvc.autotune" times the sweeps of
+ * the call's class either way.  Errors: numX or numY < 3 or numT < 2
  * (the reference's range `1...n-2` at :37 and its timeline), outer < 0
  * (`iota` at :247), a price index outside the grid (the bounds check of
  * `myResult[myYindex, myXindex]` at :236, e.g. 20*alpha*sqrt(t) <= 1),
@@ -46,7 +53,9 @@ int futhark_entry_main(struct futhark_context *ctx, struct futhark_f32_1d **out0
 
 /* The same program with every real f64 (the FP64 plain form): the f32 ->
  * f64 type substitution of LocVolCalib.fut:238-252, initGrid's scalars
- * included.  Errors as futhark_entry_main.  No counterpart in the
+ * included.  By the modes as futhark_entry_main, for beta up to 0.7 and the
+ * strikes whose price is more than about 1/48 of the spot; by FP64 sweeps
+ * otherwise.  Errors as futhark_entry_main.  No counterpart in the
  * reference, which is f32-only; named as the generator names an extra
  * `entry main_f64`. */
 int futhark_entry_main_f64(struct futhark_context *ctx,
@@ -59,8 +68,8 @@ int futhark_entry_main_f64(struct futhark_context *ctx,
 /* futhark_entry_main without device memory allocation.  No counterpart in
  * the reference: it is for callers that cannot allocate (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Same options, precision ("lvc.precision"), segment lengths and kernels as
- * futhark_entry_main, so the same prices bit for bit; the prices go to
+ * Same options, ways, precision ("lvc.precision"), segment lengths and kernels
+ * as futhark_entry_main, so the same prices bit for bit; the prices go to
  * `out`, a device array of `outer` floats owned by the caller (for example
  * from futhark_values_raw_f32_1d), enqueued on the context's stream
  * (futhark_context_sync waits for them).  Every buffer comes from one static
@@ -80,13 +89,18 @@ int futhark_entry_main_noalloc(struct futhark_context *ctx, float *out,
 
 /* Batched form: problem p has its own sizes (numX[p], numY[p], numT[p]) and
  * parameters and runs LocVolCalib.fut:211-236 (`value`).  All arrays have
- * the same length n.  `precision` as "lvc.precision".  The problems advance
- * together, per time step one launch of each sweep per segment-pair class
+ * the same length n.  `precision` as "lvc.precision".  In FP64 a problem goes by
+ * the modes of its x operator where they separate, keep the price's digits (as
+ * in futhark_entry_main_f64) and cost less than its sweeps (numX up to 64, or
+ * numY * (numT - 1) large enough against numX); its price is the same alone and in any
+ * batch.  The other problems, and all in the FP32 forms, advance together, per
+ * time step one launch of each sweep per segment-pair class
  * (each problem takes its own size class's pair, so its price is the same
  * alone and in any batch) over the problems still running (replayed from the
  * context's kept HIP graph with "lvc.graph"), until each has done its own
  * numT-1 steps.  A problem whose price index lies outside its grid
- * gives NaN (the call succeeds).  No counterpart in the reference (its
+ * gives NaN (the call succeeds).  (The FP32 forms' prices carry the rounding of
+ * FP32 sweeps, which futhark_entry_main's do not where it goes by the modes.)  No counterpart in the reference (its
  * `main` shares one size and parameter set). */
 int futhark_entry_main_batch(struct futhark_context *ctx,
                              struct futhark_f64_1d **out0,
@@ -131,12 +145,12 @@ int64_t lvc_server_submit(struct lvc_server *srv, const struct lvc_request *req)
 /* Runs one engine tick: admits queued requests, advances every resident
  * request by one time step, completes the ones that finished.  Enqueues its
  * work on the context's stream without waiting for it: the prices of the
- * requests a tick completes are copied back behind its launches.  Returns
+ * requests a tick completes are written to host memory behind its launches.  Returns
  * the number of requests completed by this tick, or -1 on error. */
 int32_t lvc_server_step(struct lvc_server *srv);
 /* Completed result for `id`: returns 1 and stores the price, 0 when not yet
  * complete, -1 for an unknown id.  For a request a tick has completed, waits
- * for that tick's price copy if it has not landed yet. */
+ * for that tick's prices if they have not landed yet. */
 int32_t lvc_server_poll(struct lvc_server *srv, int64_t id, double *price);
 /* Ticks until nothing is queued or resident.  Returns 0 or -1. */
 int32_t lvc_server_drain(struct lvc_server *srv);
