@@ -628,13 +628,33 @@ static void autotune_class(struct futhark_context *ctx, int precision, const lvc
     lvc_choose_segs(ctx, precision, q->nx, q->ny, &sx, &sy);
 }
 
+/* run_sweeps into a new device array */
+static int run_swept(struct futhark_context *ctx, int n, const lvc_problem *probs,
+                     int precision, int out_f64, void **out_mem) {
+  const size_t ob = (size_t)n * (out_f64 ? sizeof(double) : sizeof(float));
+  const int rc = lvc_dev_alloc(ctx, ob, out_mem) ||
+                 run_sweeps(ctx, n, probs, precision, out_f64, *out_mem);
+  if (rc) {
+    lvc_dev_free(ctx, *out_mem, ob);
+    *out_mem = NULL;
+  }
+  return rc;
+}
+
+/* Whether a call that goes both ways runs its modes, a few launches, on the
+ * context's second stream beside its sweeps, two short ones a step: not where
+ * launches or candidates are timed one by one. */
+static int side_by_side(const struct futhark_context *ctx) {
+  return !profiling_on(ctx) && !(ctx->cfg && ctx->cfg->autotune);
+}
+
 /* Runs a batch end to end into a new device array of n prices: in FP64 the
  * problems whose x direction separates (lvc_modes_fit), whose price the modes
  * do not lose (lvc_modes_strike) and which cost less that way (lvc_modes_pay) by
  * their modes, the others, and the FP32 forms, whose FP64 prices show the
- * arithmetic that was asked for, by the sweeps.  A problem's way depends on the precision and its
- * own sizes and parameters only, so its price has the same bits alone and in
- * any batch. */
+ * arithmetic that was asked for, by the sweeps.  A problem's way depends on the
+ * precision and its own sizes and parameters only, so its price has the same
+ * bits alone and in any batch. */
 static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *probs,
                      int precision, int out_f64, void **out_mem) {
   const size_t ob = (size_t)n * (out_f64 ? sizeof(double) : sizeof(float));
@@ -662,9 +682,11 @@ static int run_batch(struct futhark_context *ctx, int n, const lvc_problem *prob
     by[i] = by[j];
     by[j] = q;
   }
-  const int rc = lvc_dev_alloc(ctx, ob, out_mem) ||
-                 lvc_modes_batch(ctx, nm, by, *out_mem, out_f64) ||
-                 (ns && run_sweeps(ctx, ns, by + nm, precision, out_f64, *out_mem));
+  lvc_modes_mem m = {0};
+  int rc = lvc_dev_alloc(ctx, ob, out_mem) ||
+           lvc_modes_batch(ctx, ns && side_by_side(ctx), nm, by, *out_mem, out_f64, &m) ||
+           (ns && run_sweeps(ctx, ns, by + nm, precision, out_f64, *out_mem));
+  rc = lvc_modes_release(ctx, &m) || rc;
   free(by);
   if (rc) {
     lvc_dev_free(ctx, *out_mem, ob);
@@ -733,34 +755,47 @@ static lvc_problem *main_problems(struct futhark_context *ctx, const lvc_problem
 
 /* main's options into a new device array: one grid with strikes 0.001 * i
  * (:247; f32 = the reference's f32 entry, strikes and initGrid's scalars in
- * f32), by its modes where it separates (and the strikes too far for them by
- * the sweeps, over the modes' prices), else as a batch. */
+ * f32), by its modes where it separates, the strikes too far for them by the
+ * sweeps, else as a batch. */
 static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int nt,
                     double s0, double t, double alpha, double nu, double beta,
                     int f32, int precision, void **mem) {
   const lvc_problem q = main_problem(nx, ny, nt, s0, t, alpha, nu, beta, f32);
   lvc_problem *probs;
-  int rc = 0;
+  int rc = 0, first = 0, end = 0;
   *mem = NULL;
-  if (outer > 0 && lvc_modes_fit(&q)) {
+  const int modes = outer > 0 && lvc_modes_fit(&q);
+  const int ahead = modes && lvc_modes_ends_far(&q, outer, f32);
+  if (ahead)
+    lvc_modes_far(&q, outer, f32, &first, &end);
+  if (modes && (!ahead || first > 0)) {
     const size_t ob = (size_t)outer * (f32 ? sizeof(float) : sizeof(double));
     const size_t wb = (size_t)lvc_modes_main_work(outer, nx) * sizeof(double);
     double *work = NULL;
     pthread_mutex_lock(&ctx->lock);
+    const int beside = ahead && side_by_side(ctx);
     if (lvc_debugging(ctx)) /* the kernels take the index as an argument */
       lvc_note_index(ctx, q.yindex, q.xindex);
     autotune_class(ctx, precision, &q);
     rc = lvc_dev_alloc(ctx, ob, mem) || lvc_dev_alloc(ctx, wb, (void **)&work) ||
-         lvc_modes_main(ctx, &q, outer, f32, work, *mem, !f32);
-    lvc_dev_free(ctx, work, wb);
-    int first = 0, end = 0;
-    if (!rc)
+         (beside && lvc_fork(ctx));
+    const int forked = beside && !rc;
+    /* with far strikes the sweeps are enqueued first: they are the longer, and
+     * the modes beside them wait for the fork only */
+    if (!rc && !beside)
+      rc = lvc_modes_main(ctx, ctx->stream, &q, outer, first, end, f32, work, *mem, !f32);
+    if (!rc && !ahead)
       lvc_modes_far(&q, outer, f32, &first, &end);
-    if (first < end) {
+    if (!rc && first < end) {
       probs = main_problems(ctx, &q, first, end - first, f32);
       rc = !probs || run_sweeps(ctx, end - first, probs, precision, !f32, *mem);
       free(probs);
     }
+    if (!rc && beside)
+      rc = lvc_modes_main(ctx, ctx->stream2, &q, outer, first, end, f32, work, *mem, !f32);
+    if (forked && lvc_join(ctx))
+      rc = 1;
+    lvc_dev_free(ctx, work, wb);
     if (rc) {
       lvc_dev_free(ctx, *mem, ob);
       *mem = NULL;
@@ -772,7 +807,10 @@ static int run_main(struct futhark_context *ctx, int outer, int nx, int ny, int 
   if (!probs)
     return 1;
   pthread_mutex_lock(&ctx->lock);
-  rc = run_batch(ctx, outer, probs, precision, !f32, mem);
+  if (modes) /* not one strike near enough */
+    rc = run_swept(ctx, outer, probs, precision, !f32, mem);
+  else
+    rc = run_batch(ctx, outer, probs, precision, !f32, mem);
   pthread_mutex_unlock(&ctx->lock);
   free(probs);
   return rc;
@@ -969,7 +1007,7 @@ int futhark_entry_main_noalloc(struct futhark_context *ctx, float *out,
      * the caller may be capturing. */
     const int paused = ctx->prof_paused;
     ctx->prof_paused = 1;
-    rc = lvc_modes_main(ctx, &tmpl, outer, 1, (double *)ctx->scratch, out, 0);
+    rc = lvc_modes_main(ctx, ctx->stream, &tmpl, outer, 0, 0, 1, (double *)ctx->scratch, out, 0);
     ctx->prof_paused = paused;
     lvc_modes_far(&tmpl, outer, 1, &first, &end);
   }

@@ -201,7 +201,9 @@ enum {
  * strike 0.001 * i.  Several: grids[] and, per launch, tiles[]. */
 typedef struct lvc_modes_args {
   lvc_mgrid one;
-  int32_t strike_f32, pad_;
+  int32_t strike_f32;
+  int32_t far, far_end; /* options whose price is written by others */
+  int32_t pad_;
   const lvc_mgrid *grids;
   const lvc_mtile *mode_tiles, *tiles[LVC_MODES_KINDS];
   const double *strikes;     /* [options] */

@@ -144,6 +144,18 @@ double lvc_main_strike(int i, int f32) {
   return f32 ? (double)(0.001f * (float)i) : 0.001 * (double)i;
 }
 
+/* Whether main's last strike within the grid is too far: then lvc_modes_far,
+ * which looks at each strike, is worth waiting for before the launches. */
+int lvc_modes_ends_far(const lvc_problem *q, int outer, int f32) {
+  const double xe = (double)(q->nx - 1) * q->dx - (double)q->xindex * q->dx + q->s0;
+  int i = outer - 1;
+  if (1000.0 * xe < (double)i)
+    i = (int)(1000.0 * xe) + 1 < i ? (int)(1000.0 * xe) + 1 : i;
+  while (i > 0 && lvc_main_strike(i, f32) >= xe)
+    i--;
+  return !lvc_modes_strike(q, lvc_main_strike(i, f32), !f32);
+}
+
 /* main's options [*first, *end), of `outer`, that the modes leave to the
  * sweeps: from the first strike that lvc_modes_strike refuses to the grid's
  * last node.  Which way an option goes does not depend on `outer`. */
@@ -187,9 +199,10 @@ static lvc_mgrid make_grid(const lvc_problem *q, int first, int count) {
   return g;
 }
 
-static int launch(struct futhark_context *ctx, const lvc_modes_args *a, int mode_tiles, int max_nx,
-                  const int64_t tiles[LVC_MODES_KINDS], int n, void *out, int out_f64) {
-  void *st = (void *)ctx->stream;
+static int launch(struct futhark_context *ctx, hipStream_t stream, const lvc_modes_args *a,
+                  int mode_tiles, int max_nx, const int64_t tiles[LVC_MODES_KINDS], int n,
+                  void *out, int out_f64) {
+  void *st = (void *)stream;
   int tok = lvc_prof_begin(ctx, "lvc_modes");
   int e = lvc_launch_modes(st, a, mode_tiles, max_nx);
   lvc_prof_end(ctx, tok);
@@ -214,21 +227,25 @@ int64_t lvc_modes_main_work(int outer, int nx) {
   return 2 * align64(nx - 2) + (int64_t)outer * (nx - 2);
 }
 
-/* main's options on q's grid, strikes 0.001 * i: prices into out. */
-int lvc_modes_main(struct futhark_context *ctx, const lvc_problem *q, int outer, int strike_f32,
-                   double *work, void *out, int out_f64) {
+/* main's options on q's grid, strikes 0.001 * i: prices into out, those of the
+ * options [far, far_end) left out. */
+int lvc_modes_main(struct futhark_context *ctx, hipStream_t stream, const lvc_problem *q,
+                   int outer, int far, int far_end, int strike_f32, double *work, void *out,
+                   int out_f64) {
   lvc_modes_args a;
   memset(&a, 0, sizeof(a));
   a.one = make_grid(q, 0, outer);
   a.strike_f32 = strike_f32;
+  a.far = far;
+  a.far_end = far_end;
   const int modes = q->nx - 2, per = 64 / a.one.lanes;
   a.lambda = work;
   a.f = work + align64(modes);
   a.coef = work + 2 * align64(modes);
   int64_t tiles[LVC_MODES_KINDS] = {0};
   tiles[a.one.kind] = (modes + per - 1) / per;
-  return launch(ctx, &a, (modes + LVC_MODES_PER_WAVE - 1) / LVC_MODES_PER_WAVE, q->nx, tiles,
-                outer, out, out_f64);
+  return launch(ctx, stream, &a, (modes + LVC_MODES_PER_WAVE - 1) / LVC_MODES_PER_WAVE, q->nx,
+                tiles, outer, out, out_f64);
 }
 
 static int by_steps(const void *x, const void *y) {
@@ -236,11 +253,13 @@ static int by_steps(const void *x, const void *y) {
   return (a < b) - (a > b);
 }
 
-/* n problems (initGrid scalars set, lvc_modes_fit), each one's price to
- * out[out_index].  Runs of consecutive problems that differ only in the
- * strike share their modes. */
-int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs, void *out,
-                    int out_f64) {
+/* n problems (initGrid scalars set, lvc_modes_fit) on `stream` (ctx->stream, or
+ * ctx->stream2 after lvc_fork), each one's price to out[out_index].  Runs of
+ * consecutive problems that differ only in the strike share their modes.  `m`
+ * keeps the device memory, for lvc_modes_release once ctx->stream has joined. */
+int lvc_modes_batch(struct futhark_context *ctx, int beside, int n, const lvc_problem *probs,
+                    void *out, int out_f64, lvc_modes_mem *m) {
+  memset(m, 0, sizeof(*m));
   if (n == 0)
     return 0;
   /* the grids, then tiles counted per kind */
@@ -289,8 +308,7 @@ int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs
   const size_t o_out = o_grid + (size_t)n * sizeof(int32_t);
   const size_t up = o_out + (size_t)n * sizeof(int32_t);
   const size_t work = (size_t)(2 * align64(modes) + coefs) * sizeof(double);
-  char *h = malloc(up), *d = NULL;
-  double *w = NULL;
+  char *h = malloc(up);
   int rc = !h;
   if (rc) {
     lvc_set_error(ctx, "host allocation failed");
@@ -313,10 +331,14 @@ int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs
         ((int32_t *)(h + o_out))[p] = probs[p].out_index;
       }
     }
-    rc = lvc_dev_alloc(ctx, up, (void **)&d) || lvc_dev_alloc(ctx, work, (void **)&w) ||
-         lvc_upload(ctx, d, h, up);
+    m->tables_bytes = up;
+    m->work_bytes = work;
+    rc = lvc_dev_alloc(ctx, up, &m->tables) || lvc_dev_alloc(ctx, work, &m->work) ||
+         lvc_upload(ctx, m->tables, h, up) || (beside && lvc_fork(ctx));
   }
   if (!rc) {
+    char *d = m->tables;
+    double *w = m->work;
     lvc_modes_args a;
     memset(&a, 0, sizeof(a));
     a.grids = (const lvc_mgrid *)d;
@@ -329,7 +351,9 @@ int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs
     a.lambda = w;
     a.f = w + align64(modes);
     a.coef = w + 2 * align64(modes);
-    rc = launch(ctx, &a, (int)nmode, max_nx, tiles, n, out, out_f64);
+    m->forked = beside;
+    rc = launch(ctx, beside ? ctx->stream2 : ctx->stream, &a, (int)nmode, max_nx, tiles, n, out,
+                out_f64);
     if (!rc && lvc_debugging(ctx) && probs[0].out_index == 0) {
       lvc_mgrid g;
       rc = lvc_download(ctx, &g, a.grids, sizeof(g));
@@ -337,10 +361,17 @@ int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs
         lvc_note_index(ctx, g.yindex, g.xindex);
     }
   }
-  lvc_dev_free(ctx, d, up);
-  lvc_dev_free(ctx, w, work);
   free(h);
   free(grids);
   free(order);
+  return rc;
+}
+
+/* Joins a batch that ran beside ctx->stream and gives its memory back. */
+int lvc_modes_release(struct futhark_context *ctx, lvc_modes_mem *m) {
+  const int rc = m->forked && lvc_join(ctx);
+  lvc_dev_free(ctx, m->tables, m->tables_bytes);
+  lvc_dev_free(ctx, m->work, m->work_bytes);
+  memset(m, 0, sizeof(*m));
   return rc;
 }

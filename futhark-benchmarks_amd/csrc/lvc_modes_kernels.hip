@@ -578,7 +578,7 @@ __global__ __launch_bounds__(64, KIND == LVC_MODES_WAVE16 ? 1 : 2) void lvc_evol
 template <bool ONE, typename O>
 __global__ __launch_bounds__(256) void lvc_price_kernel(lvc_modes_args a, int n, O *out) {
   const int o = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (o >= n) return;
+  if (o >= n || (o >= a.far && o < a.far_end)) return;
   const lvc_mgrid G = load_grid<ONE>(a, ONE ? 0 : a.grid_of[o]);
   const int N = G.nx - 2;
   const double *c = a.coef + G.coef_off + (int64_t)(o - G.first) * N, *f = a.f + G.mode0;

@@ -216,12 +216,20 @@ int lvc_modes_fit(const lvc_problem *q);
 int lvc_modes_pay(const lvc_problem *q);
 int lvc_modes_strike(const lvc_problem *q, double strike, int out_f64);
 double lvc_main_strike(int i, int f32);
+int lvc_modes_ends_far(const lvc_problem *q, int outer, int f32);
 void lvc_modes_far(const lvc_problem *q, int outer, int f32, int *first, int *end);
 int64_t lvc_modes_main_work(int outer, int nx);
-int lvc_modes_main(struct futhark_context *ctx, const lvc_problem *q, int outer,
-                   int strike_f32, double *work, void *out, int out_f64);
-int lvc_modes_batch(struct futhark_context *ctx, int n, const lvc_problem *probs,
-                    void *out, int out_f64);
+int lvc_modes_main(struct futhark_context *ctx, hipStream_t stream, const lvc_problem *q,
+                   int outer, int far, int far_end, int strike_f32, double *work, void *out,
+                   int out_f64);
+typedef struct {
+  void *tables, *work; /* device memory of a batch by the modes */
+  size_t tables_bytes, work_bytes;
+  int forked;
+} lvc_modes_mem;
+int lvc_modes_batch(struct futhark_context *ctx, int beside, int n, const lvc_problem *probs,
+                    void *out, int out_f64, lvc_modes_mem *m);
+int lvc_modes_release(struct futhark_context *ctx, lvc_modes_mem *m);
 /* LocVolCalib's context-ready hook: the tuning cache and the scratch address */
 void lvc_context_ready(struct futhark_context *ctx);
 

@@ -93,3 +93,23 @@ def test_main_f32(market, precision):
         assert np.array_equal(got[:n // 2], ctx.main_noalloc(n // 2, *args))
     normal = (ref == 0) | (ref > 1e-30)  # f32's range
     check(got[normal].astype(np.float64), ref[normal], 1e-6)
+
+
+def test_side_by_side():
+    """Calls that go both ways run their modes on the second stream beside the
+    sweeps: the same bits as one after the other (with profiling), call after
+    call on the memory of the one before, in two contexts in turn."""
+    print("case: far strikes, modes beside sweeps", flush=True)
+    p = batch_of()
+    calls = [lambda c: c.main_f64(90, 256, 32, 32, 0.03, 5.0, 0.12, 0.1, 0.5),
+             lambda c: c.main_batch(**p, precision=lvc.PRECISION_FP64),
+             lambda c: c.main(260, 128, 40, 20, 0.03, 5.0, 0.2, 0.1, 1.0),
+             lambda c: c.main_f64(40, 32, 16, 9, 0.03, 1.0, 0.1, 0.2, 0.7),
+             lambda c: c.main_f64(3, 64, 64, 12, 0.03, 5.0, 0.2, 0.6, 0.9)]
+    with lvc.LocVolCalib(profiling=True) as one:
+        want = [call(one) for call in calls]
+    with lvc.LocVolCalib() as first, lvc.LocVolCalib() as second:
+        for ctx in (first, second, first):
+            for _ in range(3):
+                for call, ref in zip(calls, want):
+                    assert np.array_equal(call(ctx), ref)
