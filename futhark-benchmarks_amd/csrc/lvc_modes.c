@@ -76,22 +76,24 @@ static double normal_call(double d) {
   return 0.3989422804014327 * exp(-0.5 * d * d) - 0.5 * d * erfc(0.7071067811865476 * d);
 }
 
-/* A floor of the price of an option of q's grid, over the spot.  The chord
+/* A floor of the price of an option of q's grid, over the spot, as far as it
+ * takes to reach `enough`.  The chord
  * through the grid's ends, of which the modes take their sum, does not get
  * small where the price does, so what they leave of a far strike is rounding.
  * Given the volatility's path, x is the elastic process in the clock
  * V = integral of exp(2y - nu^2 t), stopped at the grid's ends: in u = the
  * integral of dx / x^beta a Brownian motion whose drift towards the strike is
  * minus the mean of beta/2 x^(beta-1), and the price at least strike^beta times
- * the normal call less what the ends take (the images).  V is at least
+ * the normal call spread up to the grid's last node, less its image behind the
+ * first.  V is at least
  * alpha^2 t times the geometric mean of the same path, whose logarithm is
  * normal, -nu^2 t / 2 with variance 4/3 nu^2 t; a price grows with V, so three
  * levels of it with the probabilities between them bound the mean.  Against
  * the scheme in 128 bits (19,000 prices, beta 0 .. 1.6, nu .01 .. 1.6, 6 .. 512
  * nodes): median 0.4 of the price, at most 1.5 times it in 99 % and 10 times on
  * grids of under 10 nodes at beta 1.5. */
-static double price_floor(const lvc_problem *q, double strike, double xe) {
-  static const double level[3] = {-0.7, 0.3, 1.3}, weight[3] = {0.376, 0.285, 0.097};
+static double price_floor(const lvc_problem *q, double strike, double xe, double enough) {
+  static const double level[3] = {1.3, 0.3, -0.7}, weight[3] = {0.097, 0.285, 0.376};
   const double s0 = q->s0, beta = q->beta, inner = (s0 - strike) / s0;
   if (inner > 0.0)
     strike = s0;
@@ -102,17 +104,17 @@ static double price_floor(const lvc_problem *q, double strike, double xe) {
   const double low = lognormal ? log(q->x0log / s0) : (pow(q->x0log, g) - sg) / g;
   const double drift =
       0.5 * beta * (strike > s0 * (1.0 + 1e-6) ? log(strike / s0) / up : sg / s0);
-  const double nt = q->nu * sqrt(q->t);
+  const double root = sqrt(q->t), nt = q->nu * root, scale = pow(strike, beta) / s0;
   double sum = 0.0;
-  for (int i = 0; i < 3; i++) {
-    const double sd = q->alpha * sqrt(q->t) * exp(nt * (level[i] / sqrt(3.0) - 0.25 * nt));
+  for (int i = 0; i < 3 && !(scale * sum >= enough); i++) {
+    const double sd = q->alpha * root * exp(nt * (level[i] / sqrt(3.0) - 0.25 * nt));
     const double m = drift * sd;
     const double v = normal_call(up / sd + m) - normal_call(end / sd + m) -
-                     normal_call((up - 2.0 * low) / sd + m);
+                     normal_call((up - 2.0 * low) / sd + m) +
+                     normal_call((end - 2.0 * low) / sd + m);
     sum += v > 0.0 ? weight[i] * sd * v : v > -1.0 ? 0.0 : v; /* a NaN stays one */
   }
-  const double floor_ = pow(strike, beta) * sum / s0;
-  return inner > floor_ ? inner : floor_;
+  return inner > scale * sum ? inner : scale * sum;
 }
 
 /* Whether the modes give the price of a strike on q's grid (lvc_modes_fit)
@@ -121,10 +123,11 @@ static double price_floor(const lvc_problem *q, double strike, double xe) {
  * rule is on the price's floor.  Error against 128 bits over the accepted ones
  * of the 19,000 prices above, modes / sweeps:
  *   FP64 (beta <= 0.7, floor 1/48 and (x_N / x_1)^beta / 250 of the spot):
- *     worst 8.5e-14 / 1.2e-13, 1 % above 2.7e-14 / 5.4e-14, rms 5.7e-15 / 1.1e-14,
- *     median 3.5e-16 / 1.5e-15; with beta up to 0.75 the worst is 2.1e-13
- *   f32 (2^-22 (x_N / x_1)^beta of the spot): worst 7.7e-9 before the price is
- *     rounded to f32, where the FP32 sweeps with refinement had 1e-7.
+ *     worst 8.5e-14 / 1.2e-13, 1 % above 2.7e-14 / 5.4e-14, rms 5.6e-15 / 1.2e-14,
+ *     median 3.6e-16 / 1.5e-15; with beta up to 0.75 the worst is 2.1e-13
+ *   f32 (2^-24 (x_N / x_1)^beta of the spot): before the price is rounded to f32,
+ *     worst 3.0e-8, 0.1 % above 2.8e-9; the FP32 sweeps with refinement had a
+ *     median of 6e-8 and a worst of 2.3e-6.
  * From the grid's last node on a price is exactly 0 either way. */
 int lvc_modes_strike(const lvc_problem *q, double strike, int out_f64) {
   const double x0 = q->s0 - (double)q->xindex * q->dx;
@@ -135,8 +138,8 @@ int lvc_modes_strike(const lvc_problem *q, double strike, int out_f64) {
     return 0;
   const double spread = pow((xe - q->dx) / (x0 + q->dx), q->beta);
   const double least = out_f64 ? fmax(1.0 / 48.0, spread / 250.0)
-                               : 0x1p-22 * fmax(1.0, spread);
-  return q->s0 - strike >= least * q->s0 || price_floor(q, strike, xe) >= least;
+                               : 0x1p-24 * fmax(1.0, spread);
+  return q->s0 - strike >= least * q->s0 || price_floor(q, strike, xe, least) >= least;
 }
 
 /* main's strike i (LocVolCalib.fut:247), in f32 for the f32 entry */
@@ -145,7 +148,10 @@ double lvc_main_strike(int i, int f32) {
 }
 
 /* Whether main's last strike within the grid is too far: then lvc_modes_far,
- * which looks at each strike, is worth waiting for before the launches. */
+ * which looks at each strike, is worth waiting for before the launches.  A
+ * strike within so many deviations of the spot is not even looked at here
+ * (half a microsecond of a call of 40); should it be far, it is found behind
+ * the launches. */
 int lvc_modes_ends_far(const lvc_problem *q, int outer, int f32) {
   const double xe = (double)(q->nx - 1) * q->dx - (double)q->xindex * q->dx + q->s0;
   int i = outer - 1;
@@ -153,7 +159,10 @@ int lvc_modes_ends_far(const lvc_problem *q, int outer, int f32) {
     i = (int)(1000.0 * xe) + 1 < i ? (int)(1000.0 * xe) + 1 : i;
   while (i > 0 && lvc_main_strike(i, f32) >= xe)
     i--;
-  return !lvc_modes_strike(q, lvc_main_strike(i, f32), !f32);
+  const double strike = lvc_main_strike(i, f32);
+  if (strike - q->s0 < (f32 ? 4.0 : 0.5) * q->alpha * sqrt(q->t) * pow(q->s0, q->beta))
+    return 0;
+  return !lvc_modes_strike(q, strike, !f32);
 }
 
 /* main's options [*first, *end), of `outer`, that the modes leave to the

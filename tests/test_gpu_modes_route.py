@@ -98,3 +98,27 @@ def test_the_index_read(shape, strike, precision):
         assert ctx.price_index() == (18, int(40 / (20 * alpha * np.sqrt(t))))
         ctx.main_f64(3, 64, 20, shape[2], *MARKET)
         assert ctx.price_index() == (10, int(64 / (20 * alpha * np.sqrt(t))))
+
+
+@pytest.mark.parametrize("market", [(0.0263, 2.2404, 0.2967, 0.4011, 0.4463),
+                                    (0.0285, 1.9693, 0.247, 0.5365, 0.3156),
+                                    (0.0219, 8.4294, 0.1329, 0.5501, 0.4267)])
+def test_the_last_cell(market):
+    """Strikes just below the grid's last node, whose price is small because the
+    node is near and not because the strike is far: the f32 entry takes the modes."""
+    print(f"case: strikes to the grid's end, {market}", flush=True)
+    with lvc.LocVolCalib(profiling=True) as ctx:
+        got, kernels = route(ctx, lambda: ctx.main(256, 256, 64, 12, *market))
+    assert kernels == {"lvc_modes", "lvc_evolve", "lvc_price"}
+    s0, t, alpha, nu, beta = (float(np.float32(v)) for v in market)
+    dx = float(np.float32(20) * np.float32(alpha) * np.float32(s0) * np.sqrt(np.float32(t)) /
+               np.float32(256))
+    last = (255 - int(s0 / dx)) * dx + s0
+    near = [int(1000 * last) - 1, int(1000 * last), int(1000 * last) + 1]
+    strikes = (np.float32(0.001) * np.float32(near)).astype(np.float64)
+    p = dict(zip(KEYS, [[v] * 3 for v in (256, 64, 12, s0)] + [strikes] +
+                 [[v] * 3 for v in (t, alpha, nu, beta)]))
+    ref = oracle.batch(*[p[k] for k in KEYS], dtype=np.float64, thomas=True, nthreads=8,
+                       grid32=True)
+    assert ref[1] > 0 and ref[2] == 0
+    assert np.all(np.abs(got[near] - ref) <= 1e-6 * ref)
