@@ -19,8 +19,9 @@ Reported:
               operations per second of the call's time steps against the
               vector peak.  Neither is near: a call's work is one grid's
               modes, a few hundred wavefronts, so it lasts as long as one
-              wavefront's chain of dependent operations, and the bound is
-              named "latency".  The duration: the event-free timed
+              wavefront's chain of dependent operations: "bound" is the
+              roof the rate is compared with, "limited_by" what holds
+              the kernel.  The duration: the event-free timed
               calls' time per call times the kernel's share of the GPU time
               per call, the share from HIP events recorded around every
               launch on the library's stream in a second pass of the same
@@ -607,7 +608,7 @@ def main():
         "kernels_us_per_launch_with_events": {k: round(v["total_us"] / max(v["count"], 1), 3)
                                               for k, v in rep32.items()},
         "ms_per_step_with_events": round(1e3 * total32p / args.steps, 4),
-        "roofline": {"bound": "latency", "kernel": dom_name,
+        "roofline": {"bound": "hbm", "limited_by": "latency", "kernel": dom_name,
                      "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 10),
                      "bytes_per_launch": bytes_launch, "avg_launch_us": round(avg_us, 3),
