@@ -651,8 +651,9 @@ __global__ __launch_bounds__(kThreads) void op_many_kernel(
     float pay[MC];
     // the models whose payoff stands: a model's path is repriced for its own
     // prices' sake only, so its mean does not depend on which share the pass
-    const uint32_t all = (1u << M) - 1u;
-    uint32_t good = 0u;
+    bool good[MC], all = false;
+#pragma unroll
+    for (int m = 0; m < MC; ++m) good[m] = false;
     if (fits) {
       LogPath<3> path[MC];
 #pragma unroll
@@ -742,11 +743,15 @@ __global__ __launch_bounds__(kThreads) void op_many_kernel(
       static_assert(D % 2 == 1, "a last step");
       step(D - 1, even);
       stream_rest(date_at, D * sizeof(Date));
+      all = true;
 #pragma unroll
       for (int m = 0; m < MC; ++m)
-        if (m < M && path[m].pay(discts + m * K, &pay[m])) good |= 1u << m;
+        if (m < M) {
+          good[m] = path[m].pay(discts + m * K, &pay[m]);
+          all = good[m] && all;
+        }
     }
-    if (__any(good != all)) {
+    if (__any(!all)) {
       // any tables, any values: all rows in private memory, starting at zero
       // (:153), indexes clamped to the row so that no input makes an access out
       // of bounds (the reference reads bb_inds unchecked, :156)
@@ -781,7 +786,7 @@ __global__ __launch_bounds__(kThreads) void op_many_kernel(
       for (int m = 0; m < MC; ++m) {
         if (m < M) {
           const float p = product_payoff<3>(mk, m, [&](int u, int d) { return rows[u][d]; });
-          if (!(good >> m & 1u)) pay[m] = p;
+          if (!good[m]) pay[m] = p;
         }
       }
     }
