@@ -147,36 +147,49 @@ double lvc_main_strike(int i, int f32) {
   return f32 ? (double)(0.001f * (float)i) : 0.001 * (double)i;
 }
 
-/* Whether main's last strike within the grid is too far: then lvc_modes_far,
- * which looks at each strike, is worth waiting for before the launches.  A
- * strike within so many deviations of the spot is not even looked at here
- * (half a microsecond of a call of 40); should it be far, it is found behind
- * the launches. */
-int lvc_modes_ends_far(const lvc_problem *q, int outer, int f32) {
+/* How many of main's strikes, from the first, are below the grid's last node. */
+static int strikes_inside(const lvc_problem *q, int f32) {
   const double xe = (double)(q->nx - 1) * q->dx - (double)q->xindex * q->dx + q->s0;
-  int i = outer - 1;
-  if (1000.0 * xe < (double)i)
-    i = (int)(1000.0 * xe) + 1 < i ? (int)(1000.0 * xe) + 1 : i;
-  while (i > 0 && lvc_main_strike(i, f32) >= xe)
+  const double n = 1000.0 * xe;
+  int i = n < 2147483647.0 ? (int)n : INT32_MAX;
+  while (i > 0 && lvc_main_strike(i - 1, f32) >= xe)
     i--;
-  const double strike = lvc_main_strike(i, f32);
-  if (strike - q->s0 < (f32 ? 4.0 : 0.5) * q->alpha * sqrt(q->t) * pow(q->s0, q->beta))
+  while (i < INT32_MAX && lvc_main_strike(i, f32) < xe)
+    i++;
+  return i;
+}
+
+/* Whether main's last strike within the grid is too far: then lvc_modes_far is
+ * worth waiting for before the launches.  A strike within so many deviations of
+ * the spot is not even looked at here (half a microsecond of a call of 40);
+ * should it be far, it is found behind the launches. */
+int lvc_modes_ends_far(const lvc_problem *q, int outer, int f32) {
+  const int inside = strikes_inside(q, f32), last = outer < inside ? outer : inside;
+  const double strike = lvc_main_strike(last > 0 ? last - 1 : 0, f32);
+  if (strike - q->s0 < (f32 ? 8.0 : 0.5) * q->alpha * sqrt(q->t) * pow(q->s0, q->beta))
     return 0;
   return !lvc_modes_strike(q, strike, !f32);
 }
 
 /* main's options [*first, *end), of `outer`, that the modes leave to the
- * sweeps: from the first strike that lvc_modes_strike refuses to the grid's
- * last node.  Which way an option goes does not depend on `outer`. */
+ * sweeps: above the last strike that a bisection finds accepted by
+ * lvc_modes_strike (a price falls with the strike, so those below it are worth
+ * more) to the grid's last node.  Which way an option goes does not depend on
+ * `outer`. */
 void lvc_modes_far(const lvc_problem *q, int outer, int f32, int *first, int *end) {
-  const double xe = (double)(q->nx - 1) * q->dx - (double)q->xindex * q->dx + q->s0;
-  int i = 0;
-  while (i < outer && lvc_modes_strike(q, lvc_main_strike(i, f32), !f32))
-    i++;
-  *first = i;
-  while (i < outer && lvc_main_strike(i, f32) < xe)
-    i++;
-  *end = i;
+  const int inside = strikes_inside(q, f32);
+  int near = -1, far = inside; /* options known to be near, and not */
+  if (far > 0 && lvc_modes_strike(q, lvc_main_strike(far - 1, f32), !f32))
+    near = far - 1;
+  while (far - near > 1) {
+    const int i = near + (far - near) / 2;
+    if (lvc_modes_strike(q, lvc_main_strike(i, f32), !f32))
+      near = i;
+    else
+      far = i;
+  }
+  *end = outer < inside ? outer : inside;
+  *first = far < *end ? far : *end;
 }
 
 /* The lanes per mode of a column of ny rows, and how its rows lie in them. */

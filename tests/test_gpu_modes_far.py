@@ -113,3 +113,31 @@ def test_side_by_side():
             for _ in range(3):
                 for call, ref in zip(calls, want):
                     assert np.array_equal(call(ctx), ref)
+
+
+def test_side_by_side_with_graph():
+    """The same under "lvc.graph", which captures the sweeps' steps."""
+    print("case: far strikes, modes beside a captured graph", flush=True)
+    p = batch_of()
+    calls = [lambda c: c.main_f64(90, 256, 32, 32, 0.03, 5.0, 0.12, 0.1, 0.5),
+             lambda c: c.main_batch(**p, precision=lvc.PRECISION_FP64),
+             lambda c: c.main_f64(40, 32, 16, 9, 0.03, 1.0, 0.1, 0.2, 0.7)]
+    with lvc.LocVolCalib() as eager, lvc.LocVolCalib(tuning={"lvc.graph": 1}) as ctx:
+        want = [call(eager) for call in calls]
+        for _ in range(3):
+            for call, ref in zip(calls, want):
+                assert np.array_equal(call(ctx), ref)
+                eager.main(4, 32, 32, 5, 0.03, 5.0, 0.2, 0.6, 0.5)
+                eager.sync()
+
+
+def test_many_strikes(gpu_ctx):
+    """Thousands of strikes within one grid, near and far."""
+    args = (64, 16, 9, 1.5, 2.0, 0.2, 0.1, 0.5)
+    print("case: far strikes, main_f64 of 9000", flush=True)
+    got = gpu_ctx.main_f64(9000, *args)
+    some = np.unique(np.linspace(0, 8999, 60).astype(int))
+    p = dict(zip(KEYS, [np.full(len(some), v) for v in args[:4]] + [0.001 * some] +
+                 [np.full(len(some), v) for v in args[4:]]))
+    check(got[some], oracle_batch(p), 1e-10)
+    assert np.array_equal(gpu_ctx.main_f64(2500, *args), got[:2500])
