@@ -309,7 +309,7 @@ int lvc_modes_batch(struct futhark_context *ctx, int beside, int n, const lvc_pr
     tiles[g.kind] += (m + per - 1) / per;
     if (g.nx > max_nx)
       max_nx = g.nx;
-    order[ng] = (int64_t)g.nt << 24 | ng; /* most steps first */
+    order[ng] = (int64_t)g.nt << 32 | ng; /* most steps first */
     grids[ng++] = g;
     p += c;
   }
@@ -340,7 +340,7 @@ int lvc_modes_batch(struct futhark_context *ctx, int beside, int n, const lvc_pr
     for (int i = 0; i < LVC_MODES_KINDS; i++)
       et[i] = (lvc_mtile *)(h + o_tiles[i]);
     for (int i = 0; i < ng; i++) {
-      const int gi = (int)(order[i] & 0xffffff);
+      const int gi = (int)(order[i] & 0xffffffff);
       const lvc_mgrid *g = &grids[gi];
       const int m = g->nx - 2, per = 64 / g->lanes;
       for (int k = 0; k < m; k += LVC_MODES_PER_WAVE)
